@@ -35,7 +35,8 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 
 // C[M x N] = A[M x K] . B[K x N] with A(m, k) = A[m sam + k sak],
 // B(k, n) = B[k sbk + n sbn]; bf16 operands, FP32 accumulation.
-// epi 0: C = acc;  1: Z = acc + bias, C = gelu(Z);  2: C = acc + bias.
+// epi 0: C = acc;  1: Z = acc + bias, C = gelu(Z);  2: C = acc + bias;
+// 3: C = acc * gelu'(Z).
 struct MmArgs {
     int M, N, K;
     const float* A;
@@ -47,6 +48,10 @@ struct MmArgs {
     const float* bias;
     float* Z;
     int epi;
+    int kchunk;                           // values of k per blockIdx.z (K: no split)
+    int64_t cz;                           // elements between the outputs of two chunks
+    float* colsum;                        // when set (ak false): sums of A's columns, per chunk
+    bool ak, bk;                          // the operand is contiguous in k, else in m (n)
 };
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
@@ -68,6 +73,8 @@ __device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, int
             a.C[o] = gelu(v);
         } else if (a.epi == 2) {
             a.C[o] = v + a.bias[cn];
+        } else if (a.epi == 3) {
+            a.C[o] = v * gelu_d(a.Z[o]);
         } else {
             a.C[o] = v;
         }
@@ -75,71 +82,118 @@ __device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, int
 }
 
 // Block 256 threads = 4 waves, 64 x 64 outputs; wave (w & 1, w >> 1) takes a
-// 32 x 32 tile (one v_mfma_f32_32x32x16_bf16 accumulator).  Operand element j
-// of lane l is row (col) l % 32 at k = k0 + 8 (l / 32) + j; out-of-range
-// elements load as zero.
+// 32 x 32 tile (one v_mfma_f32_32x32x16_bf16 accumulator).  Operands are
+// staged through LDS 32 values of k at a time, rounded to bf16 on the way:
+// [row][k], so that a lane's operand (row l % 32, 8 values of k) is one
+// 16-byte LDS read.  AK, BK: the operand is contiguous in k in memory (a
+// thread stages 8 values of k of one row, two 16-byte loads where the rows
+// are aligned), else contiguous in m or n (a thread stages 8 values of k of
+// one m or n, the 64 lanes of a load reading 64 consecutive floats).  The
+// next step's loads are in flight while this step's products run; k runs in
+// ascending order, out-of-range elements are zero.
+//
+// blockIdx.z splits k into chunks of kchunk (weight gradients: k is the row
+// of the minibatch): chunk z writes its own C + z cz.  colsum: the chunk's
+// sums over k of A's columns in FP32 (the bias gradient), by the blocks of
+// the first n tile.
+//
+// What bounds it: latency (a 4096-row step is 0.3 to 0.5 GFLOP per product).
+// Before, the gradient products read strided scalars per lane (22 us each,
+// 207 us for the 33-wide input) and one thread summed a whole column (851 us
+// for 4096 rows, four times): 4.0 ms per loss and gradient of 4096 rows of the
+// 33-256-256-256-65 network, 0.25 ms now (products 11 to 18 us each).
+template <bool AK, bool BK>
 __global__ __launch_bounds__(256) void k_mm(MmArgs a) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m0 = blockIdx.y * 64 + (w & 1) * 32;
-    const int n0 = blockIdx.x * 64 + (w >> 1) * 32;
-    const int rm = m0 + (lane & 31), cn = n0 + (lane & 31);
-    const int kh = (lane >> 5) * 8;
+    constexpr int LS = 40;                        // LDS row stride in bf16 (80 bytes: no bank conflicts at 16 bytes)
+    __shared__ __attribute__((aligned(16))) uint16_t As[2][64 * LS], Bs[2][64 * LS];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+    const int kb = (int)blockIdx.z * a.kchunk, ke = min(a.K, kb + a.kchunk);
+    // one operand's 8 values of this thread: row (m or n) r0 + r, k0 + 8 q ..
+    const int ra = AK ? t >> 2 : lane, qa = AK ? t & 3 : w;
+    const int rb = BK ? t >> 2 : lane, qb = BK ? t & 3 : w;
+    auto fetch = [&](const float* P, int64_t sr, int64_t sk, int row, int rows, int k, bool kc, bool v4, float (&f)[8]) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = 0.f;
+        if (row >= rows) return;
+        const float* p = P + (int64_t)row * sr + (int64_t)k * sk;
+        if (kc && v4 && k + 8 <= ke) {
+            const float4 u = *reinterpret_cast<const float4*>(p), v = *reinterpret_cast<const float4*>(p + 4);
+            f[0] = u.x; f[1] = u.y; f[2] = u.z; f[3] = u.w;
+            f[4] = v.x; f[5] = v.y; f[6] = v.z; f[7] = v.w;
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (k + j < ke) f[j] = p[(int64_t)j * sk];
+    };
+    const bool av4 = AK && (a.sam & 3) == 0 && (reinterpret_cast<uintptr_t>(a.A) & 15) == 0 && (kb & 3) == 0;
+    const bool bv4 = BK && (a.sbn & 3) == 0 && (reinterpret_cast<uintptr_t>(a.B) & 15) == 0 && (kb & 3) == 0;
+    auto stash = [&](uint16_t* L, int r, int q, const float (&f)[8]) {
+        uint4 o;
+        o.x = to_bf16(f[0]) | ((uint32_t)to_bf16(f[1]) << 16);
+        o.y = to_bf16(f[2]) | ((uint32_t)to_bf16(f[3]) << 16);
+        o.z = to_bf16(f[4]) | ((uint32_t)to_bf16(f[5]) << 16);
+        o.w = to_bf16(f[6]) | ((uint32_t)to_bf16(f[7]) << 16);
+        *reinterpret_cast<uint4*>(L + r * LS + q * 8) = o;
+    };
+    float cs = 0.f;
+    const bool sums = a.colsum && blockIdx.x == 0;
+    float fa[8], fb[8];
+    auto fetch2 = [&](int k0) {
+        fetch(a.A, a.sam, a.sak, m0 + ra, a.M, k0 + 8 * qa, AK, av4, fa);
+        fetch(a.B, a.sbn, a.sbk, n0 + rb, a.N, k0 + 8 * qb, BK, bv4, fb);
+    };
+    auto stash2 = [&](int b) {
+        stash(As[b], ra, qa, fa);
+        stash(Bs[b], rb, qb, fb);
+        if (!AK && sums) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cs += fa[j];
+        }
+    };
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int k0 = 0; k0 < a.K; k0 += 16) {
-        uint16_t av[8], bv[8];
+    fetch2(kb);
+    stash2(0);
+    __syncthreads();
+    const int oa = ((w & 1) * 32 + (lane & 31)) * LS + (lane >> 5) * 8;
+    const int ob = ((w >> 1) * 32 + (lane & 31)) * LS + (lane >> 5) * 8;
+    int b = 0;
+    for (int k0 = kb; k0 < ke; k0 += 32) {        // block-uniform
+        if (k0 + 32 < ke) fetch2(k0 + 32);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = k0 + kh + j;
-            const bool kin = k < a.K;
-            av[j] = to_bf16(kin && rm < a.M ? a.A[(int64_t)rm * a.sam + (int64_t)k * a.sak] : 0.f);
-            bv[j] = to_bf16(kin && cn < a.N ? a.B[(int64_t)k * a.sbk + (int64_t)cn * a.sbn] : 0.f);
+        for (int h = 0; h < 2; ++h) {
+            const bf16x8 A8 = *reinterpret_cast<const bf16x8*>(As[b] + oa + 16 * h);
+            const bf16x8 B8 = *reinterpret_cast<const bf16x8*>(Bs[b] + ob + 16 * h);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A8, B8, acc, 0, 0, 0);
         }
-        bf16x8 A8, B8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            A8[j] = __builtin_bit_cast(__bf16, av[j]);
-            B8[j] = __builtin_bit_cast(__bf16, bv[j]);
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A8, B8, acc, 0, 0, 0);
+        if (k0 + 32 < ke) stash2(b ^ 1);          // its readers passed the last barrier
+        __syncthreads();
+        b ^= 1;
     }
-    mm_store(a, acc, m0, cn, lane >> 5);
+    MmArgs o = a;
+    o.C = a.C + (int64_t)blockIdx.z * a.cz;
+    mm_store(o, acc, m0 + (w & 1) * 32, n0 + (w >> 1) * 32 + (lane & 31), lane >> 5);
+    if (!AK && sums) {                            // block-uniform: the four threads of a column, in order
+        float* red = reinterpret_cast<float*>(As[0]);
+        red[t] = cs;
+        __syncthreads();
+        if (w == 0 && m0 + lane < a.M)
+            a.colsum[(int64_t)blockIdx.z * a.cz + m0 + lane] =
+                ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
+    }
 }
 
-// The same product when both operands are contiguous in k (sak = sbk = 1),
-// K is a multiple of 16 and rows start 16-byte aligned: each lane's 8 k
-// values of A and of B come as two 16-byte loads, and the next k step's are
-// requested before this step's product.
-__device__ __forceinline__ bf16x8 pack8(const float4& u, const float4& v) {
-    bf16x8 r;
-    const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) r[j] = __builtin_bit_cast(__bf16, to_bf16(f[j]));
-    return r;
-}
-
-__global__ __launch_bounds__(256) void k_mm_vec(MmArgs a) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m0 = blockIdx.y * 64 + (w & 1) * 32;
-    const int n0 = blockIdx.x * 64 + (w >> 1) * 32;
-    const int rm = m0 + (lane & 31), cn = n0 + (lane & 31);
-    const int kh = (lane >> 5) * 8;
-    // rows past M / columns past N read row 0 / column 0 (in bounds) and are
-    // not stored
-    const float4* pa = reinterpret_cast<const float4*>(a.A + (int64_t)(rm < a.M ? rm : 0) * a.sam + kh);
-    const float4* pb = reinterpret_cast<const float4*>(a.B + (int64_t)(cn < a.N ? cn : 0) * a.sbn + kh);
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    float4 a0 = pa[0], a1 = pa[1], b0 = pb[0], b1 = pb[1];
-    for (int k0 = 16; k0 < a.K; k0 += 16) {
-        const float4 na0 = pa[k0 / 4], na1 = pa[k0 / 4 + 1], nb0 = pb[k0 / 4], nb1 = pb[k0 / 4 + 1];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pack8(a0, a1), pack8(b0, b1), acc, 0, 0, 0);
-        a0 = na0; a1 = na1; b0 = nb0; b1 = nb1;
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pack8(a0, a1), pack8(b0, b1), acc, 0, 0, 0);
-    mm_store(a, acc, m0, cn, lane >> 5);
+// g[i] = sum over the chunks z, in order, of part[z np + i]
+__global__ __launch_bounds__(256) void k_sum_chunks(int64_t np, int nz, const float* __restrict__ part,
+                                                    float* __restrict__ g) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    float s = 0.f;
+    for (int z = 0; z < nz; ++z) s += part[(int64_t)z * np + i];
+    g[i] = s;
 }
 
 // ------------------------------------------------------------ fused inference
@@ -148,7 +202,7 @@ __global__ __launch_bounds__(256) void k_mm_vec(MmArgs a) {
 // layer-wise kernels apply when they load them), weights come from the FP32
 // master parameters, and only the unstandardised outputs reach HBM.  Each
 // wave takes 32-column blocks of a layer in turn, both 32-row halves at once
-// (k order, products and epilogue as k_mm / k_mm_vec), so the outputs equal
+// (k order, products and epilogue as k_mm), so the outputs equal
 // the layer-wise path's bit for bit.  Limits: at most kFiL layers, widths up to kFiW.
 constexpr int kFiR = 64, kFiW = 256, kFiS = kFiW + 8, kFiL = 8;   // rows, max width, LDS row stride
 
@@ -273,14 +327,14 @@ __global__ void k_unstandardise(int64_t n, int d, float* __restrict__ Y, const f
     const int j = (int)(i % d);
     Y[i] = Y[i] * sd[j] + mu[j];
 }
-// rows of X (and Y) picked by idx into Xb (Yb), standardised
+// rows of X (and Y) picked by idx (null: in order) into Xb (Yb), standardised
 __global__ void k_gather_std(int64_t nb, int d, const int64_t* __restrict__ idx, const float* __restrict__ X,
                              const float* __restrict__ mu, const float* __restrict__ sd, float* __restrict__ Xb) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nb * d) return;
     const int64_t r = i / d;
     const int j = (int)(i - r * d);
-    Xb[i] = (X[idx[r] * d + j] - mu[j]) / sd[j];
+    Xb[i] = (X[(idx ? idx[r] : r) * d + j] - mu[j]) / sd[j];
 }
 // dY = 2 (Yp - Y) / (n d) and per-block partial sums of (Yp - Y)^2
 __global__ __launch_bounds__(256) void k_mse(int64_t n, int d, const float* __restrict__ Yp, const float* __restrict__ Y,
@@ -301,19 +355,6 @@ __global__ __launch_bounds__(256) void k_mse(int64_t n, int d, const float* __re
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
-// dZ = dH * gelu'(Z)
-__global__ void k_gelu_bwd(int64_t n, const float* __restrict__ dH, const float* __restrict__ Z, float* __restrict__ dZ) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dZ[i] = dH[i] * gelu_d(Z[i]);
-}
-// db[j] = sum_r dZ[r][j]  (one thread per column, rows in order: deterministic)
-__global__ void k_colsum(int64_t n, int d, const float* __restrict__ dZ, float* __restrict__ db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= d) return;
-    float s = 0.f;
-    for (int64_t r = 0; r < n; ++r) s += dZ[r * d + j];
-    db[j] = s;
-}
 __global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                        float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -328,6 +369,8 @@ __global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict
 
 inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+constexpr int kGradChunks = 32;           // row chunks of a weight gradient, at most
+
 }  // namespace
 
 struct Mlp {
@@ -339,6 +382,7 @@ struct Mlp {
     DevBuf norm;                          // in_mean, in_std, out_mean, out_std
     DevBuf act;                           // H_0..H_L and Z_0..Z_{L-1} for a batch
     DevBuf tmp, part, idx;
+    DevBuf gpart;                         // [chunk][np]: the row chunks' gradients
     int64_t cap = 0;                      // rows the activation buffers hold
     int64_t adam_t = 0;
     int layers() const { return (int)din.size(); }
@@ -379,14 +423,15 @@ int Mlp::reserve(int64_t rows) {
     return 0;
 }
 
-static hipError_t mm(const MmArgs& a, hipStream_t st) {
+static hipError_t mm(MmArgs a, hipStream_t st) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64));
-    auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool vec = a.sak == 1 && a.sbk == 1 && a.K >= 16 && a.K % 16 == 0 && a.sam % 4 == 0 && a.sbn % 4 == 0 &&
-                     al16(a.A) && al16(a.B);
-    if (vec) hipLaunchKernelGGL(k_mm_vec, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(k_mm, grid, dim3(256), 0, st, a);
+    if (a.kchunk <= 0 || a.kchunk > a.K) a.kchunk = a.K;
+    if ((a.ak ? a.sak : a.sam) != 1 || (a.bk ? a.sbk : a.sbn) != 1 || (a.colsum && a.ak)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), (unsigned)((a.K + a.kchunk - 1) / a.kchunk));
+    if (a.ak && a.bk) hipLaunchKernelGGL((k_mm<true, true>), grid, dim3(256), 0, st, a);
+    else if (a.ak) hipLaunchKernelGGL((k_mm<true, false>), grid, dim3(256), 0, st, a);
+    else if (!a.bk) hipLaunchKernelGGL((k_mm<false, false>), grid, dim3(256), 0, st, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
@@ -397,6 +442,7 @@ int Mlp::forward(int64_t n, hipStream_t st) {
         a.M = (int)n; a.N = dout[l]; a.K = din[l];
         a.A = A + hoff(l); a.sam = din[l]; a.sak = 1;
         a.B = P() + woff[l]; a.sbk = 1; a.sbn = din[l];          // B(k, j) = W[j][k]
+        a.ak = a.bk = true;
         a.bias = P() + boff[l];
         a.scm = dout[l];
         if (l + 1 < layers()) {
@@ -423,30 +469,39 @@ int Mlp::backward(int64_t n, const float* dY, hipStream_t st) {
     if (dY != bufA) return -1;
     float* dZ = bufA;
     float* dH = bufB;
+    // weight gradients sum over the rows: split into at most kGradChunks chunks
+    // of 128 rows or more, so that a minibatch's few 64 x 64 output tiles
+    // fill the chip; the chunks' gradients (parameter layout) meet at the end
+    // (the chunks' gradients take at most 256 MiB, or one chunk's)
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(kGradChunks, (int64_t(64) << 20) / np));
+    const int chunk = (int)(((n + most - 1) / most + 127) / 128 * 128);
+    const int nz = (int)((n + chunk - 1) / chunk);
+    if (gpart.alloc((size_t)nz * np * sizeof(float))) return -3;
+    float* GP = (float*)gpart.get();
     for (int l = layers() - 1; l >= 0; --l) {
-        // dW_l = dZ^T H_l : (dout x n) . (n x din)
+        // dW_l = dZ^T H_l : (dout x n) . (n x din), db_l = column sums of dZ
         MmArgs g{};
         g.M = dout[l]; g.N = din[l]; g.K = (int)n;
         g.A = dZ; g.sam = 1; g.sak = dout[l];
         g.B = A + hoff(l); g.sbk = din[l]; g.sbn = 1;
-        g.C = G() + woff[l]; g.scm = din[l]; g.epi = 0;
+        g.C = GP + woff[l]; g.scm = din[l]; g.epi = 0;
+        g.kchunk = chunk; g.cz = np; g.colsum = GP + boff[l];
         CFDWM_HIP(mm(g, st));
-        hipLaunchKernelGGL(k_colsum, dim3(nb256(dout[l])), dim3(256), 0, st, n, dout[l], (const float*)dZ, G() + boff[l]);
-        CFDWM_HIP(hipGetLastError());
         if (l == 0) break;
-        // dH_l = dZ W_l : (n x dout) . (dout x din);  dZ_{l-1} = dH_l * gelu'(Z_{l-1})
+        // dZ_{l-1} = (dZ W_l) * gelu'(Z_{l-1}) : (n x dout) . (dout x din)
         dH = dZ == bufA ? bufB : bufA;
         MmArgs h{};
         h.M = (int)n; h.N = din[l]; h.K = dout[l];
         h.A = dZ; h.sam = dout[l]; h.sak = 1;
         h.B = P() + woff[l]; h.sbk = din[l]; h.sbn = 1;
-        h.C = dH; h.scm = din[l]; h.epi = 0;
+        h.C = dH; h.scm = din[l]; h.epi = 3;
+        h.Z = A + zoff(l - 1);
+        h.ak = true;
         CFDWM_HIP(mm(h, st));
-        hipLaunchKernelGGL(k_gelu_bwd, dim3(nb256(n * din[l])), dim3(256), 0, st, n * din[l], (const float*)dH,
-                           (const float*)(A + zoff(l - 1)), dH);
-        CFDWM_HIP(hipGetLastError());
         dZ = dH;
     }
+    hipLaunchKernelGGL(k_sum_chunks, dim3(nb256(np)), dim3(256), 0, st, np, nz, (const float*)GP, G());
+    CFDWM_HIP(hipGetLastError());
     return 0;
 }
 
@@ -601,17 +656,14 @@ int cfdwm_mlp_loss_grad_device(cfdwm_mlp* h, int64_t n, const float* X, const fl
     Mlp& M = h->m;
     hipStream_t st = Engine::get().stream();
     if (M.reserve(n)) return -3;
-    std::vector<int64_t> id(n);
-    for (int64_t r = 0; r < n; ++r) id[r] = r;
-    if (M.idx.upload(id.data(), n * sizeof(int64_t), st)) return -3;
     float* A = (float*)M.act.get();
-    hipLaunchKernelGGL(k_gather_std, dim3(nb256(n * M.nin)), dim3(256), 0, st, n, M.nin, (const int64_t*)M.idx.get(), X,
+    hipLaunchKernelGGL(k_gather_std, dim3(nb256(n * M.nin)), dim3(256), 0, st, n, M.nin, (const int64_t*)nullptr, X,
                        (const float*)M.nin_mu(), (const float*)M.nin_sd(), A + M.hoff(0));
     CFDWM_HIP(hipGetLastError());
     if (int e = M.forward(n, st)) return e;
     // targets standardised into the dY buffer's slot, then MSE in place
     float* Yb = (float*)M.tmp.get() + (M.tmp.size() / sizeof(float)) / 2;
-    hipLaunchKernelGGL(k_gather_std, dim3(nb256(n * M.nout)), dim3(256), 0, st, n, M.nout, (const int64_t*)M.idx.get(), Y,
+    hipLaunchKernelGGL(k_gather_std, dim3(nb256(n * M.nout)), dim3(256), 0, st, n, M.nout, (const int64_t*)nullptr, Y,
                        (const float*)M.nout_mu(), (const float*)M.nout_sd(), Yb);
     CFDWM_HIP(hipGetLastError());
     const unsigned nbk = nb256(n * M.nout);

@@ -119,3 +119,33 @@ def test_fused_inference_equals_layerwise(shape):
     assert np.all(np.isfinite(big))
     assert np.array_equal(big, small), float(np.max(np.abs(big - small)))
     m.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nin,width,nh,nout,n", [(1, 1, 1, 1, 1), (33, 65, 2, 1, 31), (5, 64, 0, 3, 129),
+                                                 (30, 63, 1, 64, 128), (33, 256, 3, 65, 4173)])
+def test_gradient_at_tile_and_chunk_edges(nin, width, nh, nout, n):
+    """Loss and gradient at sizes around the 64 x 64 output tiles, the 32-wide
+    k steps and the 128-row chunks of the weight gradients.  Tolerance: FP32
+    sums against the oracle's float64 ones on the same bf16 operands (1e-6),
+    and the few operands whose rounding to bf16 flips between the two (2^-9
+    of an element each): 1e-4 of a parameter block's norm."""
+    import torch
+    from cfdwavemaker_amd.mlp import Mlp
+    dims, p = _net(nin, width, nh, nout, 16)
+    X, Y, norm = _data(max(n, 8), nin, nout, 17)
+    X, Y = X[:n].astype(np.float32), Y[:n].astype(np.float32)
+    m = Mlp(nin, width, nh, nout)
+    m.set_params(p)
+    m.set_norm(*norm)
+    loss, g = m.loss_grad(torch.tensor(X, device="cuda"), torch.tensor(Y, device="cuda"))
+    m.close()
+    normf = tuple(np.asarray(a, np.float32).astype(np.float64) for a in norm)
+    lr, gr = mlp_ref.loss_grad(p, dims, X, Y, normf, "bf16")
+    assert abs(loss - lr) <= 1e-4 * lr
+    q = 0
+    for d, o in dims:
+        for sz in (d * o, o):
+            a, b = g[q:q + sz], gr[q:q + sz]
+            assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), (d, o, sz)
+            q += sz
