@@ -327,4 +327,71 @@ int build_profile_basis_cached(double kmax, double h, int sign, double tol, int 
     return e.first;
 }
 
+namespace {
+DepthNodes nodes_of(int S, double a) {
+    DepthNodes N;
+    N.S = S; N.a = a;
+    for (int j = 0; j < S; ++j) {
+        const double xi = std::cos(3.14159265358979323846 * j / (S - 1));
+        N.xi.push_back(xi);
+        N.z.push_back(j == S - 1 ? -1.0 : -std::expm1(a * (1.0 - xi) / 2.0) / std::expm1(a));
+        N.w.push_back((j & 1 ? -1.0 : 1.0) * (j == 0 || j == S - 1 ? 0.5 : 1.0));
+    }
+    return N;
+}
+}  // namespace
+
+int build_depth_nodes(double kmaxh, DepthNodes& out) {
+    const int j = (int)std::ceil(std::log(std::max(kmaxh, 1e-6) / 0.1) / std::log(1.1));
+    const double X = 0.1 * std::pow(1.1, j);
+    static std::mutex mu;
+    static std::map<int, std::pair<int, DepthNodes>> cache;
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = cache.find(j);
+    if (it == cache.end()) {
+        // off-node depths, dense near the surface, and wavenumbers of all scales
+        constexpr int NZ = 64, NK = 48;
+        double zt[NZ], kt[NK], te[NZ][NK], tg[NZ][NK];
+        for (int b = 0; b < NK; ++b) kt[b] = X * std::pow((b + 1.0) / NK, 2.0);
+        for (int b = 0; b < NZ; ++b) {
+            zt[b] = -std::pow((b + 0.37) / NZ, 2.0);
+            for (int k = 0; k < NK; ++k) {
+                te[b][k] = std::exp(kt[k] * zt[b]);
+                tg[b][k] = std::exp(-kt[k] * (zt[b] + 2.0));
+            }
+        }
+        std::pair<int, DepthNodes> best{-1, DepthNodes()};
+        std::vector<double> pe(64 * NK), pg(64 * NK);
+        for (int S = 8; S <= 64 && best.first; S += 2) {
+            for (double a : {1.0, 1.5, 2.0, 2.5, 3.0, 4.0}) {
+                DepthNodes N = nodes_of(S, a);
+                for (int s = 0; s < S; ++s)
+                    for (int k = 0; k < NK; ++k) {
+                        pe[s * NK + k] = std::exp(kt[k] * N.z[s]);
+                        pg[s * NK + k] = std::exp(-kt[k] * (N.z[s] + 2.0));
+                    }
+                for (int b = 0; b < NZ && N.err <= 1e-13; ++b) {
+                    const double xi = 1.0 - 2.0 * std::log1p(-zt[b] * std::expm1(a)) / a;
+                    double den = 0, ve[NK] = {}, vg[NK] = {};
+                    for (int s = 0; s < S; ++s) {
+                        const double d = xi - N.xi[s];
+                        const double L = N.w[s] / (d == 0 ? 1e-290 : d);
+                        den += L;
+                        for (int k = 0; k < NK; ++k) {
+                            ve[k] += L * pe[s * NK + k];
+                            vg[k] += L * pg[s * NK + k];
+                        }
+                    }
+                    for (int k = 0; k < NK; ++k)
+                        N.err = std::max(N.err, std::fabs(ve[k] / den - te[b][k]) + std::fabs(vg[k] / den - tg[b][k]));
+                }
+                if (N.err <= 4e-15 && (best.first || N.err < best.second.err)) best = {0, N};
+            }
+        }
+        it = cache.emplace(j, best).first;
+    }
+    out = it->second.second;
+    return it->second.first;
+}
+
 }  // namespace cfdwm

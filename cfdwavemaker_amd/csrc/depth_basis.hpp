@@ -65,4 +65,18 @@ int build_profile_basis_cached(double kmax, double h, int sign, double tol, int 
 // ratio-1.1 grid; the basis is scale invariant), thread-safe.
 int build_depth_basis_cached(double kmax, double tmax, double tol, int rmax, DepthBasis& B);
 
+// Interpolation nodes for the profiles e^{kappa z} +- e^{-kappa (z + 2h)},
+// kappa in [0, kmax], on z in [-h, 0] to rounding: Chebyshev points xi_s in
+// [-1, 1] of the map z(xi) = -h (e^{a (1 - xi) / 2} - 1) / (e^a - 1), which
+// crowds them towards the surface where the profiles are steep, with their
+// barycentric weights.  Returns 0 with the fewest of 8, 10, ... 64 nodes whose
+// measured error is <= 4e-15 (profiles are <= 2), -1 when 64 do not suffice.
+// Scale invariant in kmax h; cached on a ratio-1.1 grid, thread-safe.
+struct DepthNodes {
+    int S = 0;
+    double a = 0, err = 0;
+    std::vector<double> z, xi, w;    // z in units of h
+};
+int build_depth_nodes(double kmaxh, DepthNodes& N);
+
 }  // namespace cfdwm

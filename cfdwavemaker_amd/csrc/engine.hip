@@ -47,6 +47,18 @@ int DevBuf::alloc(size_t bytes) {
     n_ = bytes;
     return 0;
 }
+bool DevBuf::try_alloc(size_t bytes) {
+    if (bytes <= n_ && p_) return true;
+    release();
+    if (bytes == 0) return true;
+    if (hipMalloc(&p_, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        p_ = nullptr;
+        return false;
+    }
+    n_ = bytes;
+    return true;
+}
 int DevBuf::upload(const void* src, size_t bytes, hipStream_t st) {
     if (alloc(bytes)) return -3;
     if (bytes) CFDWM_HIP(hipMemcpyAsync(p_, src, bytes, hipMemcpyHostToDevice, st));
@@ -84,6 +96,12 @@ hipEvent_t Engine::take_event() {
 hipStream_t Engine::side_stream() {
     if (!side_ && hipStreamCreateWithFlags(&side_, hipStreamNonBlocking) != hipSuccess) side_ = nullptr;
     return side_;
+}
+std::shared_ptr<QdSpace> Engine::qd_space() {
+    std::lock_guard<std::mutex> lk(qd_mu_);
+    auto s = qd_space_.lock();
+    if (!s) qd_space_ = s = std::make_shared<QdSpace>();
+    return s;
 }
 void Engine::prof_begin(hipStream_t st) {
     if (!prof_) return;
@@ -455,6 +473,46 @@ void Sea::release_qform() {
     qf_ext_ = false;
 }
 
+const Sea::QdMeta* Sea::qd_meta(int* rc) {
+    *rc = 0;
+    std::lock_guard<std::mutex> lk(qd_mu_);
+    if (qd_ || qd_none_) return qd_.get();
+    const PairTable& P = tab.filt;
+    const int N = tab.comp.n;
+    double kmx = 0;
+    for (const PairRec64& r : P.rec) kmx = std::max(kmx, std::max(std::fabs(r.kP), std::fabs(r.kM)));
+    DepthNodes D;
+    if (build_depth_nodes(kmx * tab.in.depth, D) != 0) {
+        qd_none_ = true;
+        return nullptr;
+    }
+    auto M = std::make_unique<QdMeta>();
+    M->npad = (N + 63) / 64 * 64;
+    M->S = D.S; M->a = D.a; M->err = D.err;
+    M->nf = 2;
+    for (const PairRec64& r : P.rec)
+        if (r.cvP != 0.0 || r.cvM != 0.0) { M->nf = 3; break; }
+    M->kend_h.assign(M->npad / 64, 0);
+    for (int i = 0; i < N; ++i)
+        if (P.mhi[i] > i + 1) {
+            int32_t& ke = M->kend_h[i / 64];
+            ke = std::max(ke, std::min(M->npad, (P.mhi[i] + 15) / 16 * 16));
+        }
+    std::vector<double> nd;
+    for (double z : D.z) nd.push_back(z * tab.in.depth);
+    nd.insert(nd.end(), D.xi.begin(), D.xi.end());
+    nd.insert(nd.end(), D.w.begin(), D.w.end());
+    hipStream_t st = Engine::get().stream();
+    if (M->nodes.upload(nd.data(), nd.size() * sizeof(double), st) ||
+        M->kend.upload(M->kend_h.data(), M->kend_h.size() * sizeof(int32_t), st) ||
+        hipStreamSynchronize(st) != hipSuccess) {         // host staging vectors go out of scope
+        *rc = -3;
+        return nullptr;
+    }
+    qd_ = std::move(M);
+    return qd_.get();
+}
+
 const Sea::SmitDev* Sea::smit_tables() {
     if (smit_) return smit_.get();
     std::vector<SmitComp> comp;
@@ -783,12 +841,19 @@ int Grid::fill_slots(int nslot, const double* slot_t, const int* slot_dst, bool 
         const int rc = qform_fill(nslot, slot_t, C.ncol, C.cols, C, L);
         if (rc < 0) return rc;
         qf_used = rc == 1;
+    } else {
+        const int rc = qd_fill(nslot, slot_t, C.ncol, C.cols, C, L);
+        if (rc < 0) return rc;
+        qf_used = rc == 1;
     }
     // with the pair sums on the matrix cores the column and level passes are
     // O(N) per column: split them over component segments when the grid alone
     // does not fill the GPU
     const int64_t ncomp = sea->tab.comp.n;
-    if (qf_used) C.nseg = pick_nseg(C.ncol * nslot, 64 * ncomp);
+    // (FP64: 16 components or more per segment; with fewer, the reduction
+    // over the segments takes longer than the sums)
+    const int64_t crec = (sizeof(R) == 8 ? 4 : 64) * ncomp;
+    if (qf_used) C.nseg = pick_nseg(C.ncol * nslot, crec);
     C.seg = qf_used ? sea->comp_segments(C.nseg) : sea->segments(false, C.nseg);
     if (!C.seg) return -3;
     // the linear-term bases (L.lin_c, set with the forms) take all 16 levels
@@ -797,7 +862,7 @@ int Grid::fill_slots(int nslot, const double* slot_t, const int* slot_dst, bool 
     const bool lin16 = qf_used && L.lin_c && level_chunk == 8 && g.nl <= 16;
     const int lchunk = lin16 ? 16 : level_chunk;
     const int64_t lthr = level_threads(nslot, C.ncol, g.nl, lchunk, true);
-    const int lseg = pick_nseg(lthr, qf_used ? 64 * ncomp : nrec);
+    const int lseg = pick_nseg(lthr, qf_used ? crec : nrec);
     if constexpr (sizeof(R) == 4) {
         if (!lin16) L.lin_c = nullptr;
     }
@@ -1056,6 +1121,87 @@ int Grid::qform_fill(int nslot, const double* slot_t, int64_t ncol, const int32_
     return 1;
 }
 
+int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<double>& C,
+                  LevelJob<double>& L) {
+    if (!qform_ || sea->nfilt() == 0 || ncol <= 0) return 0;
+    // a fill of few points is over in the pair loop (split over pair segments)
+    // before the forms' few waves have walked their tables: one update at 1024
+    // components takes 4.1 ms in the pair loop against 5.3 at 1024 points, 6.1
+    // against 5.3 at 2048; with 312 components 0.89 against 0.29 at 512 points
+    if ((int64_t)nslot * ncol * g.nl < 2 * ((sea->tab.comp.n + 63) / 64 * 64)) return 0;
+    const CompTable& c = sea->tab.comp;
+    double scale[4] = {1, 1, 1, 1};
+    for (int s = 0; s < nslot; ++s) {
+        // one ramp factor for all components at a slot's time
+        scale[s] = freq_ramp_host(slot_t[s], c.rt[0], c.ts[0], c.du[0]);
+        for (int i = 1; i < c.n; ++i)
+            if (freq_ramp_host(slot_t[s], c.rt[i], c.ts[i], c.du[i]) != scale[s]) return 0;
+    }
+    // the nodes span [-depth of the sea, 0]
+    if (g.h > sea->tab.in.depth) return 0;
+    int rc = 0;
+    const Sea::QdMeta* M = sea->qd_meta(&rc);
+    if (!M) return rc;
+    const int npad = M->npad, S = M->S, nf = M->nf, nform = 1 + nf * S;
+    if (npad > 4096) return 0;                    // a node's tables would exceed 768 MiB
+    const int64_t P = (int64_t)nslot * ncol;
+    // workspace: at most 512 MiB of Z operands and 256 MiB of tables (or one
+    // node's); without the memory the pair loop runs
+    const int64_t ppad_all = (P + 63) / 64 * 64;
+    const int64_t chunk = std::min(ppad_all, std::max<int64_t>(64, (int64_t(512) << 20) / (16LL * npad) / 64 * 64));
+    const size_t zn = (size_t)chunk * npad, nn = (size_t)npad * npad;
+    const int grp = (int)std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(256) << 20) / (int64_t)(2 * nf * nn * sizeof(double))));
+    if (!qout_.try_alloc((size_t)nform * ppad_all * sizeof(double))) return 0;
+    if (!qd_space_) qd_space_ = Engine::get().qd_space();
+    std::lock_guard<std::mutex> lk(qd_space_->mu);
+    if (!qd_space_->z.try_alloc(2 * zn * sizeof(double)) || !qd_space_->tab.try_alloc((2 + 2 * nf * grp) * nn * sizeof(double)))
+        return 0;
+    const SeaDev<double>& D = sea->dev<double>();
+    hipStream_t st = Engine::get().stream();
+    QdJob J;
+    J.n = c.n; J.npad = npad; J.ncol = ncol; J.cols = cols; J.g = g;
+    for (int s = 0; s < nslot; ++s) J.slot_t[s] = slot_t[s];
+    J.x0 = sea->tab.in.x0; J.y0 = sea->tab.in.y0;
+    J.ph = D.ph;
+    J.zc = (double*)qd_space_->z.get();
+    J.zs = J.zc + zn;
+    J.b = (const double*)qd_space_->tab.get();
+    J.kend = (const int32_t*)M->kend.get();
+    J.out = (double*)qout_.get();
+    J.ostride = ppad_all;
+    J.nf = nf;
+    QdBuild B;
+    B.nf = nf;
+    B.n = c.n; B.npad = npad; B.frow = D.frow; B.fmhi = D.fmhi; B.uvw = D.fuvw; B.x = D.fx;
+    B.zs = (const double*)M->nodes.get();
+    B.b = (double*)qd_space_->tab.get();
+    for (J.p0 = 0; J.p0 < P; J.p0 += chunk) {
+        J.P = std::min(chunk, P - J.p0);
+        J.ppad = (J.P + 63) / 64 * 64;
+        PROF("k_qd_zgen", launch_qd_zgen(J, st));
+        for (int q = 0; q < S; q += grp) {
+            B.eta = q == 0;
+            B.node0 = q;
+            B.nn = std::min(grp, S - q);
+            J.form0 = q == 0 ? 0 : 1 + nf * q;
+            J.nform = (q == 0 ? 1 : 0) + nf * B.nn;
+            PROF("k_qd_build", launch_qd_build(B, st));
+            PROF("k_qd_forms", launch_qd_forms(J, st));
+        }
+    }
+    C.pairs = 0;
+    C.q2d = J.out;
+    L.qd = J.out + ppad_all;
+    L.qd_S = S;
+    L.qd_nf = nf;
+    L.qd_stride = ppad_all;
+    L.qd_xi = (const double*)M->nodes.get() + S;
+    L.qd_a = M->a;
+    L.qd_h = sea->tab.in.depth;
+    for (int s = 0; s < 4; ++s) C.q2scale[s] = L.qf_scale[s] = scale[s];
+    return 1;
+}
+
 // initialize_kinematics slot times (lsgrid_spline.cpp:678, :767)
 void Grid::init_slot_times(double* tt) const {
     const double t0i = d.t0;
@@ -1115,6 +1261,7 @@ size_t Grid::refill_z_bytes() const {
 
 void Grid::release_workspace() {
     zbuf_.release();
+    qd_space_.reset();
     qs_key_.release();
     qs_rec_.release();
     qs_tmp_.release();

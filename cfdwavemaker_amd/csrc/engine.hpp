@@ -29,6 +29,7 @@ struct ColumnJob {
     const float* q2 = nullptr;            // [nq2][q2stride] per-point partials (GRID)
     int nq2 = 0;
     int64_t q2stride = 0;
+    const double* q2d = nullptr;          // GRID, FP64: the eta2 form's values (scaled with q2scale)
     double q2scale[4] = {1, 1, 1, 1};     // per slot ramp factor of the partials (GRID)
     double q2_rt = 0, q2_ts = 0, q2_du = 0;  // POINTS: the ramp triple shared by all components
     double *o_eta1 = nullptr, *o_eta2 = nullptr, *o_gx = nullptr, *o_gy = nullptr, *o_gz = nullptr, *o_gp = nullptr;
@@ -71,6 +72,13 @@ struct LevelJob {
     const float* lin_c = nullptr;         // [n][4 x 16]: a(k), a(2k), b(k), b(2k), zeros past the ranks
     const float* lin_mu = nullptr;        // [4][16]: m_q log2 e, -2 h m_q log2 e (cosh-type), the same (sinh-type)
     int lin_R = 0, lin_Rw = 0;
+    // GRID, FP64: u, v, w pair sums at the depth nodes (qform64.hip), carried
+    // to the levels by barycentric interpolation in xi = 1 - 2 ln(1 - z/h (e^a - 1)) / a
+    const double* qd = nullptr;           // [qd_nf qd_S][qd_stride]: u, v, w (qd_nf 2: u, w) at node 0, at node 1, ...
+    int qd_S = 0, qd_nf = 3;
+    int64_t qd_stride = 0;
+    const double* qd_xi = nullptr;        // [qd_S] nodes, [qd_S] barycentric weights
+    double qd_a = 0, qd_h = 1;
     const Segment* seg = nullptr;         // nseg segments of the table in use (blockIdx.y)
     int nseg = 1;
     double* partial = nullptr;            // nseg > 1: [seg][thread][3 LC + 6] partial sums
@@ -175,6 +183,10 @@ hipError_t launch_query_sort(int64_t n, const GridGeom& g, const TQ* x, const TQ
 hipError_t launch_qf_zgen(const QfJob& J, hipStream_t st);
 hipError_t launch_qf_forms(const QfJob& J, hipStream_t st);
 hipError_t launch_qf_build(const QfBuild& B, hipStream_t st);
+// FP64 fills (qform64.hip): Z operands, one group's tables, one group's forms
+hipError_t launch_qd_zgen(const QdJob& J, hipStream_t st);
+hipError_t launch_qd_build(const QdBuild& B, hipStream_t st);
+hipError_t launch_qd_forms(const QdJob& J, hipStream_t st);
 hipError_t launch_qf_persist(const QfJob* jobs, const QfTile* tiles, int ntiles, int blocks, int nlv, hipStream_t st);
 // eta range of the columns of a fill (minus swl) -> eb[2]; then per filtered
 // pair record the levels where its profile exponentials exceed e^{-T}
@@ -221,6 +233,8 @@ public:
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     int alloc(size_t bytes);                 // keeps contents when large enough
+    // as alloc, but a failed allocation is no error: false, and the buffer empty
+    bool try_alloc(size_t bytes);
     int upload(const void* src, size_t bytes, hipStream_t st);
     void* get() const { return p_; }
     size_t size() const { return n_; }
@@ -236,6 +250,16 @@ struct KernelTimes {
     int64_t count = 0;
 };
 
+// Workspace of the FP64 forms: Z operands of one chunk of points and the
+// tables of one group of forms, both rebuilt by every fill.  One for all
+// grids: work on the library stream runs in order, and mu is held while a
+// fill's launches are queued, so that fills from several threads do not
+// interleave.  The grids that used it hold it; it is freed with the last.
+struct QdSpace {
+    std::mutex mu;
+    DevBuf z, tab;
+};
+
 class Engine {
 public:
     static Engine& get();
@@ -244,6 +268,7 @@ public:
     // a second stream (default priority) for work that overlaps the main
     // stream's, forked and joined with events; created on first use
     hipStream_t side_stream();
+    std::shared_ptr<QdSpace> qd_space();
     // timing: record an event pair around a launch when enabled
     void prof_enable(bool on) { prof_ = on; }
     bool prof_on() const { return prof_; }
@@ -260,6 +285,8 @@ private:
     std::map<std::string, KernelTimes> times_;
     std::vector<hipEvent_t> pool_;
     hipEvent_t take_event();
+    std::mutex qd_mu_;
+    std::weak_ptr<QdSpace> qd_space_;
 };
 
 // A launch timed with an event pair when timing is on; errors return -3.
@@ -346,6 +373,17 @@ public:
     // stay valid until release_qform or the memory's reuse.
     int qform_tables_into(void* mem, const QfTables** out);
     void release_qform();
+    // FP64: the depth nodes of this sea's profiles and the tile ends of its
+    // pair table (built once); null when no node set of at most 64 reaches
+    // rounding (kmax h beyond about 600), or on a device error (*rc < 0)
+    struct QdMeta {
+        int npad = 0, S = 0, nf = 3;         // nf 2: every v coefficient is zero (a sea along x)
+        double a = 0, err = 0;
+        DevBuf nodes;                        // [S] depths, [S] xi, [S] barycentric weights
+        DevBuf kend;
+        std::vector<int32_t> kend_h;
+    };
+    const QdMeta* qd_meta(int* rc);
     // bf16 products per term of the forms (3: hi/lo split, 1: hi only) and the
     // depth-basis tolerance (0: 1e-6 for 3 products, 1e-4 for 1 product)
     int qf_products = 3;
@@ -371,6 +409,9 @@ private:
     std::map<std::pair<bool, int>, std::unique_ptr<DevBuf>> seg_cache_;
     std::map<int, std::unique_ptr<DevBuf>> cseg_cache_;
     std::unique_ptr<QfTables> qf_;
+    std::unique_ptr<QdMeta> qd_;
+    std::mutex qd_mu_;
+    bool qd_none_ = false;
     int qform_build(QfTables& T, uint16_t* b, uint16_t* beta);
     bool qf_ext_ = false;                    // the tables live in caller memory
 public:
@@ -494,6 +535,10 @@ private:
     void qform_attach(ColumnJob<float>& C, LevelJob<float>& L);
     int qform_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<float>& C,
                    LevelJob<float>& L);
+    // the FP64 forms of a fill: 1 when they ran, 0 when the pair loop has to, < 0 on error
+    std::shared_ptr<QdSpace> qd_space_;
+    int qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<double>& C,
+                LevelJob<double>& L);
     void init_slot_times(double* tt) const;
 public:
     // batched refill over many grids (refill_batched)

@@ -123,6 +123,8 @@ __device__ __forceinline__ void col_store(const SeaDev<R>& S, const ColumnJob<R>
             double q = 0.;
             for (int k = 0; k < J.nq2; ++k) q += (double)J.q2[(int64_t)k * J.q2stride + P.q];
             e2 += J.q2scale[P.slot] * q;
+        } else if (J.q2d) {
+            e2 += J.q2scale[P.slot] * J.q2d[P.q];
         }
         J.eta_grid[(int64_t)J.slot_dst[P.slot] * J.ncell + P.col] = (R)(v[0] + e2 + S.swl);
     } else {
@@ -599,7 +601,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
         const bool own = i >= sg.own_lo && i < sg.own_hi;
         const bool sec = secf && (direct || (sizeof(R) == 4 ? row_active(S.rowActive, i) : S.rowActive[i] != 0));
         // (form-assisted fills, F8, launch only with the forms: no pair rows)
-        const bool prs = F8 == 0 && sec && !(GRID && J.qf) && i >= sg.rlo && i < sg.rhi;
+        const bool prs = F8 == 0 && sec && !(GRID && (J.qf || J.qd)) && i >= sg.rlo && i < sg.rhi;
         if (!own && !prs) continue;
         const PhaseRec pi = ld_rec<R>(S.ph, i);
         const CompRec<R> c = ld_rec<R>(S.cr, i);
@@ -823,6 +825,44 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
                 U[l] += sc * (double)su[l];
                 V[l] += sc * (double)sv[l];
                 W[l] += sc * (double)sw[l];
+            }
+        }
+    }
+    if constexpr (GRID && sizeof(R) == 8) {
+        if (J.qd && blockIdx.y == 0) {
+            // pair sums from the depth nodes: sum_s w_s Q_s / (xi - xi_s) over
+            // sum_s w_s / (xi - xi_s); a level on a node takes that node's
+            // value through a weight of 1e290
+            const double em = expm1(J.qd_a) / J.qd_h;
+            double xi[LC], den[LC], su[LC], sv[LC], sw[LC];
+#pragma unroll
+            for (int l = 0; l < LC; ++l) {
+                xi[l] = 1. - 2. * (log1p(-zp[l] * em) / J.qd_a);
+                den[l] = su[l] = sv[l] = sw[l] = 0.;
+            }
+            const double* Q = J.qd + PP.cq;
+            for (int s = 0; s < J.qd_S; ++s) {
+                const double xs = ld_const(J.qd_xi, s), ws = ld_const(J.qd_xi, J.qd_S + s);
+                const double qu = Q[(int64_t)(J.qd_nf * s) * J.qd_stride];
+                const double qv = J.qd_nf == 3 ? Q[(int64_t)(3 * s + 1) * J.qd_stride] : 0.;
+                const double qw = Q[(int64_t)(J.qd_nf * (s + 1) - 1) * J.qd_stride];
+#pragma unroll
+                for (int l = 0; l < LC; ++l) {
+                    const double d = xi[l] - xs;
+                    const double b = ws / (d == 0. ? 1e-290 : d);
+                    den[l] += b;
+                    su[l] = fma(b, qu, su[l]);
+                    sv[l] = fma(b, qv, sv[l]);
+                    sw[l] = fma(b, qw, sw[l]);
+                }
+            }
+            const double sc = J.qf_scale[PP.slot];
+#pragma unroll
+            for (int l = 0; l < LC; ++l) {
+                const double f = sc / den[l];
+                U[l] += f * su[l];
+                V[l] += f * sv[l];
+                W[l] += f * sw[l];
             }
         }
     }

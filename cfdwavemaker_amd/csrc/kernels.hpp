@@ -137,6 +137,38 @@ struct QfBuild {
                                           // and form f > 0 to b at index f - 1
 };
 
+// FP64 quadratic forms of an s-grid fill (qform64.hip): form 0 is eta2, form
+// 1 + nf s + f the field f (u, v, w; u, w when nf is 2) at depth node s.  Z holds cos and sin of
+// ppad points x npad components, b the tables of nform forms from form0 on
+// ([nform][2][npad x npad] in 16 x 8 tiles).
+struct QdJob {
+    int64_t p0 = 0, P = 0, ppad = 0;     // chunk of points [p0, p0 + P), padded to 64
+    int n = 0, npad = 0;                  // components, padded to 64
+    int64_t ncol = 0;
+    const int32_t* cols = nullptr;
+    GridGeom g{};
+    double slot_t[4] = {0, 0, 0, 0};
+    double x0 = 0, y0 = 0;
+    const PhaseRec* ph = nullptr;
+    double *zc = nullptr, *zs = nullptr;  // ppad x npad each
+    const double* b = nullptr;
+    int form0 = 0, nform = 0, nf = 3;
+    const int32_t* kend = nullptr;        // per 64-row tile of i: end of its m range (multiple of 16)
+    double* out = nullptr;                // [forms][ostride]
+    int64_t ostride = 0;
+};
+struct QdBuild {
+    int n = 0, npad = 0;
+    int eta = 0;                          // eta2's tables first
+    int node0 = 0, nn = 0, nf = 3;        // the nf fields at nodes node0 .. node0 + nn
+    const int64_t* frow = nullptr;
+    const int32_t* fmhi = nullptr;
+    const UvwRec<double>* uvw = nullptr;
+    const XRec<double>* x = nullptr;
+    const double* zs = nullptr;           // node depths
+    double* b = nullptr;                  // [2 eta + 2 nf nn][npad x npad]
+};
+
 // Smit et al. s-coordinate point evaluation (smit.hip).  eta1/eta2 are the
 // points' Sharma-Dean elevations (eta2 unused for order < 1); sc and sp are
 // the Smit coefficients of the components and of the filtered pair table

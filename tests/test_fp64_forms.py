@@ -1,0 +1,78 @@
+"""FP64 s-grid fills through the depth nodes and quadratic forms: grids around the
+tile edges against the oracle's column body, and the forms against the pair loop."""
+import numpy as np
+import pytest
+
+from cfdwavemaker_amd.seastate import make_sea
+from tests.conftest import scaled_err
+
+# rounding of the interpolation (4e-15 of a profile of size <= 2) and of FP64
+# sums over up to 2e4 pairs, far inside the library's FP64 contract of 1e-9
+TOL = 1e-11
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from cfdwavemaker_amd import engine
+    engine.load()
+    return engine
+
+
+def _ignore(dom, frac):
+    return (dom[0], dom[0] + frac * (dom[1] - dom[0]), dom[2], dom[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nfreq,ndir,nx,ny,nl,kw", [
+    (2, 1, 40, 26, 4, {}),                       # one pair
+    (63, 1, 16, 16, 5, {}),                      # one short 64-row tile
+    (64, 1, 17, 16, 4, {}),                      # one whole tile
+    (13, 5, 33, 8, 7, {}),                       # 65 components: a second tile of one row
+    (24, 8, 8, 9, 16, dict(depth=150.0)),        # deep: more nodes
+    (40, 4, 11, 9, 11, dict(depth=6.0)),         # shallow: fewest nodes
+    (48, 3, 64, 4, 4, dict(bandwidth=0.7, cutoff=1.9)),   # filtered rows end early
+    (30, 4, 20, 11, 6, dict(swl=1.5, ignore=0.4)),
+])
+def test_fill_and_update_vs_oracle(eng, oracle, nfreq, ndir, nx, ny, nl, kw):
+    s = make_sea(nfreq, 3.0, 9.0, kw.get("depth", 40.0), seed=nfreq, ndir=ndir).as_dict()
+    for k in ("bandwidth", "cutoff", "swl"):
+        if k in kw:
+            s[k] = kw[k]
+    dom = (10.0, 10.0 + 7.0 * max(nx - 1, 1), -5.0, -5.0 + 6.0 * max(ny - 1, 1))
+    ig = _ignore(dom, kw["ignore"]) if "ignore" in kw else (1e12, -1e12, 1e12, -1e12)
+    args = (dom, nx, ny, nl, 3.0, 0.5, 0.7, 1.5, s["depth"], s.get("swl", 0.0), ig, 0)
+    g = eng.Sea(s, precision=eng.FP64, with_direct=False).grid(*args)
+    o = oracle.sea(s).grid(*args)
+    for step in range(2):
+        if step:
+            g.force_update(3.75)
+            o.force_update(3.75)
+        for f in ("ETA", "UX", "UY", "UZ"):
+            a, b = g.export(f), o.export(f)
+            if not np.any(b):
+                assert not np.any(a), f
+                continue
+            assert scaled_err(a, b) <= TOL, (step, f, scaled_err(a, b))
+
+
+@pytest.mark.gpu
+def test_forms_and_pair_loop_agree(eng, monkeypatch):
+    """The same fill through both routes (a grid of fewer points than twice
+    the padded component count takes the pair loop)."""
+    s = make_sea(20, 3.0, 9.0, 40.0, seed=4, ndir=4).as_dict()
+    dx = 8.0
+    big = eng.Sea(s, with_direct=False).grid((0.0, 31 * dx, 0.0, 31 * dx), 32, 32, 4, 0.0, 0.5, 0.7, 1.5, 40.0)
+    small = eng.Sea(s, with_direct=False).grid((0.0, 2 * dx, 0.0, 2 * dx), 3, 3, 4, 0.0, 0.5, 0.7, 1.5, 40.0)
+    for f, tail in (("ETA", ()), ("UX", (4,)), ("UY", (4,)), ("UZ", (4,))):
+        a = big.export(f).reshape((4, 32, 32) + tail)[:, :3, :3].ravel()
+        assert scaled_err(a, small.export(f)) <= TOL, f
+
+
+@pytest.mark.gpu
+def test_components_ramped_apart_take_the_pair_loop(eng, oracle):
+    s = make_sea(12, 3.0, 9.0, 40.0, seed=5).as_dict()
+    s["ramptime"], s["starttime"], s["duration"] = np.linspace(1, 4, 12), np.zeros(12), np.full(12, 1e6)
+    args = ((0.0, 100.0, 0.0, 60.0), 32, 16, 4, 0.5, 0.5, 0.7, 1.5, 40.0)
+    g, o = eng.Sea(s, with_direct=False).grid(*args), oracle.sea(s).grid(*args)
+    for f in ("ETA", "UX", "UZ"):
+        assert scaled_err(g.export(f), o.export(f)) <= TOL, f
