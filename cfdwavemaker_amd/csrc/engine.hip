@@ -546,6 +546,13 @@ template <>
 const SeaDev<float>& Sea::dev<float>() const { return d32_; }
 
 namespace {
+// points padded to whole tiles of the forms kernels
+int64_t qf_pad(int64_t n) { return (n + kQfTile - 1) / kQfTile * kQfTile; }
+// Z operands of one chunk of points: 8 bytes per (point, component), at most 2 GiB
+int64_t qf_chunk_cap(int npad) {
+    return std::max<int64_t>(kQfTile, ((int64_t)1 << 31) / ((int64_t)npad * 8) / kQfTile * kQfTile);
+}
+
 // FP32 point batches: the filtered eta2 pair sum as the MFMA quadratic form
 // (form 0 of the sea's tables) when the batch is large and every component
 // has the same frequency-ramp triple (the ramp factor is then one number per
@@ -560,9 +567,8 @@ int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, cons
     const Sea::QfTables* T = nullptr;
     if (const int rc = s.qform_tables(&T); rc != 1) return rc;
     const int npad = T->npad;
-    const int64_t ppad_all = (n + 127) / 128 * 128;
-    const int64_t cap = std::max<int64_t>(128, ((int64_t)1 << 31) / ((int64_t)npad * 8) / 128 * 128);
-    const int64_t chunk = std::min(ppad_all, cap);
+    const int64_t ppad_all = qf_pad(n);
+    const int64_t chunk = std::min(ppad_all, qf_chunk_cap(npad));
     const size_t zn = (size_t)chunk * npad;
     if (s.qz.alloc(zn * 4 * sizeof(uint16_t)) || s.qo.alloc((size_t)ppad_all * sizeof(float))) return -3;
     QfJob Q;
@@ -577,7 +583,7 @@ int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, cons
     Q.b = T->nlv == 1 ? T->betap : T->bp;
     Q.nbarr = 4; Q.nlv = 3;
     Q.ftype = (const int8_t*)T->ftype.get();
-    Q.nform = 1;
+    Q.nform = Q.ncos = 1;
     Q.kend = (const int32_t*)T->kend.get();
     Q.out = (float*)s.qo.get();
     Q.ostride = ppad_all;
@@ -585,7 +591,7 @@ int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, cons
     for (int64_t p0 = 0; p0 < n; p0 += chunk) {
         Q.p0 = p0;
         Q.P = std::min(chunk, n - p0);
-        Q.ppad = (Q.P + 127) / 128 * 128;
+        Q.ppad = qf_pad(Q.P);
         PROF("k_qf_zgen", launch_qf_zgen(Q, st));
         PROF("k_qf_forms", launch_qf_forms(Q, st));
     }
@@ -939,10 +945,8 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
     qf_skip = QF_USED;
     const int npad = T->npad, R = T->rank;
     const int64_t P = (int64_t)nslot * ncol;
-    const int64_t ppad_all = (P + 127) / 128 * 128;
-    // Z operands of one chunk of points: 8 bytes per (point, component), at most 2 GiB
-    const int64_t cap = std::max<int64_t>(128, ((int64_t)1 << 31) / ((int64_t)npad * 8) / 128 * 128);
-    qf_chunk_ = std::min(ppad_all, cap);
+    const int64_t ppad_all = qf_pad(P);
+    qf_chunk_ = std::min(ppad_all, qf_chunk_cap(npad));
     qf_P_ = P;
     const size_t zn = (size_t)qf_chunk_ * npad;
     uint16_t* z = nullptr;
@@ -968,22 +972,24 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
     Q.ostride = ppad_all;
     Q.p0 = 0;
     Q.P = std::min(qf_chunk_, P);
-    Q.ppad = (Q.P + 127) / 128 * 128;
+    Q.ppad = qf_pad(Q.P);
     qf_split_ = T->nlv == 1;
     if (!qf_split_) {                             // every form, three products per term
         Q.b = T->bp;
         Q.nbarr = 4; Q.nlv = 3;
         Q.nform = T->nform;
+        Q.ncos = 1 + 2 * R;
     } else {                                      // eta2 at three products; velocity forms at one
         Q.b = T->betap;
         Q.nbarr = 4; Q.nlv = 3;
-        Q.nform = 1;
+        Q.nform = Q.ncos = 1;
         QfJob& V = qj2_;
         V = Q;
         V.b = T->bp;
         V.nbarr = T->nbarr; V.nlv = 1;
         V.ftype = Q.ftype + 1;
         V.nform = T->nform - 1;
+        V.ncos = 2 * R;
         V.out = Q.out + ppad_all;
     }
     // executed MFMA flops per padded point and form: a 128-wide i tile runs
@@ -1028,7 +1034,7 @@ int Grid::qform_run() {
     for (int64_t p0 = 0; p0 < qf_P_; p0 += qf_chunk_) {
         Q.p0 = p0;
         Q.P = std::min(qf_chunk_, qf_P_ - p0);
-        Q.ppad = (Q.P + 127) / 128 * 128;
+        Q.ppad = qf_pad(Q.P);
         PROF("k_qf_zgen", launch_qf_zgen(Q, st));
         if (qf_split_) {
             // eta2 at three products, then the velocity forms at one.  With
@@ -1253,9 +1259,8 @@ size_t Grid::refill_z_bytes() const {
     const Sea::QfTables* T = nullptr;
     if (sea->qform_meta(&T) != 1) return 0;
     const int64_t ncol = d.ignore_at_init ? nact_ : (int64_t)g.nx * g.ny;
-    const int64_t ppad = (4 * ncol + 127) / 128 * 128;
-    const int64_t cap = std::max<int64_t>(128, ((int64_t)1 << 31) / ((int64_t)T->npad * 8) / 128 * 128);
-    if (ppad > cap) return 0;
+    const int64_t ppad = qf_pad(4 * ncol);
+    if (ppad > qf_chunk_cap(T->npad)) return 0;
     return (size_t)ppad * T->npad * 4 * sizeof(uint16_t);
 }
 
@@ -1274,31 +1279,38 @@ struct BatchShape {
     int order, blocks, gf, gp;
 };
 
+// point tiles and forms (or form pairs) of a job in a launch of one kind
+int batch_ptiles(const QfJob& J, int kind) { return (int)(kind == kQfTileEta ? (J.P + 127) / 128 : J.ppad / 256); }
+int batch_forms(const QfJob& J, int kind) { return kind == kQfTilePair ? qf_pairs(J.nform, J.ncos) : J.nform; }
+
 // Tile lists of a batched launch.  order 0: all tiles by decreasing cost
 // (point-tile cost ~ the job's i-range work), so round-robin blocks get equal
 // shares; order 1: job by job (decreasing cost), inside a job groups of gf
 // forms x gp point tiles (cache locality of the job's tables and operands:
 // consecutive blocks share a group's B tables and Z tiles).
-std::vector<QfTile> batch_tiles(const std::vector<QfJob>& jobs, const std::vector<double>& cost, const BatchShape& b) {
+std::vector<QfTile> batch_tiles(const std::vector<QfJob>& jobs, const std::vector<double>& cost, const BatchShape& b,
+                                int kind) {
     std::vector<int> idx(jobs.size());
     for (size_t j = 0; j < jobs.size(); ++j) idx[j] = (int)j;
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int c) { return cost[a] > cost[c]; });
     std::vector<QfTile> t;
-    if (b.order == 0) {
-        for (int j : idx) {
-            const int npt = (int)(jobs[j].ppad / 128);
-            for (int f = 0; f < jobs[j].nform; ++f)
-                for (int p = 0; p < npt; ++p) t.push_back(QfTile{j, p, f, 0});
-        }
-        std::stable_sort(t.begin(), t.end(), [&](const QfTile& a, const QfTile& c) { return cost[a.job] > cost[c.job]; });
-    } else {
-        const int gf = std::max(1, b.gf), gp = std::max(1, b.gp);
-        for (int j : idx) {
-            const int npt = (int)(jobs[j].ppad / 128), nf = jobs[j].nform;
+    auto put = [&](int j, int p, int q) {
+        int form = q;
+        bool two = false;
+        if (kind == kQfTilePair) qf_pair(jobs[j].nform, jobs[j].ncos, q, &form, &two);
+        t.push_back(QfTile{j, p, form, two ? 1 : 0});
+    };
+    for (int j : idx) {
+        const int npt = batch_ptiles(jobs[j], kind), nf = batch_forms(jobs[j], kind);
+        if (b.order == 0) {
+            for (int f = 0; f < nf; ++f)
+                for (int p = 0; p < npt; ++p) put(j, p, f);
+        } else {
+            const int gf = std::max(1, b.gf), gp = std::max(1, b.gp);
             for (int f0 = 0; f0 < nf; f0 += gf)
                 for (int p0 = 0; p0 < npt; p0 += gp)
                     for (int f = f0; f < std::min(nf, f0 + gf); ++f)
-                        for (int p = p0; p < std::min(npt, p0 + gp); ++p) t.push_back(QfTile{j, p, f, 0});
+                        for (int p = p0; p < std::min(npt, p0 + gp); ++p) put(j, p, f);
         }
     }
     return t;
@@ -1325,9 +1337,9 @@ DevBuf& batch_arena() {
 }
 
 struct TuneKey {
-    int nlv, jobs_log2, tiles_log2;
+    int kind, jobs_log2, tiles_log2;
     bool operator<(const TuneKey& o) const {
-        if (nlv != o.nlv) return nlv < o.nlv;
+        if (kind != o.kind) return kind < o.kind;
         return jobs_log2 != o.jobs_log2 ? jobs_log2 < o.jobs_log2 : tiles_log2 < o.tiles_log2;
     }
 };
@@ -1436,8 +1448,8 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
         // and their costs; a grid whose velocity forms take one product adds
         // its eta2 form to the three-product list and its velocity forms to
         // the one-product list
-        std::vector<QfJob> jobs3, jobs1;
-        std::vector<double> cost3, cost1;
+        std::vector<QfJob> jobs3, jobse, jobs1;
+        std::vector<double> cost3, coste, cost1;
         std::vector<char> joined(grp.size(), 0);
         for (size_t k = 0; k < grp.size(); ++k) {
             const int rc = grp[k]->batch_begin();
@@ -1446,9 +1458,10 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
                 joined[k] = 1;
                 const Sea::QfTables* T = nullptr;
                 (void)grp[k]->sea->qform_meta(&T);
-                jobs3.push_back(grp[k]->batch_job());
-                cost3.push_back(T->cost);
-                if (grp[k]->batch_split()) {
+                const bool split = grp[k]->batch_split();
+                (split ? jobse : jobs3).push_back(grp[k]->batch_job());
+                (split ? coste : cost3).push_back(T->cost);
+                if (split) {
                     jobs1.push_back(grp[k]->batch_job2());
                     cost1.push_back(T->cost);
                 }
@@ -1464,12 +1477,12 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
             S.setup_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - h0).count();
         }
         // one persistent launch per product mode, its shape from the tuner
-        auto launch_list = [&](const std::vector<QfJob>& jobs, const std::vector<double>& cost, int nlv) -> int {
+        auto launch_list = [&](const std::vector<QfJob>& jobs, const std::vector<double>& cost, int kind) -> int {
             if (jobs.empty()) return 0;
             if (djobs.upload(jobs.data(), jobs.size() * sizeof(QfJob), st)) return -3;
             int64_t ntile = 0;
-            for (const QfJob& J : jobs) ntile += (J.ppad / 128) * J.nform;
-            const TuneKey key{nlv, ilog2((int64_t)jobs.size()), ilog2(ntile)};
+            for (const QfJob& J : jobs) ntile += (int64_t)batch_ptiles(J, kind) * batch_forms(J, kind);
+            const TuneKey key{kind, ilog2((int64_t)jobs.size()), ilog2(ntile)};
             BatchShape choice{-1, 0, 0, 0};
             {
                 std::lock_guard<std::mutex> lk(tune_mutex());
@@ -1481,11 +1494,11 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
                 if (std::sscanf(e, "%d,%d,%d,%d", &b.order, &b.blocks, &b.gf, &b.gp) >= 2) choice = b;
             }
             auto run = [&](const BatchShape& b, float* ms) -> int {
-                const std::vector<QfTile> tl = batch_tiles(jobs, cost, b);
+                const std::vector<QfTile> tl = batch_tiles(jobs, cost, b, kind);
                 if (dtiles.upload(tl.data(), tl.size() * sizeof(QfTile), st)) return -3;
                 CFDWM_HIP(hipEventRecord(e0, st));
                 CFDWM_HIP(launch_qf_persist((const QfJob*)djobs.get(), (const QfTile*)dtiles.get(), (int)tl.size(),
-                                            b.blocks, nlv, st));
+                                            b.blocks, kind, st));
                 CFDWM_HIP(hipEventRecord(e1, st));
                 CFDWM_HIP(hipEventSynchronize(e1));
                 CFDWM_HIP(hipEventElapsedTime(ms, e0, e1));
@@ -1516,8 +1529,9 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
             S.group_ptiles = choice.gp;
             return 0;
         };
-        if (int rc = launch_list(jobs3, cost3, 3)) { cleanup_all(); return rc; }
-        if (int rc = launch_list(jobs1, cost1, 1)) { cleanup_all(); return rc; }
+        if (int rc = launch_list(jobs3, cost3, kQfTileForm)) { cleanup_all(); return rc; }
+        if (int rc = launch_list(jobse, coste, kQfTileEta)) { cleanup_all(); return rc; }
+        if (int rc = launch_list(jobs1, cost1, kQfTilePair)) { cleanup_all(); return rc; }
         for (size_t k = 0; k < grp.size(); ++k) {
             const int rc = joined[k] ? grp[k]->batch_end() : grp[k]->refill();
             if (rc) { cleanup_all(); return rc; }

@@ -187,7 +187,8 @@ hipError_t launch_qf_build(const QfBuild& B, hipStream_t st);
 hipError_t launch_qd_zgen(const QdJob& J, hipStream_t st);
 hipError_t launch_qd_build(const QdBuild& B, hipStream_t st);
 hipError_t launch_qd_forms(const QdJob& J, hipStream_t st);
-hipError_t launch_qf_persist(const QfJob* jobs, const QfTile* tiles, int ntiles, int blocks, int nlv, hipStream_t st);
+// kind: kQfTileForm (three products), kQfTilePair (one product), kQfTileEta
+hipError_t launch_qf_persist(const QfJob* jobs, const QfTile* tiles, int ntiles, int blocks, int kind, hipStream_t st);
 // eta range of the columns of a fill (minus swl) -> eb[2]; then per filtered
 // pair record the levels where its profile exponentials exceed e^{-T}
 template <typename R>

@@ -86,8 +86,9 @@ struct GridGeom {
 // are bf16 hi/lo pairs in a tiled layout: rows in blocks of 32, k in blocks
 // of 16, a 32 x 16 tile stored as 512 contiguous values in two 32 x 8 halves
 // (k 0-7, then 8-15), each row's 8 values contiguous.
+constexpr int kQfTile = 256;              // points of a chunk are padded to whole point tiles
 struct QfJob {
-    int64_t p0 = 0, P = 0, ppad = 0;     // chunk of points [p0, p0 + P), padded to 128
+    int64_t p0 = 0, P = 0, ppad = 0;     // chunk of points [p0, p0 + P), padded to kQfTile
     int n = 0, npad = 0;                  // components, padded to 128
     int grid = 1;                         // points: slot-major s-grid columns, else arrays
     int64_t ncol = 0;
@@ -105,6 +106,7 @@ struct QfJob {
     int nlv = 3;                          // bf16 products per term: 3 (hi/lo split) or 1 (hi only, nbarr 2 or 4)
     const int8_t* ftype = nullptr;        // per form: 0 cos-type, 1 sin-type
     int nform = 0;
+    int ncos = 0;                         // of them cos-type, which come first
     const int32_t* kend = nullptr;        // per 64-wide tile of i: end of its m range (multiple of 16)
     float* out = nullptr;                 // [nform][ostride]
     int64_t ostride = 0;
@@ -113,10 +115,26 @@ struct QfJob {
     unsigned long long* clk = nullptr;
 };
 
-// One tile of a batched forms launch: job (sea state), point tile, form.
+// One tile of a batched forms launch: job (sea state), point tile, form (the
+// first of a pair, two != 0 when it has a second).
 struct QfTile {
-    int job, ptile, form, pad;
+    int job, ptile, form, two;
 };
+enum { kQfTileForm = 0, kQfTilePair = 1, kQfTileEta = 2 };
+
+// Form pairs of a launch at one product per term: the ncos cos-type forms,
+// then the sin-type ones, each type in pairs with an odd last form on its own.
+#if defined(__HIPCC__)
+#define CFDWM_HD __host__ __device__
+#else
+#define CFDWM_HD
+#endif
+CFDWM_HD inline int qf_pairs(int nform, int ncos) { return (ncos + 1) / 2 + (nform - ncos + 1) / 2; }
+CFDWM_HD inline void qf_pair(int nform, int ncos, int q, int* form, bool* two) {
+    const int pc = (ncos + 1) / 2;
+    *form = q < pc ? 2 * q : ncos + 2 * (q - pc);
+    *two = *form + 1 < (q < pc ? ncos : nform);
+}
 
 // Device build of the form tables from the FP32 pair records (qform.hip).
 struct QfBuild {

@@ -117,21 +117,18 @@ __global__ __launch_bounds__(256) void k_qf_zgen(QfJob J) {
 // ----------------------------------------------------------- quadratic forms
 // Form f of a launch:  Q_f(p) = sum_i e1_pi sum_m B1_f[i][m] c_pm + e2_pi sum_m B2_f[i][m] s_pm
 // with (e1, e2) = (c, s) for cos-type forms and (s, c) for sin-type forms.
-// One tile of work is (128 points, form): 4 waves, one per SIMD, walk the i
-// range in tiles of 128; wave (w & 1, w >> 1) takes 64 points x 64 i as
-// 2 x 2 MFMA 32 x 32 blocks for each of the two products, computed with
-// the table operand first, so that each lane's accumulator holds one point
-// and 16 values of i.  The k (= m)
-// range of an i tile runs from its first row (pairs have m > i) to the end
-// of its filtered rows.  Per k step (16 values of m) the block stages the A
-// operands of its 128 points and the B operands of its 128 i (4 arrays x 4
-// row blocks each, 32 KiB) in LDS, each operand tile read from L2 once per
-// block.  The epilogue of an i tile multiplies the accumulators by c or s
-// of the same (point, i), read as runs of four consecutive i (8 bytes), and
-// sums over i in the lane; one exchange between the two half-waves and one
-// between the two waves of a point range at the end write Q_f(p).  Single-job launches swizzle blocks in
-// groups of 8 forms x 32 point tiles so that the Z and B tables a group
-// reads stay in the last-level cache.
+// One tile of work is (64 NP points, form): 4 waves, one per SIMD, walk the i
+// range in tiles of 128 and, per i tile, the cosine and then the sine product;
+// wave (w & 1, w >> 1) takes 32 NP points x 64 i as NP x 2 MFMA 32 x 32 blocks,
+// computed with the table operand first, so that each lane's accumulator holds
+// one point and 16 values of i.  The k (= m) range of an i tile runs from its
+// first row (pairs have m > i) to the end of its filtered rows; the waves of
+// the tile's second 64 rows leave out its first 64 values of k (m <= i there).
+// The epilogue of a product multiplies the accumulators by c or s of the same
+// (point, i) and sums over i in the lane; one exchange between the two
+// half-waves and one between the two waves of a point range at the end write
+// Q_f(p).  Single-job launches swizzle blocks in groups of 8 forms x 32 point
+// tiles so that the Z and B tables a group reads stay in the last-level cache.
 constexpr int kQfGF = 8, kQfGP = 32;
 
 __device__ __forceinline__ bf16x8 lds8(const char* base, int off) {
@@ -149,45 +146,531 @@ __device__ __forceinline__ gu16p uni_ptr(const uint16_t* p) {
     return reinterpret_cast<gu16p>(((uint64_t)hi << 32) | lo);
 }
 
+// 16 bytes per lane from a wave-uniform base
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 uni_load4(const uint16_t* base, int off) {
+    return *reinterpret_cast<const u32x4 __attribute__((address_space(1)))*>(uni_ptr(base) + off);
+}
+
 // Operands move global -> LDS directly (global_load_lds_dwordx4, no
-// registers) through four LDS stages, three steps ahead of the products.
-// NLV is the number of bf16 products per term: 3 (hi*hi + lo*hi + hi*lo of
-// table and Z operands, about 16 significant bits) or 1 (hi*hi, about 8
-// significant bits; only the hi arrays are staged).  A stage holds NA = 4
-// (NLV 3) or 2 (NLV 1) operand arrays for the block's 128 points and 128 i,
-// 8 NA KiB.  Step j of an i tile:
-//   1. s_waitcnt vmcnt(2 NA) lgkmcnt(0) + s_barrier: the requests of step
-//      j + 1 (issued during step j - 2) have landed for all waves, and all
-//      waves' LDS reads of step j - 1 are done;
-//   2. the 8 NLV products of step j (operand set X) are issued interleaved
-//      with the 4 NA LDS reads of step j + 1's operands (set Y, stage
-//      (j + 1) % 4) and the 2 NA requests of step j + 3 (stage (j + 3) % 4 =
-//      (j - 1) % 4, last read during step j - 2, before step j - 1's
-//      barrier), so the matrix pipe stays busy while they issue.
-// The barrier is an asm statement with a memory clobber after an explicit
-// s_waitcnt: __syncthreads() would also wait for the requests of steps
-// j + 2 and j + 3.  Every wave runs every step of the block's k range: table
-// entries below the pair triangle (m <= i) and past a row tile's filtered end
-// are zero, so the extra products add exact zeros, and the step body has no
-// branch.
-template <int NLV>
+// registers) through three LDS stages.  NLV is the number of bf16 products per
+// term: 3 (hi*hi + lo*hi + hi*lo of table and Z operands, about 16 significant
+// bits) or 1 (hi*hi, about 8 significant bits; only the hi arrays are staged).
+// A stage holds two operand sets of the block's 64 NP points and 128 i: with
+// NLV 1 two consecutive k steps (16 values of m each), with NLV 3 the hi and
+// the lo arrays of one k step; 24 KiB at NP = 4, so that two blocks share a
+// CU's LDS and its registers (the accumulators take 128 of 256) and one block
+// computes while the other waits.  Stage j is worked off in phases of 2 NP
+// products whose operands were read from LDS one phase earlier:
+//   NLV 1   A: set 0, reading set 1     | sync | B: set 1, reading set 0 of stage j + 1
+//   NLV 3   A: hi x hi, reading lo      | sync | B: lo x hi | C: hi x lo, reading hi of stage j + 1
+// The sync (s_waitcnt, then s_barrier as asm with a memory clobber:
+// __syncthreads() would wait for every request) says that stage j + 1 has
+// landed for all waves and that all waves have read stage j, whose buffer the
+// requests of stage j + 3 then fill; they have two stages' time to land.
+// NP = 4 serves three products; NP = 2 three products in launches too small for
+// two blocks of the wide tile per CU, and one product in launches too small for
+// a form pair (below) per CU.
+//
+// What bounds three products: the matrix pipe at the clock that random bf16
+// operands leave it (near 1.9 GHz; hipBLASLt reaches 1.21 PFLOP/s on an 8192^3
+// product of this card).  43 forms, 30,300 points, 320 components: 0.94 ms,
+// 1.15 PFLOP/s executed, against 1.21 ms with one block of 128-point tiles per
+// CU, whose waits nothing covered.
+//
+// The table rows of a 32-row block are read from LDS in the order that puts
+// the 16 rows of a lane's accumulator (8 q + 4 h + e, q < 4, h the half-wave)
+// on the i values 16 (q / 2) + 8 h + 4 (q % 2) + e: the 8-value runs that the
+// same lane holds in the Z tiles, so the epilogue reads whole 1 KiB tiles.
+template <int NLV, int NP>
 __device__ __forceinline__ void qf_tile_il(const QfJob& J, int ptile, int form) {
     static_assert(NLV == 1 || NLV == 3, "one or three bf16 products per term");
-    constexpr int NB = 4;                         // stages
-    constexpr int NA = NLV == 1 ? 2 : 4;          // operand arrays per side in a stage
-    constexpr int SB = 8192 * NA;                 // stage bytes
-    constexpr int NF = 4 * NA;                    // operand fragments per set
-    constexpr int NG = 2 * NA;                    // request chunks per step = issue groups
-    constexpr int PG = 8 * NLV / NG;              // products per issue group (3 or 2)
+    constexpr int NB = 3;                         // stages
+    constexpr int G = NP / 2 + 1;                 // groups of four 1 KiB tiles per operand set: points, then table rows
+    constexpr int ND = 2 * G;                     // requests per wave and stage
+    constexpr int SB = ND * 4096;                 // stage bytes
+    constexpr int NF = NP + 2;                    // operand fragments of a set
     __shared__ __attribute__((aligned(16))) char lds[NB][SB];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wp = w & 1, wi = w >> 1;
+    const int wv = __builtin_amdgcn_readfirstlane(w);
+    const int wp = wv & 1, wi = wv >> 1;
     const int nkb = J.npad >> 4;
     const size_t nn = (size_t)J.npad * J.npad;
     // tables: 4 arrays per form (B1 hi, B1 lo, B2 hi, B2 lo) or 2 (B1 hi, B2 hi)
     const uint16_t* __restrict__ Bf = J.b + (size_t)form * J.nbarr * nn;
     const int bhs = J.nbarr == 4 ? 2 : 1;         // arrays between B1 hi and B2 hi
     const bool sint = J.ftype[form] != 0;
+    const int64_t PB = (int64_t)ptile * (64 * NP);
+    const int64_t rbB = PB >> 5;
+    const int64_t P0 = PB + wp * (32 * NP);
+    const int hl = lane >> 5, cl32 = lane & 31;
+    const int loff = (hl * 256 + cl32 * 8) * 2;
+    const int irow = (cl32 & 16) | ((cl32 & 4) << 1) | ((cl32 & 8) >> 1) | (cl32 & 3);
+    const int loffB = (hl * 256 + irow * 8) * 2;
+    float tp[NP];                                 // per lane: points P0 + 32 a + cl32
+#pragma unroll
+    for (int a = 0; a < NP; ++a) tp[a] = 0.f;
+    const int lo8 = lane * 8;
+    typedef __attribute__((address_space(3))) void* lds_vp;
+    typedef const __attribute__((address_space(1))) void* glb_vp;
+#define QF_WAIT(VM) __builtin_amdgcn_s_waitcnt(((VM) & 15) | (7 << 4) | (((VM) >> 4) << 14))
+#define QF_BARRIER() __asm__ volatile("s_barrier" ::: "memory")
+    const uint16_t* gp[ND];                       // request r of a stage at k step 0 (wave-uniform)
+    auto dma = [&](int r, int kb, int st) {
+        __builtin_amdgcn_global_load_lds((glb_vp)(uni_ptr(gp[r] + kb * 512) + lo8),
+                                         (lds_vp)(lds[0] + st * SB + (r * 4 + wv) * 1024), 16, 0, 0);
+    };
+    // fragment f of operand set u of a stage: f < NP the point block f, else table block f - NP
+    auto frag = [&](int st, int u, int f) {
+        const char* L = lds[0] + st * SB + u * (G * 4096);
+        return f < NP ? lds8(L, (wp * NP + f) * 1024 + loff)
+                      : lds8(L, ((G - 1) * 4 + wi * 2 + (f - NP)) * 1024 + loffB);
+    };
+    constexpr int KS = NLV == 1 ? 2 : 1;          // k steps per stage
+    for (int it = 0; it < J.npad; it += 128) {
+        const int t0 = it >> 6;
+        const int kb_lo = it >> 4;
+        const int kb_hi = __builtin_amdgcn_readfirstlane(max(J.kend[t0], J.kend[t0 + 1]) >> 4);
+        if (kb_hi <= kb_lo) continue;                 // block-uniform
+        const int ns = (kb_hi - kb_lo + KS - 1) / KS; // stages (a last odd k step reads zero table entries)
+        const int skip = wi ? 4 / KS : 0;             // stages this wave leaves out
+        const int ib0 = it >> 5;
+        // rows of this wave that have pairs at all
+        const bool rows = __builtin_amdgcn_readfirstlane(J.kend[t0 + wi]) > it + wi * 64;
+#pragma unroll 1
+        for (int cs = 0; cs < 2; ++cs) {
+            f32x16 acc[NP * 2];
+#pragma unroll
+            for (int q = 0; q < NP * 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+#pragma unroll
+            for (int r = 0; r < ND; ++r) {
+                const int u = r / G, g = r % G;
+                // NLV 1: set u is k step u of the hi arrays; NLV 3: u = 0 hi, 1 lo
+                const int arr = NLV == 1 ? 0 : u, k = NLV == 1 ? u : 0;
+                gp[r] = g < G - 1 ? J.zc_hi + (int64_t)(2 * cs + arr) * J.zn + ((rbB + 4 * g + wv) * nkb + k) * 512
+                                  : Bf + (size_t)(cs * bhs + arr) * nn + ((int64_t)(ib0 + wv) * nkb + k) * 512;
+            }
+            auto request = [&](int j, int st, int r0, int r1) {
+                if (j >= ns) return;                  // block-uniform
+#pragma unroll
+                for (int r = 0; r < ND; ++r)
+                    if (r >= r0 && r < r1) dma(r, kb_lo + j * KS, st);
+            };
+            bf16x8 X[NF], Y[NF];
+            auto mma = [&](const bf16x8& t, const bf16x8& z, int q) {
+                acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t, z, acc[q], 0, 0, 0);
+            };
+            // waits until at most the last VM requests are outstanding; near the
+            // end fewer were issued: wait for all
+            auto sync = [&](bool last) {
+                __builtin_amdgcn_sched_barrier(0);    // this phase's LDS reads are issued before the wait
+                if (last) QF_WAIT(0);
+                else QF_WAIT(ND);
+                QF_BARRIER();
+            };
+            int s0 = 0, s1 = 1, s2 = 2;               // buffers of stages j, j + 1, j + 2
+            request(0, 0, 0, ND);
+            request(1, 1, 0, ND);
+            request(2, 2, 0, NLV == 1 ? ND / 2 : ND);
+            if (ns > 2) QF_WAIT(NLV == 1 ? ND + ND / 2 : 2 * ND);
+            else QF_WAIT(0);
+            QF_BARRIER();
+            auto rotate = [&]() {
+                const int t = s0;
+                s0 = s1; s1 = s2; s2 = t;
+            };
+            int j = 0;
+            // the stages whose table entries are zero for this wave's rows: requests and syncs only
+            for (; j < min(skip, ns); ++j) {
+                if constexpr (NLV == 1) request(j + 2, s2, ND / 2, ND);
+                sync(j + 2 >= ns);
+                request(j + 3, s0, 0, NLV == 1 ? ND / 2 : ND);
+                rotate();
+            }
+            if (j < ns) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) X[f] = frag(s0, 0, f);
+            }
+            // products of set z (table fragments z[NP], z[NP + 1]) with the reads
+            // of fragments into y from operand set u of stage buffer st between them
+            auto phase = [&](const bf16x8 (&x)[NF], bf16x8 (&y)[NF], int st, int u) {
+#pragma unroll
+                for (int q = 0; q < 2 * NP; ++q) {
+                    mma(x[NP + (q & 1)], x[q >> 1], q);
+                    if (q < NF) y[q] = frag(st, u, q);
+                    if (q & 1) __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int f = 2 * NP; f < NF; ++f) y[f] = frag(st, u, f);
+            };
+#pragma unroll 1
+            for (; j < ns; ++j) {
+                if constexpr (NLV == 1) {
+                    phase(X, Y, s0, 1);
+                    request(j + 2, s2, ND / 2, ND);
+                    sync(j + 2 >= ns);
+                    request(j + 3, s0, 0, ND / 2);
+                    phase(Y, X, s1, 0);
+                } else {
+                    phase(X, Y, s0, 1);
+                    sync(j + 2 >= ns);
+                    request(j + 3, s0, 0, ND);
+#pragma unroll
+                    for (int q = 0; q < 2 * NP; ++q) mma(Y[NP + (q & 1)], X[q >> 1], q);
+                    __builtin_amdgcn_sched_barrier(0);
+                    Y[NP] = X[NP];
+                    Y[NP + 1] = X[NP + 1];
+                    phase(Y, X, s1, 0);
+                }
+                rotate();
+            }
+            // every wave is past its reads before the next product's requests
+            QF_WAIT(0);
+            QF_BARRIER();
+            if (rows) {                               // wave-uniform
+                // element r of block (a, b): point P0 + 32 a + cl32,
+                // i = it + 64 wi + 32 b + 16 (r / 8) + 8 hl + r % 8
+                const uint16_t* zrow = J.zc_hi + ((cs != 0) != sint ? 2 * J.zn : 0) +
+                                       ((P0 >> 5) * nkb + (it >> 4) + wi * 4) * 512;
+#pragma unroll
+                for (int a = 0; a < NP; ++a) {
+                    float s = 0.f, sl = 0.f;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            const uint16_t* z = zrow + ((int64_t)a * nkb + 2 * b + t) * 512;
+                            const u32x4 hv = uni_load4(z, lo8), lv = uni_load4(z + J.zn, lo8);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                const uint32_t hw = hv[e >> 1], lw = lv[e >> 1];
+                                const float vh = __uint_as_float((e & 1) ? hw & 0xFFFF0000u : hw << 16);
+                                const float vl = __uint_as_float((e & 1) ? lw & 0xFFFF0000u : lw << 16);
+                                if (NLV == 1) {       // the order of qf_pair_tile
+                                    s += acc[a * 2 + b][8 * t + e] * vh;
+                                    sl += acc[a * 2 + b][8 * t + e] * vl;
+                                } else {
+                                    s += acc[a * 2 + b][8 * t + e] * (vh + vl);
+                                }
+                            }
+                        }
+                    tp[a] += s;
+                    if (NLV == 1) tp[a] += sl;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    }
+#undef QF_WAIT
+#undef QF_BARRIER
+    // lane l ends with points P0 + 64 c + l: its own half's i sums plus the other half's
+    float* red = reinterpret_cast<float*>(lds[0]);
+    float tot[NP / 2];
+#pragma unroll
+    for (int c = 0; c < NP / 2; ++c) {
+        const float t0 = tp[2 * c] + __shfl_xor(tp[2 * c], 32);
+        const float t1 = tp[2 * c + 1] + __shfl_xor(tp[2 * c + 1], 32);
+        tot[c] = hl ? t1 : t0;
+    }
+    __syncthreads();
+    if (wi)
+#pragma unroll
+        for (int c = 0; c < NP / 2; ++c) red[wp * 32 * NP + 64 * c + lane] = tot[c];
+    __syncthreads();
+    if (!wi)
+#pragma unroll
+        for (int c = 0; c < NP / 2; ++c) {
+            const int64_t p = P0 + 64 * c + lane;
+            if (p < J.P) J.out[(int64_t)form * J.ostride + J.p0 + p] = tot[c] + red[wp * 32 * NP + 64 * c + lane];
+        }
+}
+
+// Velocity forms of the bf16 mode (one product per term): one block of 8 waves
+// per CU evaluates two forms of one type for 256 points, 128 i at a time.
+//
+// What bounds these launches is the operands' way: with one form per block the
+// requests for tables and Z operands took 14.8 ms of a 16.7 ms launch (262,144
+// points, 1024 components, 26 forms) when only an eighth of the matrix
+// products were left in it, and the epilogue's c and s another 3.5 ms; past L2
+// they moved 92 GB.  Two forms share the staged Z operands and the epilogue's
+// c and s, and two blocks' worth of rows share each table row: 512 rows per
+// 2^16 products where 768 passed before, and half the epilogue's loads.
+// The wave tile is 64 points x 64 i x 2 forms (128 accumulator registers).
+//
+// The block's work is one stream of stages (32 values of k: two operand sets),
+// pass after pass ((i tile, cosine or sine product)), four LDS stages of 32
+// KiB, requests three and a half stages ahead and running on across pass ends,
+// so that the next pass's operands land during the epilogue.  Stage j:
+//   A: products of set 0, reading set 1 | sync | B: products of set 1, reading set 0 of the stage after
+// and the sync says that the stage after j has landed for all waves and that
+// all waves have read stage j, whose buffer then takes the fourth stage after.
+// The c or s of the epilogue are read as 16-byte runs of 8 i per lane (see
+// qf_tile_il): the hi parts a stage ahead, the lo parts while the hi parts'
+// products run.
+//
+// Measured on the launch above: 17.5 ms with one form, 128 points and both
+// products per block (two blocks per CU), 16.7 with 256 points, 14.8 now, 1.03
+// PFLOP/s executed.  Of these, the matrix products and barriers alone take
+// 10.2, the LDS reads 1.0, the epilogue 1.4, the requests 2.3 (0.8 of them
+// because the operands come from past L2).
+constexpr int kPairStage = 32768;
+__device__ __forceinline__ void qf_pair_tile(const QfJob& J, int ptile, int form, bool two) {
+    constexpr int NB = 4;
+    __shared__ __attribute__((aligned(16))) char lds[NB][kPairStage];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wp = wv & 3, wi = wv >> 2;
+    const int nkb = J.npad >> 4;
+    const size_t nn = (size_t)J.npad * J.npad;
+    const int bhs = J.nbarr == 4 ? 2 : 1;
+    const uint16_t* __restrict__ Bf = J.b + (size_t)form * J.nbarr * nn;
+    // the block's second form; without one the first again, its values unused
+    const size_t f2 = two ? (size_t)J.nbarr * nn : 0;
+    const bool sint = J.ftype[form] != 0;
+    const int64_t P0 = (int64_t)ptile * 256 + wp * 64;
+    const int hl = lane >> 5, cl32 = lane & 31;
+    const int loff = lane * 16;
+    const int irow = (cl32 & 16) | ((cl32 & 4) << 1) | ((cl32 & 8) >> 1) | (cl32 & 3);
+    const int loffB = (hl * 256 + irow * 8) * 2;
+    const int lo8 = lane * 8;
+    typedef __attribute__((address_space(3))) void* lds_vp;
+    typedef const __attribute__((address_space(1))) void* glb_vp;
+#define QF_WAIT(VM) __builtin_amdgcn_s_waitcnt(((VM) & 15) | (7 << 4) | (((VM) >> 4) << 14))
+    // k steps of the i tile it, in stages (a last odd k step reads zero table entries)
+    auto stages = [&](int it) {
+        const int t0 = it >> 6;
+        const int kb_hi = __builtin_amdgcn_readfirstlane(max(J.kend[t0], J.kend[t0 + 1]) >> 4);
+        return max(0, (kb_hi - (it >> 4) + 1) >> 1);
+    };
+    int left = 0;                                     // stages of the stream not yet worked off
+    for (int it = 0; it < J.npad; it += 128) left += 2 * stages(it);
+    if (left > 0) {
+        // request cursor: pass (rit, rcs), stage rj of rns; bases of this wave's tiles at the pass's first k step
+        int rit = -128, rcs = 1, rj = 0, rns = 0;
+        const uint16_t *ga = nullptr, *gb = nullptr;
+        auto next_pass = [&](int& it, int& cs, int& ns) {
+            if (cs == 0) { cs = 1; return; }
+            cs = 0;
+            do { it += 128; ns = stages(it); } while (ns == 0);
+        };
+        auto dma = [&](const uint16_t* g, int r, int st) {
+            __builtin_amdgcn_global_load_lds((glb_vp)(uni_ptr(g) + lo8),
+                                             (lds_vp)(lds[0] + st * kPairStage + (r * 8 + wv) * 1024), 16, 0, 0);
+        };
+        int toreq = left;                             // stages not yet requested
+        // first half of a request: the point operands of both sets; second half: the table rows
+        auto req_a = [&](int st) {
+            if (toreq <= 0) return;
+            if (rj == rns) {
+                next_pass(rit, rcs, rns);
+                rj = 0;
+                ga = J.zc_hi + (int64_t)(2 * rcs) * J.zn + (((int64_t)ptile * 8 + wv) * nkb + (rit >> 4)) * 512;
+                gb = Bf + (wv >> 2) * f2 + (size_t)(rcs * bhs) * nn +
+                     ((int64_t)((rit >> 5) + (wv & 3)) * nkb + (rit >> 4)) * 512;
+            }
+            dma(ga + rj * 1024, 0, st);
+            dma(ga + rj * 1024 + 512, 1, st);
+        };
+        auto req_b = [&](int st) {
+            if (toreq <= 0) return;
+            dma(gb + rj * 1024, 2, st);
+            dma(gb + rj * 1024 + 512, 3, st);
+            ++rj;
+            --toreq;
+        };
+        // fragments of set u: 0, 1 the points, 2 .. 5 the table rows of (form, i block)
+        auto frag = [&](int st, int u, int f) {
+            const char* L = lds[0] + st * kPairStage + u * 8192;
+            return f < 2 ? lds8(L, (wp * 2 + f) * 1024 + loff)
+                         : lds8(L + 16384, (((f - 2) >> 1) * 4 + wi * 2 + ((f - 2) & 1)) * 1024 + loffB);
+        };
+        bf16x8 X[6], Y[6];
+        f32x16 acc[8];                                // [(form * 2 + i block) * 2 + point block]
+        auto clear = [&]() {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+        };
+        auto phase = [&](const bf16x8 (&x)[6], bf16x8 (&y)[6], int st, int u) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[2 + (q >> 1)], x[q & 1], acc[q], 0, 0, 0);
+                if (q < 6) y[q] = frag(st, u, q);
+                if (q & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        float tp[2][2] = {{0.f, 0.f}, {0.f, 0.f}};    // [form][point block]
+        req_a(0); req_b(0); req_a(1); req_b(1); req_a(2); req_b(2); req_a(3);
+        QF_WAIT(0);
+        __asm__ volatile("s_barrier" ::: "memory");
+        int it = -128, cs = 1, ns = 0, buf = 0;
+        while (left > 0) {                            // one pass; block-uniform
+            next_pass(it, cs, ns);
+            // the waves of the tile's second 64 rows leave out its first 64 k: m <= i there
+            const int skip = min(wi ? 2 : 0, ns);
+            const uint16_t* zrow = J.zc_hi + ((cs != 0) != sint ? 2 * J.zn : 0) +
+                                   ((P0 >> 5) * nkb + (it >> 4) + wi * 4) * 512;
+            u32x4 eh[8];
+            auto load_hi = [&]() {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) eh[q] = uni_load4(zrow + ((int64_t)(q >> 2) * nkb + (q & 3)) * 512, lo8);
+            };
+            // the next stage has landed once only the newest two stages' requests
+            // (and, in a pass's last stage, the epilogue's 8 loads) are outstanding;
+            // fewer were issued near the stream's end
+            auto sync = [&](bool end) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (left < 4) QF_WAIT(0);
+                else if (end) QF_WAIT(16);
+                else QF_WAIT(8);
+                __asm__ volatile("s_barrier" ::: "memory");
+            };
+            clear();
+            int j = 0;
+            for (; j < skip; ++j) {
+                const bool end = j == ns - 1;
+                if (end) load_hi();
+                req_b((buf + 3) & 3);
+                sync(end);
+                req_a(buf);
+                --left;
+                buf = (buf + 1) & 3;
+            }
+#pragma unroll
+            for (int f = 0; f < 6; ++f) X[f] = frag(buf, 0, f);
+#pragma unroll 1
+            for (; j < ns; ++j) {
+                const bool end = j == ns - 1;
+                if (end) load_hi();
+                phase(X, Y, buf, 1);
+                req_b((buf + 3) & 3);
+                sync(end);
+                req_a(buf);
+                const int nb = (buf + 1) & 3;
+                phase(Y, X, nb, 0);
+                --left;
+                buf = nb;
+            }
+            // element r of block (f, b, a): point P0 + 32 a + cl32, i = it + 64 wi + 32 b + 16 (r / 8) + 8 hl + r % 8
+            u32x4 el[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                el[q] = uni_load4(zrow + J.zn + ((int64_t)(q >> 2) * nkb + (q & 3)) * 512, lo8);
+            auto weigh = [&](const u32x4 (&e)[8]) {
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const uint32_t hw = e[4 * a + t][k >> 1];
+                            const float v = __uint_as_float((k & 1) ? hw & 0xFFFF0000u : hw << 16);
+                            s0 += acc[(t >> 1) * 2 + a][8 * (t & 1) + k] * v;
+                            s1 += acc[4 + (t >> 1) * 2 + a][8 * (t & 1) + k] * v;
+                        }
+                    tp[0][a] += s0;
+                    tp[1][a] += s1;
+                }
+            };
+            weigh(eh);
+            weigh(el);
+        }
+#undef QF_WAIT
+        // lane l: point P0 + l, its own half's i sums plus the other half's; then the two i halves
+        float* red = reinterpret_cast<float*>(lds[0]);
+        float tot[2];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            const float t0 = tp[f][0] + __shfl_xor(tp[f][0], 32);
+            const float t1 = tp[f][1] + __shfl_xor(tp[f][1], 32);
+            tot[f] = hl ? t1 : t0;
+        }
+        __syncthreads();
+        if (wi) {
+            red[wp * 64 + lane] = tot[0];
+            red[256 + wp * 64 + lane] = tot[1];
+        }
+        __syncthreads();
+        if (!wi) {
+            const int64_t p = P0 + lane;
+            if (p < J.P) {
+                float* o = J.out + (int64_t)form * J.ostride + J.p0 + p;
+                o[0] = tot[0] + red[wp * 64 + lane];
+                if (two) o[J.ostride] = tot[1] + red[256 + wp * 64 + lane];
+            }
+        }
+    } else if (!wi) {
+        const int64_t p = P0 + lane;
+        if (p < J.P) {
+            float* o = J.out + (int64_t)form * J.ostride + J.p0 + p;
+            o[0] = 0.f;
+            if (two) o[J.ostride] = 0.f;
+        }
+    }
+}
+
+// Blocks of an XCD (round-robin dispatch) walk the form pairs of two point
+// tiles together: the two tiles' Z operands stay in its L2 (1 MiB of hi parts
+// each at 1024 components), the tables stream through the last-level cache and
+// serve both tiles.  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
+// 32 point tiles, 89 GB one point tile at a time, 73 GB two at a time.
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_qf_pairs(QfJob J, int npt) {
+    const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3;
+    const int in = sq % (2 * np);
+    const int ptile = (sq / (2 * np) * 2 + (in & 1)) * 8 + (blockIdx.x & 7);
+    if (ptile >= npt) return;                         // whole block, before any barrier
+    int form;
+    bool two;
+    qf_pair(J.nform, J.ncos, in >> 1, &form, &two);
+    if (!J.clk) {
+        qf_pair_tile(J, ptile, form, two);
+        return;
+    }
+    const unsigned long long c0 = clock64(), w0 = wall_clock64();
+    qf_pair_tile(J, ptile, form, two);
+    if (threadIdx.x == 0) {
+        atomicAdd(J.clk, clock64() - c0);
+        atomicAdd(J.clk + 1, wall_clock64() - w0);
+    }
+}
+
+// The eta2 form: one form, three products per term.  A block of 4 waves, one
+// per SIMD, takes 128 points and 128 i at a time with the cosine and the sine
+// products together (64 x 64 per wave, 128 accumulator and 203 other
+// registers), four 32 KiB stages of one k step, requests three steps ahead.
+// Step j of an i tile:
+//   1. s_waitcnt vmcnt(8) lgkmcnt(0) + s_barrier: the requests of step j + 1
+//      (issued during step j - 2) have landed for all waves, and all waves'
+//      LDS reads of step j - 1 are done;
+//   2. the 24 products of step j (operand set X) are issued interleaved with
+//      the 16 LDS reads of step j + 1's operands (set Y, stage (j + 1) % 4)
+//      and the 8 requests of step j + 3 (stage (j + 3) % 4 = (j - 1) % 4, last
+//      read during step j - 2, before step j - 1's barrier).
+// The sums run in one fixed order, the cosine and sine terms of an i together:
+// whoever rounds functions of eta2 to bf16, as the surrogate's network does
+// with its inputs, sees any other order.  Measured: 2.0 ms for 262,144 points
+// and 1024 components (1.77e12 FLOP executed); qf_tile_il takes the same, and
+// 8 waves on 128 points x 256 i, which read the points' operands 3.5 instead
+// of 5.5 times, 2.1 ms.
+__device__ __forceinline__ void qf_eta_tile(const QfJob& J, int ptile) {
+    constexpr int NB = 4;                         // stages
+    constexpr int NA = 4;                         // operand arrays per side in a stage
+    constexpr int SB = 8192 * NA;                 // stage bytes
+    constexpr int NF = 4 * NA;                    // operand fragments per set
+    constexpr int NG = 2 * NA;                    // request chunks per step = issue groups
+    constexpr int PG = 24 / NG;                   // products per issue group
+    __shared__ __attribute__((aligned(16))) char lds[NB][SB];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int wp = w & 1, wi = w >> 1;
+    const int nkb = J.npad >> 4;
+    const size_t nn = (size_t)J.npad * J.npad;
+    const uint16_t* __restrict__ Bf = J.b;       // B1 hi, B1 lo, B2 hi, B2 lo
+    const bool sint = J.ftype[0] != 0;
     const int64_t PB = (int64_t)ptile * 128;
     const int64_t rbB = PB >> 5;
     const int64_t P0 = PB + wp * 64;
@@ -230,13 +713,13 @@ __device__ __forceinline__ void qf_tile_il(const QfJob& J, int ptile, int form) 
         for (int q = 0; q < 8; ++q)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
-        // product s (< 8 NLV) of a step: level s / 8 (hi x hi, lo x hi, hi x
+        // product s (< 24) of a step: level s / 8 (hi x hi, lo x hi, hi x
         // lo of table x Z), accumulator s % 8; an accumulator's products are
         // 8 issues apart
         auto mma = [&](const bf16x8 (&op)[NF], int s) {
             const int lv = s >> 3, q = s & 7, cs = q & 1, a2 = q >> 2, b = (q >> 1) & 1;
-            const int fa = NLV == 1 ? a2 * NA + cs : a2 * 4 + 2 * cs + (lv == 2 ? 1 : 0);
-            const int fb = NLV == 1 ? 2 * NA + b * NA + cs : 8 + b * 4 + 2 * cs + (lv == 1 ? 1 : 0);
+            const int fa = a2 * 4 + 2 * cs + (lv == 2 ? 1 : 0);
+            const int fb = 8 + b * 4 + 2 * cs + (lv == 1 ? 1 : 0);
             acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[fb], op[fa], acc[q], 0, 0, 0);
         };
         // one step: products of operand set x, reads of step j + 1 into set y
@@ -254,15 +737,12 @@ __device__ __forceinline__ void qf_tile_il(const QfJob& J, int ptile, int form) 
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        // global array of chunk r: A arrays c_hi, c_lo, s_hi, s_lo (NLV 3) or
-        // c_hi, s_hi (NLV 1); B arrays likewise
+        // global array of chunk r: A arrays c_hi, c_lo, s_hi, s_lo; B arrays likewise
 #pragma unroll
         for (int r = 0; r < NG; ++r) {
             const int a = r % NA;
-            const int ga = NLV == 1 ? 2 * a : a;                       // Z array index
-            const int gb = NLV == 1 ? a * bhs : a;                     // table array index
-            gp[r] = r < NA ? J.zc_hi + (int64_t)ga * J.zn + (rbB + wv) * nkb * 512
-                           : Bf + (size_t)gb * nn + (int64_t)(ib0 + wv) * nkb * 512;
+            gp[r] = r < NA ? J.zc_hi + (int64_t)a * J.zn + (rbB + wv) * nkb * 512
+                           : Bf + (size_t)a * nn + (int64_t)(ib0 + wv) * nkb * 512;
         }
         // requests past the last step re-read step kb_hi - 1 (in bounds, unused)
         const int kl = kb_hi - 1;
@@ -329,16 +809,27 @@ __device__ __forceinline__ void qf_tile_il(const QfJob& J, int ptile, int form) 
     __syncthreads();
     if (!wi) {
         const int64_t p = P0 + lane;
-        if (p < J.P) J.out[(int64_t)form * J.ostride + J.p0 + p] = tot + red[wp * 64 + lane];
+        if (p < J.P) J.out[J.p0 + p] = tot + red[wp * 64 + lane];
+    }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void k_qf_eta(QfJob J) {
+    if (!J.clk) {
+        qf_eta_tile(J, blockIdx.x);
+        return;
+    }
+    const unsigned long long c0 = clock64(), w0 = wall_clock64();
+    qf_eta_tile(J, blockIdx.x);
+    if (threadIdx.x == 0) {
+        atomicAdd(J.clk, clock64() - c0);
+        atomicAdd(J.clk + 1, wall_clock64() - w0);
     }
 }
 
 // Single-job launch: block -> (point tile, form) through the swizzle.
-// One product per term stages 64 KiB of LDS per block: with the accumulators
-// in VGPRs (no AGPRs) two blocks share a CU, one computing while the other
-// waits at its barrier.  Three products stage 128 KiB: one block per CU.
-template <int NLV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NLV == 1 ? 2 : 1, 2)))
+template <int NLV, int NP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_qf_forms_il(QfJob J, int npt) {
     const int id = blockIdx.x;
     const int per = kQfGF * kQfGP;
@@ -349,29 +840,32 @@ void k_qf_forms_il(QfJob J, int npt) {
     const int form = fg * kQfGF + in / kQfGP;
     if (ptile >= npt || form >= J.nform) return;      // whole block, before any barrier
     if (!J.clk) {
-        qf_tile_il<NLV>(J, ptile, form);
+        qf_tile_il<NLV, NP>(J, ptile, form);
         return;
     }
     const unsigned long long c0 = clock64(), w0 = wall_clock64();
-    qf_tile_il<NLV>(J, ptile, form);
+    qf_tile_il<NLV, NP>(J, ptile, form);
     if (threadIdx.x == 0) {
         atomicAdd(J.clk, clock64() - c0);
         atomicAdd(J.clk + 1, wall_clock64() - w0);
     }
 }
 
-// Persistent launch over the tiles of many jobs (sea states): block b takes
+// Persistent launches over the tiles of many jobs (sea states): block b takes
 // tiles b, b + gridDim.x, ... of the ordered tile list; every block exits
-// after its last tile.
-template <int NLV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NLV == 1 ? 2 : 1, 2)))
-void k_qf_forms_persist(const QfJob* __restrict__ jobs,
-                                                          const QfTile* __restrict__ tiles, int ntiles) {
+// after its last tile.  KIND 0: (256 points, form) tiles at three products,
+// two blocks per CU; 1: (256 points, form pair) tiles at one product, one block
+// of 8 waves per CU; 2: (128 points) tiles of the eta2 forms, one block per CU.
+template <int KIND>
+__global__ __launch_bounds__(KIND == 1 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(KIND == 2 ? 1 : 2, 2)))
+void k_qf_forms_persist(const QfJob* __restrict__ jobs, const QfTile* __restrict__ tiles, int ntiles) {
     for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const QfTile tl = tiles[t];
         const QfJob J = jobs[tl.job];
         __syncthreads();                              // the previous tile's LDS readers are done
-        qf_tile_il<NLV>(J, tl.ptile, tl.form);
+        if constexpr (KIND == 0) qf_tile_il<3, 4>(J, tl.ptile, tl.form);
+        else if constexpr (KIND == 1) qf_pair_tile(J, tl.ptile, tl.form, tl.two != 0);
+        else qf_eta_tile(J, tl.ptile);
     }
 }
 
@@ -450,7 +944,8 @@ hipError_t launch_qf_build(const QfBuild& B, hipStream_t st) {
 
 static bool qf_shape_ok(const QfJob& J) {
     if ((J.nlv != 1 && J.nlv != 3) || (J.nbarr != 2 && J.nbarr != 4) || (J.nlv == 3 && J.nbarr != 4)) return false;
-    return !((J.ppad & 127) || (J.npad & 127) || J.ppad < J.P || J.npad < J.n);
+    if (J.ncos < 0 || J.ncos > J.nform) return false;
+    return !((J.ppad & (kQfTile - 1)) || (J.npad & 127) || J.ppad < J.P || J.npad < J.n);
 }
 
 hipError_t launch_qf_zgen(const QfJob& J, hipStream_t st) {
@@ -464,26 +959,43 @@ hipError_t launch_qf_zgen(const QfJob& J, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_qf_persist(const QfJob* jobs, const QfTile* tiles, int ntiles, int blocks, int nlv, hipStream_t st) {
+hipError_t launch_qf_persist(const QfJob* jobs, const QfTile* tiles, int ntiles, int blocks, int kind, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    if (blocks <= 0 || (nlv != 1 && nlv != 3)) return hipErrorInvalidValue;
-    if (nlv == 1)
-        hipLaunchKernelGGL(k_qf_forms_persist<1>, dim3((unsigned)blocks), dim3(256), 0, st, jobs, tiles, ntiles);
-    else
-        hipLaunchKernelGGL(k_qf_forms_persist<3>, dim3((unsigned)blocks), dim3(256), 0, st, jobs, tiles, ntiles);
+    if (blocks <= 0) return hipErrorInvalidValue;
+    const dim3 g((unsigned)blocks);
+    if (kind == kQfTileForm) hipLaunchKernelGGL(k_qf_forms_persist<0>, g, dim3(256), 0, st, jobs, tiles, ntiles);
+    else if (kind == kQfTilePair) hipLaunchKernelGGL(k_qf_forms_persist<1>, g, dim3(512), 0, st, jobs, tiles, ntiles);
+    else if (kind == kQfTileEta) hipLaunchKernelGGL(k_qf_forms_persist<2>, g, dim3(256), 0, st, jobs, tiles, ntiles);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
 hipError_t launch_qf_forms(const QfJob& J, hipStream_t st) {
     if (J.P <= 0 || J.nform <= 0) return hipSuccess;
     if (!qf_shape_ok(J)) return hipErrorInvalidValue;
-    const int npt = (int)(J.ppad / 128);
+    // eta2 alone
+    if (J.nlv == 3 && J.nform == 1) {
+        hipLaunchKernelGGL(k_qf_eta, dim3((unsigned)((J.P + 127) / 128)), dim3(256), 0, st, J);
+        return hipGetLastError();
+    }
+    // one product per term: form pairs where they give every CU a block
+    if (J.nlv == 1 && J.ppad / 256 * qf_pairs(J.nform, J.ncos) >= 256) {
+        const int np = (int)(J.ppad / 256);
+        hipLaunchKernelGGL(k_qf_pairs, dim3((unsigned)((np + 15) / 16 * 16 * qf_pairs(J.nform, J.ncos))), dim3(512), 0, st,
+                           J, np);
+        return hipGetLastError();
+    }
+    // 256-point tiles where they give every CU its two blocks, else 128
+    const bool wide = J.nlv == 3 && J.ppad / 256 * J.nform >= 512;
+    const int npt = (int)(wide ? J.ppad / 256 : (J.P + 127) / 128);
     const int nfg = (J.nform + kQfGF - 1) / kQfGF, npg = (npt + kQfGP - 1) / kQfGP;
     const unsigned nblk = (unsigned)((int64_t)nfg * npg * kQfGF * kQfGP);
     if (J.nlv == 1)
-        hipLaunchKernelGGL(k_qf_forms_il<1>, dim3(nblk), dim3(256), 0, st, J, npt);
+        hipLaunchKernelGGL((k_qf_forms_il<1, 2>), dim3(nblk), dim3(256), 0, st, J, npt);
+    else if (wide)
+        hipLaunchKernelGGL((k_qf_forms_il<3, 4>), dim3(nblk), dim3(256), 0, st, J, npt);
     else
-        hipLaunchKernelGGL(k_qf_forms_il<3>, dim3(nblk), dim3(256), 0, st, J, npt);
+        hipLaunchKernelGGL((k_qf_forms_il<3, 2>), dim3(nblk), dim3(256), 0, st, J, npt);
     return hipGetLastError();
 }
 

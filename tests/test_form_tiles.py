@@ -1,0 +1,48 @@
+"""The forms kernels at the edges of their tiles: a grid large enough for the
+form-pair launch against the same columns in a grid that takes the small tile,
+for component counts around the 128-row tiles, rows that end early and an odd
+number of forms of a type.  Both run the same bf16 operands, so they differ by
+the order of FP32 sums only: 1e-5 of the field scale, the library's FP32 bound."""
+import numpy as np
+import pytest
+
+from cfdwavemaker_amd.seastate import make_sea
+from tests.conftest import scaled_err
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from cfdwavemaker_amd import engine
+    engine.load()
+    return engine
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nfreq,ndir,depth,kw", [
+    (5, 2, 30.0, {}),                            # far below one tile
+    (64, 1, 20.0, {}),                           # half a tile: the second 64 rows have no pairs
+    (65, 1, 60.0, {}),                           # one row into the second half
+    (32, 4, 100.0, {}),                          # one whole tile
+    (43, 3, 45.0, {}),                           # 129: one row into a second tile
+    (60, 4, 150.0, dict(bandwidth=0.6)),         # 240, rows that end inside a tile
+    (100, 4, 10.0, dict(cutoff=2.0)),            # 400, rows past the cutoff empty
+])
+@pytest.mark.parametrize("mode", ["bf16", "fp32"])
+def test_large_launch_equals_small(eng, mode, nfreq, ndir, depth, kw):
+    s = make_sea(nfreq, 2.0, 8.0, depth, seed=nfreq, ndir=ndir).as_dict()
+    s.update(kw)
+    prec = eng.BF16 if mode == "bf16" else eng.FP32
+    dx = 6.0
+    n, m = 96, 5                                 # 36,864 and 100 column-slots
+    big = eng.Sea(s, precision=prec, with_direct=False).grid((0.0, (n - 1) * dx, 0.0, (n - 1) * dx), n, n, 4, 0.0,
+                                                             0.5, 0.7, 1.5, depth)
+    small = eng.Sea(s, precision=prec, with_direct=False).grid((0.0, (m - 1) * dx, 0.0, (m - 1) * dx), m, m, 4, 0.0,
+                                                               0.5, 0.7, 1.5, depth)
+    assert big.qform_info() and small.qform_info()
+    for f, tail in (("ETA", ()), ("UX", (4,)), ("UY", (4,)), ("UZ", (4,))):
+        a = big.export(f).reshape((4, n, n) + tail)[:, :m, :m].ravel()
+        b = small.export(f)
+        if not np.any(b):
+            assert not np.any(a)
+            continue
+        assert scaled_err(a, b) <= 1e-5, (f, scaled_err(a, b))
