@@ -1267,9 +1267,8 @@ size_t Grid::refill_z_bytes() const {
 void Grid::release_workspace() {
     zbuf_.release();
     qd_space_.reset();
-    qs_key_.release();
+    qs_cnt_.release();
     qs_rec_.release();
-    qs_tmp_.release();
 }
 
 namespace {
@@ -1780,23 +1779,16 @@ int Grid::write_vtk_dump(bool last) {
 // Query batches from this size on are evaluated in cell order.
 constexpr int64_t kQuerySortMin = 65536;
 
-// Device bytes of the cell-ordering buffers of an n-query batch (keys and
-// records, input and sorted halves, and the radix sort's scratch, each part
-// 256-byte aligned); 0 below the ordering threshold.
+// The cell-ordering buffers of an n-query batch (tile counts, then records,
+// each part 256-byte aligned); 0 below the ordering threshold.
 template <typename TQ>
-int query_ws_bytes(int64_t n, int ncol, size_t* bytes) {
-    *bytes = 0;
+size_t query_ws_bytes(int64_t n, int nx, int ny) {
     if (n < kQuerySortMin || n > INT32_MAX) return 0;
-    int bits = 1;
-    while (((int64_t)1 << bits) < ncol) ++bits;
-    size_t tmp = 0;
-    CFDWM_HIP(query_sort_tmp_bytes<TQ>(n, bits, &tmp));
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    *bytes = up(2 * n * sizeof(uint32_t)) + up(2 * n * sizeof(QRec<TQ>)) + up(std::max<size_t>(tmp, 256));
-    return 0;
+    return up(query_bins_bytes(n, nx, ny)) + up(n * sizeof(QRec<TQ>));
 }
-template int query_ws_bytes<float>(int64_t, int, size_t*);
-template int query_ws_bytes<double>(int64_t, int, size_t*);
+template size_t query_ws_bytes<float>(int64_t, int, int);
+template size_t query_ws_bytes<double>(int64_t, int, int);
 
 template <typename R, typename TQ>
 int Grid::run_query(int64_t n, const TQ* t, double tconst, const TQ* x, const TQ* y, const TQ* z,
@@ -1813,39 +1805,22 @@ int Grid::run_query(int64_t n, const TQ* t, double tconst, const TQ* x, const TQ
     J.o_eta = eta; J.o_u = u; J.o_v = v; J.o_w = w;
     J.o_aos = aos;
     hipStream_t st = Engine::get().stream();
-    const int64_t ncol = (int64_t)g.nx * g.ny;
     if (n >= kQuerySortMin && n <= INT32_MAX) {
         // large batches run in cell order (qsort.hip)
-        int bits = 1;
-        while (((int64_t)1 << bits) < ncol) ++bits;
-        size_t tmp = 0;
-        CFDWM_HIP(query_sort_tmp_bytes<TQ>(n, bits, &tmp));
-        uint32_t* keys = nullptr;
+        const size_t cb = (query_bins_bytes(n, g.nx, g.ny) + 255) / 256 * 256;
+        uint32_t* cnt = nullptr;
         QRec<TQ>* rec = nullptr;
-        void* tbuf = nullptr;
-        size_t tlen = 0;
-        if (ws) {
-            // caller's workspace (the allocation-free entry): keys, records, sort scratch
-            size_t need = 0;
-            if (int e = query_ws_bytes<TQ>(n, (int)ncol, &need)) return e;
-            if (need > ws_bytes) { set_error("query workspace too small"); return -1; }
-            auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-            char* b = (char*)ws;
-            keys = (uint32_t*)b;
-            rec = (QRec<TQ>*)(b + up(2 * n * sizeof(uint32_t)));
-            tbuf = b + up(2 * n * sizeof(uint32_t)) + up(2 * n * sizeof(QRec<TQ>));
-            tlen = std::max<size_t>(tmp, 256);
+        if (ws) {                             // caller's workspace (the allocation-free entry)
+            if (query_ws_bytes<TQ>(n, g.nx, g.ny) > ws_bytes) { set_error("query workspace too small"); return -1; }
+            cnt = (uint32_t*)ws;
+            rec = (QRec<TQ>*)((char*)ws + cb);
         } else {
-            if (qs_key_.alloc(2 * n * sizeof(uint32_t)) || qs_rec_.alloc(2 * n * sizeof(QRec<TQ>)) ||
-                qs_tmp_.alloc(std::max<size_t>(tmp, 256)))
-                return -3;
-            keys = (uint32_t*)qs_key_.get();
+            if (qs_cnt_.alloc(cb) || qs_rec_.alloc(n * sizeof(QRec<TQ>))) return -3;
+            cnt = (uint32_t*)qs_cnt_.get();
             rec = (QRec<TQ>*)qs_rec_.get();
-            tbuf = qs_tmp_.get();
-            tlen = qs_tmp_.size();
         }
-        PROF("k_query_sort", (launch_query_sort<TQ>(n, g, x, y, z, bits, keys, rec, tbuf, tlen, st)));
-        J.srec = rec + n;
+        PROF("k_query_sort", (launch_query_bins<TQ>(n, g, x, y, z, cnt, rec, st)));
+        J.srec = rec;
     }
     PROF("k_query", (launch_query<R, TQ>(J, st)));
     return 0;

@@ -170,15 +170,13 @@ template <typename R, typename TQ>
 hipError_t launch_query(const QueryJob<R, TQ>& J, hipStream_t st);
 template <typename R>
 hipError_t launch_pack(const PackJob<R>& J, hipStream_t st);
-// Cell order of a query batch (qsort.hip): key[p] = column of query p's cell,
-// rec[p] = (x, y, z, p), then a radix sort of (key, rec) over key_bits bits.
-// keys and recs hold 2 n entries (input half, sorted half), tmp tmp_bytes
-// (query_sort_tmp_bytes).  On return recs + n holds the cell-ordered records.
+// Cell order of a query batch (qsort.hip): recs receives (x, y, z, p) of every
+// query p, grouped by tiles of neighbouring columns; counts holds
+// query_bins_bytes bytes of scratch.
+size_t query_bins_bytes(int64_t n, int nx, int ny);
 template <typename TQ>
-hipError_t query_sort_tmp_bytes(int64_t n, int key_bits, size_t* tmp_bytes);
-template <typename TQ>
-hipError_t launch_query_sort(int64_t n, const GridGeom& g, const TQ* x, const TQ* y, const TQ* z, int key_bits,
-                             uint32_t* keys, QRec<TQ>* recs, void* tmp, size_t tmp_bytes, hipStream_t st);
+hipError_t launch_query_bins(int64_t n, const GridGeom& g, const TQ* x, const TQ* y, const TQ* z, uint32_t* counts,
+                             QRec<TQ>* recs, hipStream_t st);
 // Z operands, then the MFMA quadratic form of the filtered eta2 pair sum
 hipError_t launch_qf_zgen(const QfJob& J, hipStream_t st);
 hipError_t launch_qf_forms(const QfJob& J, hipStream_t st);
@@ -554,7 +552,7 @@ private:
     DevBuf f_[19];
     DevBuf q_in_, q_out_;
     DevBuf pk_eta_, pk_C_, pk_D_;             // query records of the two active slots
-    DevBuf qs_key_, qs_rec_, qs_tmp_;         // cell-ordered query batches
+    DevBuf qs_cnt_, qs_rec_;                  // cell-ordered query batches
     template <typename R>
     int pack();
     template <typename R>
@@ -621,10 +619,10 @@ struct BatchStats {
     double setup_ms = 0;                     // host time of the groups' set-up (incl. waiting for the builds)
 };
 int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, BatchStats* stats);
-// Device bytes of the cell-ordering buffers of an n-query batch on a grid of
-// ncol columns (0 below the ordering threshold); 0 or a negative code.
+// Device bytes of the cell-ordering buffers of an n-query batch on an nx x ny
+// grid (0 below the ordering threshold).
 template <typename TQ>
-int query_ws_bytes(int64_t n, int ncol, size_t* bytes);
+size_t query_ws_bytes(int64_t n, int nx, int ny);
 // Grid::query_device_f32 with the ordering buffers in a fixed device array
 // (noalloc.hip): allocates no device memory; too large a batch gives -1.
 int query_device_f32_noalloc(Grid& grid, int64_t n, double t, const float* x, const float* y, const float* z,

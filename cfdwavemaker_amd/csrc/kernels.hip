@@ -1009,7 +1009,8 @@ __global__ __launch_bounds__(256) void k_grad_dt(const R* __restrict__ D, R* __r
 // The two time slots a query reads, (tstep+1)%4 and (tstep+2)%4, are packed
 // after every fill/update by k_pack:
 //   column record (8 R): eta(tid1) eta(tid2) eta_t(tid1) eta_t(tid2) eta_x(0) eta_x(1) eta_y(0) eta_y(1)
-//   node records C and D (16 R each): for u, v, w in turn f, f_t, f_x, f_y, f_s,
+//   node records C and D (16 R each): for u, v, w in turn the piece f, f_x, f_y, f_s,
+//     then the piece u_t, v_t, w_t, pad;
 //     C from time slot tid1 and derivative slot 0, D from tid2 and derivative slot 1.
 // Levels are the fastest index, so the corners l and l+1 of a query share a
 // cache line and one query touches 8 node lines instead of 8 x 30 arrays.
@@ -1023,16 +1024,16 @@ __global__ __launch_bounds__(256) void k_pack(PackJob<R> J) {
     R c[16], d[16];
 #pragma unroll
     for (int f = 0; f < 3; ++f) {
-        c[5 * f + 0] = J.F[f][J.tid1 * per + n];
-        c[5 * f + 1] = J.Ft[f][J.tid1 * per + n];
-        c[5 * f + 2] = J.Fx[f][n];
-        c[5 * f + 3] = J.Fy[f][n];
-        c[5 * f + 4] = J.Fs[f][n];
-        d[5 * f + 0] = J.F[f][J.tid2 * per + n];
-        d[5 * f + 1] = J.Ft[f][J.tid2 * per + n];
-        d[5 * f + 2] = J.Fx[f][per + n];
-        d[5 * f + 3] = J.Fy[f][per + n];
-        d[5 * f + 4] = J.Fs[f][per + n];
+        c[4 * f + 0] = J.F[f][J.tid1 * per + n];
+        c[4 * f + 1] = J.Fx[f][n];
+        c[4 * f + 2] = J.Fy[f][n];
+        c[4 * f + 3] = J.Fs[f][n];
+        c[12 + f] = J.Ft[f][J.tid1 * per + n];
+        d[4 * f + 0] = J.F[f][J.tid2 * per + n];
+        d[4 * f + 1] = J.Fx[f][per + n];
+        d[4 * f + 2] = J.Fy[f][per + n];
+        d[4 * f + 3] = J.Fs[f][per + n];
+        d[12 + f] = J.Ft[f][J.tid2 * per + n];
     }
     c[15] = 0;
     d[15] = 0;
@@ -1074,9 +1075,10 @@ __device__ __forceinline__ double cart2sigmaS(double zpt, double e, double h, do
 }
 
 // The same map in FP32 for FP32 grids (k_query<float, .>): divisions by the
-// grid constants become products with their reciprocals, pow and atan the
-// FP32 library functions.  The sigma coordinate then carries a few 1e-7 of
-// absolute error, far below the FP32 grid values' own.
+// grid constants become products with their reciprocals, pow the hardware's
+// 2^(b log2 x) (x in [0, tanab]: its relative error grows only where the result
+// is small), atan the FP32 library function.  The sigma coordinate then carries
+// a few 1e-7 of absolute error, far below the FP32 grid values' own.
 struct QueryConst {
     double inv_dx, inv_dy, inv_dt;     // 1 / dx, 1 / dy, 1 / dt
     float h, swl, tanab;               // the FP64 map's depth, swl and tanab
@@ -1087,7 +1089,7 @@ __device__ __forceinline__ float cart2sigmaS_f(float zpt, float e, const QueryCo
     float sigma = (z - (e - K.swl)) / (K.h + (e - K.swl));
     sigma = sigma < -1.f ? -1.f : sigma;
     sigma = sigma > 0.f ? 0.f : sigma;
-    return 1.f - atanf(powf(-sigma * K.tanab, K.itb)) * K.ita;
+    return 1.f - atanf(__builtin_amdgcn_exp2f(K.itb * __builtin_amdgcn_logf(-sigma * K.tanab))) * K.ita;
 }
 
 // A packed record of N values (N a multiple of 4) at a 16-byte aligned
@@ -1112,59 +1114,109 @@ __device__ __forceinline__ void load_rec(R (&r)[N], const R* __restrict__ p) {
     }
 }
 
-// x stage of spline_interp_velo (lsgrid_spline.cpp:386-502) for the three
-// fields of the node pair (lo at i, hi at i+1): Hermite value, and linear
-// d/dy, d/dt, d/ds.
-template <typename R>
-__device__ __forceinline__ void xstage(R (&xr)[3], R (&yr)[3], R (&tr)[3], R (&sr)[3],
-                                       const R* __restrict__ plo, const R* __restrict__ phi, R xd, R dx) {
-    R a[16], b[16];
-    load_rec(a, plo);
-    load_rec(b, phi);
-#pragma unroll
-    for (int f = 0; f < 3; ++f) {
-        const int o = 5 * f;
-        const R ac = dx * a[o + 2] - (b[o] - a[o]);
-        const R bc = -dx * b[o + 2] + (b[o] - a[o]);
-        xr[f] = herm(a[o], b[o], ac, bc, xd);
-        yr[f] = lin(a[o + 3], b[o + 3], xd);
-        tr[f] = lin(a[o + 1], b[o + 1], xd);
-        sr[f] = lin(a[o + 4], b[o + 4], xd);
-    }
+// Four lanes serve four queries together: a node record is four 16-byte (FP64:
+// 32-byte) pieces, lane f < 3 of the quad takes field f's {value, d/dx, d/dy,
+// d/ds} and lane 3 the three d/dt, so that a load of the wavefront reads 16
+// whole records where a record per lane touched 64 lines in each of four
+// loads.  The weights of a query come from its own lane by quad broadcasts.
+template <int Q>
+__device__ __forceinline__ int quad_bc(int v) {
+    return __builtin_amdgcn_mov_dpp(v, Q * 0x55, 0xF, 0xF, true);
+}
+template <int Q>
+__device__ __forceinline__ float quad_bc(float v) {
+    return __int_as_float(quad_bc<Q>(__float_as_int(v)));
+}
+template <int Q>
+__device__ __forceinline__ double quad_bc(double v) {
+    return __hiloint2double(quad_bc<Q>(__double2hiint(v)), quad_bc<Q>(__double2loint(v)));
 }
 
-// x, y and s stages of spline_interp_velo (lsgrid_spline.cpp:386-502) on one
-// time slot's records for all three fields: value v and d/dt vt at (xd, yd, sd)
-// inside the cell of columns col = {(i,j), (i,j+1), (i+1,j), (i+1,j+1)} between
-// levels l and l+1, both edge clamped (lsgrid_spline.cpp:375-384).  Each record
-// is read once.
+// herm(f0, f1, d f0' - (f1 - f0), -d f1' + (f1 - f0), u) as weights of f0, f1, f0', f1'
 template <typename R>
-__device__ __forceinline__ void slot_velo(R (&v)[3], R (&vt)[3], const R* __restrict__ pk, const int64_t (&col)[4],
-                                          int nl, int l, R xd, R yd, R sd, R dx, R dy, R ds) {
-    const int lp = min(l + 1, nl - 1);
-    R yv[2][3], sv[2][3], tv[2][3];
+struct Herm4 {
+    R a, b, c, d;
+};
+template <typename R>
+__device__ __forceinline__ Herm4<R> herm_w(R u, R d) {
+    const R v = (R)1 - u, w = u * v, e = w * (v - u);
+    return {v + e, u - e, d * (w * v), -(d * (w * u))};
+}
+// the same for one lane of the quad: lane 3 interpolates linearly
+template <typename R>
+__device__ __forceinline__ Herm4<R> quad_w(R u, R d, bool lin3) {
+    Herm4<R> w = herm_w(u, d);
+    if (lin3) w = {(R)1 - u, u, (R)0, (R)0};
+    return w;
+}
+template <typename R>
+__device__ __forceinline__ R herm4(const Herm4<R>& w, R f0, R f1, R d0, R d1) {
+    return w.a * f0 + w.b * f1 + w.c * d0 + w.d * d1;
+}
+
+// x, y and s stages of spline_interp_velo (lsgrid_spline.cpp:386-502) of one
+// query on one time slot's records, this lane's piece: S[0] is the field's
+// value (lanes 0-2), S[0..2] the three d/dt (lane 3).  Byte offsets of this
+// lane's piece at level 0 of the cell's columns (i, j), (i, j + 1), (i + 1, j),
+// (i + 1, j + 1) in col, levels l and lp (both edge clamped,
+// lsgrid_spline.cpp:375-384).
+// O: 32-bit byte offsets for packed slots below 4 GiB, else 64-bit ones.
+template <typename O, typename R>
+__device__ __forceinline__ void quad_slot(R (&S)[3], const R* __restrict__ pk, const O (&col)[4], int l, int lp,
+                                          const Herm4<R>& wx, const Herm4<R>& wy, const Herm4<R>& ws, R xd,
+                                          R yd, R sd) {
+    R Y[2][4];
 #pragma unroll
     for (int lv = 0; lv < 2; ++lv) {
-        const int ll = lv ? lp : l;
-        R x0[3], y0[3], t0[3], s0[3], x1[3], y1[3], t1[3], s1[3];
-        xstage(x0, y0, t0, s0, pk + 16 * (col[0] * nl + ll), pk + 16 * (col[2] * nl + ll), xd, dx);
-        xstage(x1, y1, t1, s1, pk + 16 * (col[1] * nl + ll), pk + 16 * (col[3] * nl + ll), xd, dx);
+        const O lo = (O)(lv ? lp : l) * (O)(16 * sizeof(R));
+        R X[2][4];
 #pragma unroll
-        for (int f = 0; f < 3; ++f) {
-            const R ac = dy * y0[f] - (x1[f] - x0[f]);
-            const R bc = -dy * y1[f] + (x1[f] - x0[f]);
-            yv[lv][f] = herm(x0[f], x1[f], ac, bc, yd);
-            sv[lv][f] = lin(s0[f], s1[f], yd);
-            tv[lv][f] = lin(t0[f], t1[f], yd);
+        for (int jj = 0; jj < 2; ++jj) {
+            R a[4], b[4];
+            load_rec(a, reinterpret_cast<const R*>(reinterpret_cast<const char*>(pk) + (O)(col[jj] + lo)));
+            load_rec(b, reinterpret_cast<const R*>(reinterpret_cast<const char*>(pk) + (O)(col[2 + jj] + lo)));
+            X[jj][0] = herm4(wx, a[0], b[0], a[1], b[1]);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) X[jj][k] = lin(a[k], b[k], xd);
         }
-    }
+        Y[lv][0] = herm4(wy, X[0][0], X[1][0], X[0][2], X[1][2]);
 #pragma unroll
-    for (int f = 0; f < 3; ++f) {
-        const R a = ds * sv[0][f] - (yv[1][f] - yv[0][f]);
-        const R b = -ds * sv[1][f] + (yv[1][f] - yv[0][f]);
-        v[f] = herm(yv[0][f], yv[1][f], a, b, sd);
-        vt[f] = lin(tv[0][f], tv[1][f], sd);
+        for (int k = 1; k < 4; ++k) Y[lv][k] = lin(X[0][k], X[1][k], yd);
     }
+    S[0] = herm4(ws, Y[0][0], Y[1][0], Y[0][3], Y[1][3]);
+    S[1] = lin(Y[0][1], Y[1][1], sd);
+    S[2] = lin(Y[0][2], Y[1][2], sd);
+}
+
+// A query's cell and the fractions in it, held by its own lane.
+template <typename R>
+struct QueryCell {
+    int c00, dj, di, l0, l1;       // column of (i, j), steps to j + 1 and i + 1 (0 at the edge), base levels of the slots
+    R xd, yd, s0, s1, td;
+};
+// u, v, w of query Q of the quad, given to its lane
+template <int Q, typename O, typename R>
+__device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, const R* __restrict__ pkC,
+                                           const R* __restrict__ pkD, int nl, int piece, R dx, R dy, R ds, R dt) {
+    const bool lin3 = piece == 3;
+    const O per = (O)nl * (O)(16 * sizeof(R));
+    const O c00 = (O)quad_bc<Q>(C.c00) * per + (O)(piece * 4 * sizeof(R));
+    const O dj = (O)quad_bc<Q>(C.dj) * per, di = (O)quad_bc<Q>(C.di) * per;
+    const O col[4] = {c00, c00 + dj, c00 + di, c00 + di + dj};
+    const R xd = quad_bc<Q>(C.xd), yd = quad_bc<Q>(C.yd), s0 = quad_bc<Q>(C.s0), s1 = quad_bc<Q>(C.s1);
+    const int l0 = quad_bc<Q>(C.l0), l1 = quad_bc<Q>(C.l1);
+    const Herm4<R> wx = quad_w(xd, dx, lin3), wy = quad_w(yd, dy, lin3);
+    R A[3], B[3];
+    quad_slot<O>(A, pkC, col, l0, min(l0 + 1, nl - 1), wx, wy, quad_w(s0, ds, lin3), xd, yd, s0);
+    quad_slot<O>(B, pkD, col, l1, min(l1 + 1, nl - 1), wx, wy, quad_w(s1, ds, lin3), xd, yd, s1);
+    // the t stage of lane f's field with lane 3's d/dt of that field
+    R ta = quad_bc<3>(A[0]), tb = quad_bc<3>(B[0]);
+    const R ta1 = quad_bc<3>(A[1]), tb1 = quad_bc<3>(B[1]), ta2 = quad_bc<3>(A[2]), tb2 = quad_bc<3>(B[2]);
+    if (piece == 1) { ta = ta1; tb = tb1; }
+    if (piece == 2) { ta = ta2; tb = tb2; }
+    const R r = herm4(herm_w(quad_bc<Q>(C.td), dt), A[0], B[0], ta, tb);
+    const R u = quad_bc<0>(r), v = quad_bc<1>(r), w = quad_bc<2>(r);
+    if (piece == Q) { ov[0] = u; ov[1] = v; ov[2] = w; }
 }
 }  // namespace
 
@@ -1173,10 +1225,23 @@ __device__ __forceinline__ void slot_velo(R (&v)[3], R (&vt)[3], const R* __rest
 // fraction taken in float.  TQ: coordinate/output type of the queries.  With
 // J.srec thread k evaluates the k-th query in cell order; p is always the
 // query's index in the caller's arrays.
-template <typename R, typename TQ>
+// What bounds it (1e7 queries, 748 us): the loads of the 16 node records, 1 KiB
+// per query through the L1 (260 us), the results' scattered stores (130), and
+// 1314 vector instructions per wavefront (330 at the issue limit), which overlap
+// only in part; a register cap that gives more waves spills and loses.  Cell-
+// ordered blocks are dealt so that each XCD takes one contiguous range of them:
+// neighbouring cells then share an L2 (past L2 154 instead of 270 MB per 1e6
+// queries).
+template <typename R, typename TQ, typename O>
 __global__ __launch_bounds__(256) void k_query(QueryJob<R, TQ> J, QueryConst K) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= J.n) return;
+    int64_t blk = blockIdx.x;
+    if (J.srec) {
+        const int64_t per = gridDim.x >> 3;           // a multiple of 8 blocks (launch_query)
+        blk = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    }
+    const int64_t kq = blk * 256 + threadIdx.x;
+    const bool live = kq < J.n;
+    const int64_t k = live ? kq : J.n - 1;            // whole quads run
     int64_t p = k;
     double xpt, ypt, zpt;
     if (J.srec) {
@@ -1246,18 +1311,23 @@ __global__ __launch_bounds__(256) void k_query(QueryJob<R, TQ> J, QueryConst K) 
     int l0 = (int)k0, l1 = (int)k1;
     l0 = l0 < 0 ? 0 : (l0 > nl - 1 ? nl - 1 : l0);
     l1 = l1 < 0 ? 0 : (l1 > nl - 1 ? nl - 1 : l1);
-    const R ds = (R)g.ds;
     const double rmp = J.ramp_scale ? (double)J.ramp_scale[p] : 1.0;
     const TQ oeta = (TQ)((double)eta * rmp);
-    R VC[3], VCt[3], VD[3], VDt[3];
-    slot_velo(VC, VCt, J.pk_C, ac, nl, l0, xd, yd, sd0, dx, dy, ds);
-    slot_velo(VD, VDt, J.pk_D, ac, nl, l1, xd, yd, sd1, dx, dy, ds);
+    QueryCell<R> Q;
+    Q.c00 = (int)ac[0]; Q.dj = j1 - j; Q.di = (i1 - i) * ny;
+    Q.l0 = l0; Q.l1 = l1;
+    Q.xd = xd; Q.yd = yd; Q.s0 = sd0; Q.s1 = sd1; Q.td = tdR;
+    const R ds = (R)g.ds;
+    R vel[3] = {0, 0, 0};
+    const int piece = threadIdx.x & 3;
+    quad_query<0, O>(vel, Q, J.pk_C, J.pk_D, nl, piece, dx, dy, ds, dt);
+    quad_query<1, O>(vel, Q, J.pk_C, J.pk_D, nl, piece, dx, dy, ds, dt);
+    quad_query<2, O>(vel, Q, J.pk_C, J.pk_D, nl, piece, dx, dy, ds, dt);
+    quad_query<3, O>(vel, Q, J.pk_C, J.pk_D, nl, piece, dx, dy, ds, dt);
+    if (!live) return;
     TQ ov[3];
 #pragma unroll
-    for (int f = 0; f < 3; ++f) {
-        const R a = dt * VCt[f] - (VD[f] - VC[f]), b = -dt * VDt[f] + (VD[f] - VC[f]);
-        ov[f] = (TQ)((double)herm(VC[f], VD[f], a, b, tdR) * rmp);
-    }
+    for (int f = 0; f < 3; ++f) ov[f] = (TQ)((double)vel[f] * rmp);
     if (J.o_aos) {
         // {eta, u, v, w} of the query in one vector store (16 B FP32, 2 x 16 B FP64)
         if constexpr (sizeof(TQ) == 4) {
@@ -1489,7 +1559,11 @@ hipError_t launch_query(const QueryJob<R, TQ>& J, hipStream_t st) {
     K.inv_dx = 1.0 / J.g.dx; K.inv_dy = 1.0 / J.g.dy; K.inv_dt = 1.0 / J.dt;
     K.h = (float)J.g.h; K.swl = (float)J.g.swl; K.tanab = (float)J.tanab;
     K.ita = (float)(1.0 / J.tan_a); K.itb = (float)(1.0 / J.tan_b); K.inv_ds = (float)(1.0 / J.g.ds);
-    hipLaunchKernelGGL((k_query<R, TQ>), dim3(nblk(J.n)), dim3(256), 0, st, J, K);
+    const unsigned nb = J.srec ? (nblk(J.n) + 7) / 8 * 8 : nblk(J.n);
+    if ((int64_t)J.g.nx * J.g.ny * J.g.nl * 16 * (int64_t)sizeof(R) <= (int64_t)UINT32_MAX)
+        hipLaunchKernelGGL((k_query<R, TQ, uint32_t>), dim3(nb), dim3(256), 0, st, J, K);
+    else
+        hipLaunchKernelGGL((k_query<R, TQ, uint64_t>), dim3(nb), dim3(256), 0, st, J, K);
     return hipGetLastError();
 }
 

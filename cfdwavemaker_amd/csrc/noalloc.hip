@@ -2,13 +2,13 @@
 // cfdwm_grid_query_device_f32 for callers that cannot allocate device memory
 // (code under HIP graph capture, tight serving loops, harnesses that forbid
 // hipMalloc).  Batches of 65,536 queries or more are evaluated in cell order;
-// the keys, query records and radix-sort scratch of that ordering live here in
-// a file-scope device array instead of the grid's own buffers.  Each GPU holds
+// the tile counts and query records of that ordering live here in a file-scope
+// device array instead of the grid's own buffers.  Each GPU holds
 // its own copy of the array until the process ends.  Calls are enqueued on
 // the library stream, one after another, so they never overlap; a caller that
 // enqueued a query on another stream while one of these runs would race for
-// the array.  Nothing in the array needs clearing: the key pass writes every
-// key and record, the sort writes its own scratch.
+// the array.  Nothing in the array needs clearing: the counting pass writes
+// every count, the placing pass every record.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -20,6 +20,7 @@ namespace cfdwm {
 
 namespace {
 constexpr size_t kScratchBytes = size_t(64) << 20;     // 64 MiB per GPU
+constexpr int64_t kMaxQueries = 1115336;               // the entry's limit; their buffers take 34 MiB at most
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -56,20 +57,10 @@ int query_device_f32_noalloc(Grid& grid, int64_t n, double t, const float* x, co
                              float* eta, float* u, float* v, float* w) {
     if (n <= 0) return 0;
     if (int e = Engine::get().init()) return e;
-    const int ncol = grid.g.nx * grid.g.ny;
-    size_t need = 0;
-    if (int e = query_ws_bytes<float>(n, ncol, &need)) return e;
-    if (need > kScratchBytes) {
-        // the largest batch whose ordering buffers fit the array
-        int64_t lo = 0, hi = n;
-        while (hi - lo > 1) {
-            const int64_t mid = lo + (hi - lo) / 2;
-            size_t b = 0;
-            if (query_ws_bytes<float>(mid, ncol, &b)) return -3;
-            (b <= kScratchBytes ? lo : hi) = mid;
-        }
+    const size_t need = query_ws_bytes<float>(n, grid.g.nx, grid.g.ny);
+    if (n > kMaxQueries || need > kScratchBytes) {
         set_error("allocation-free query: " + std::to_string(n) + " queries exceed the maximum of " +
-                  std::to_string(lo) + " for this grid (" + std::to_string(kScratchBytes >> 20) +
+                  std::to_string(kMaxQueries) + " for this grid (" + std::to_string(kScratchBytes >> 20) +
                   " MiB of device scratch)");
         return -1;
     }

@@ -75,3 +75,34 @@ def test_device_f32_queries_cell_order_matches_caller_order(precision, shape):
         b, s = b.cpu().numpy(), s.cpu().numpy()
         assert np.all(np.isfinite(b))
         assert np.array_equal(b, s)
+
+
+@pytest.mark.parametrize("nx,ny,nl,n", [(1, 1, 1, 65536), (1, 37, 3, 65537), (130, 1, 5, 70_001), (67, 131, 4, 300_003),
+                                        (300, 260, 2, 1_100_000)])
+def test_tiles_of_odd_grids(nx, ny, nl, n):
+    """Grids one column or level wide, tiles that overhang the grid, batch sizes
+    around the ordering threshold, the blocks' shares and the largest tile
+    counts; a cluster of queries in one cell and a run of NaN coordinates (which
+    clamp to an edge cell): bit for bit what batches below the threshold give."""
+    from cfdwavemaker_amd import engine as eng
+    import torch
+    from cfdwavemaker_amd.seastate import make_sea
+    sea = eng.Sea(make_sea(6, 1.0, 8.0, 20.0, seed=1, ndir=2).as_dict(), precision=eng.FP32, with_direct=False)
+    dom = (3.0, 3.0 + 2.0 * (nx - 1), -4.0, -4.0 + 3.0 * (ny - 1))
+    g = sea.grid(dom, nx, ny, nl, 0.0, 0.5, 0.7, 1.5, 20.0)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(dom[0] - 5, dom[1] + 5, n).astype(np.float32)
+    y = rng.uniform(dom[2] - 5, dom[3] + 5, n).astype(np.float32)
+    z = rng.uniform(-21.0, 2.0, n).astype(np.float32)
+    x[: n // 3], y[: n // 3] = dom[0], dom[2]
+    x[n // 2: n // 2 + 70] = np.nan
+    X, Y, Z = (torch.tensor(a, device="cuda") for a in (x, y, z))
+    big = torch.full((n, 4), 7.0, dtype=torch.float32, device="cuda")
+    small = torch.full((n, 4), 8.0, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    g.kinematics_device_f32(n, 0.2, X.data_ptr(), Y.data_ptr(), Z.data_ptr(), big.data_ptr())
+    for a in range(0, n, 50_000):
+        m = min(50_000, n - a)
+        g.kinematics_device_f32(m, 0.2, X[a:].data_ptr(), Y[a:].data_ptr(), Z[a:].data_ptr(), small[a:].data_ptr())
+    eng.sync()
+    assert torch.equal(torch.nan_to_num(big, nan=1e30), torch.nan_to_num(small, nan=1e30))
