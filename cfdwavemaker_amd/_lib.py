@@ -138,7 +138,7 @@ def load(path: str | None = None) -> C.CDLL:
     L.cfdwm_grid_export.restype = _i64
     L.cfdwm_grid_export.argtypes = [C.c_void_p, C.c_int, _dp]
     L.cfdwm_grid_query.restype = C.c_int
-    L.cfdwm_grid_query.argtypes = [C.c_void_p, _i64] + [_dp] * 5
+    L.cfdwm_grid_query.argtypes = [C.c_void_p, _i64] + [C.c_void_p] * 5
     L.cfdwm_grid_query_device_f32.restype = C.c_int
     L.cfdwm_grid_query_device_f32.argtypes = [C.c_void_p, _i64, _d] + [C.c_void_p] * 7
     L.cfdwm_grid_query_device_f32_noalloc.restype = C.c_int

@@ -65,6 +65,38 @@ int DevBuf::upload(const void* src, size_t bytes, hipStream_t st) {
     return 0;
 }
 
+// ----------------------------------------------------------------- PinPool
+PinPool::~PinPool() {
+    for (void* p : idle_) (void)hipHostFree(p);
+}
+void* PinPool::take() {
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (!idle_.empty()) {
+            void* p = idle_.back();
+            idle_.pop_back();
+            return p;
+        }
+    }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+void PinPool::put(void* p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (idle_.size() < kKeep) {
+            idle_.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 // ------------------------------------------------------------------ Engine
 Engine& Engine::get() {
     static Engine e;
@@ -101,6 +133,12 @@ std::shared_ptr<QdSpace> Engine::qd_space() {
     std::lock_guard<std::mutex> lk(qd_mu_);
     auto s = qd_space_.lock();
     if (!s) qd_space_ = s = std::make_shared<QdSpace>();
+    return s;
+}
+std::shared_ptr<PinPool> Engine::pin_pool() {
+    std::lock_guard<std::mutex> lk(qd_mu_);
+    auto s = pin_pool_.lock();
+    if (!s) pin_pool_ = s = std::make_shared<PinPool>();
     return s;
 }
 void Engine::prof_begin(hipStream_t st) {
@@ -228,6 +266,8 @@ int Sea::upload_t(bool with_direct) {
 
 int Sea::upload(bool with_direct) {
     if (int e = Engine::get().init()) return e;
+    pins = Engine::get().pin_pool();
+    pins->put(pins->take());                 // the first small query finds a buffer
     return prec == kFP32 ? upload_t<float>(with_direct) : upload_t<double>(with_direct);
 }
 
@@ -1778,6 +1818,8 @@ int Grid::write_vtk_dump(bool last) {
 
 // Query batches from this size on are evaluated in cell order.
 constexpr int64_t kQuerySortMin = 65536;
+// Host batches up to this size run on pinned memory (Grid::query).
+constexpr int64_t kQueryPinMax = PinPool::kBytes / (8 * sizeof(double));
 
 // The cell-ordering buffers of an n-query batch (tile counts, then records,
 // each part 256-byte aligned); 0 below the ordering threshold.
@@ -1832,6 +1874,34 @@ int Grid::query(int64_t n, const double* t, const double* x, const double* y, co
     if (n <= 0) return 0;
     hipStream_t st = Engine::get().stream();
     std::lock_guard<std::mutex> lk(sea->mu);
+    // small batches: the kernel reads its inputs from pinned memory and writes
+    // the results there, one launch and one wait where five copies of a few
+    // bytes cost 25 us (8192 queries: 44 against 102 us; twice as many: slower)
+    if (n <= kQueryPinMax && sea->pins) {
+        struct Pin {
+            PinPool& pool;
+            void* p;
+            ~Pin() { pool.put(p); }
+        } pin{*sea->pins, sea->pins->take()};
+        if (pin.p) {
+            double* b = (double*)pin.p;
+            double* o = b + 4 * n;
+            const size_t nb = n * sizeof(double);
+            std::memcpy(b, t, nb);
+            std::memcpy(b + n, x, nb);
+            std::memcpy(b + 2 * n, y, nb);
+            std::memcpy(b + 3 * n, z, nb);
+            const int rc = prec == kFP32
+                ? run_query<float, double>(n, b, 0.0, b + n, b + 2 * n, b + 3 * n, nullptr, nullptr, nullptr, nullptr, nullptr, o)
+                : run_query<double, double>(n, b, 0.0, b + n, b + 2 * n, b + 3 * n, nullptr, nullptr, nullptr, nullptr, nullptr, o);
+            // (whatever was launched is done with the buffer before it goes back)
+            const hipError_t e = hipStreamSynchronize(st);
+            if (rc) return rc;
+            CFDWM_HIP(e);
+            std::memcpy(out4, o, 4 * nb);
+            return 0;
+        }
+    }
     if (q_in_.alloc(4 * n * sizeof(double)) || q_out_.alloc(4 * n * sizeof(double))) return -3;
     double* b = (double*)q_in_.get();
     double* o = (double*)q_out_.get();

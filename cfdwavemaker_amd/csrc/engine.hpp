@@ -243,6 +243,22 @@ private:
     size_t n_ = 0;
 };
 
+// Pinned host buffers of kBytes each that kernels read and write in place
+// (small batches of the host entries: no copies up or down).  One per running
+// call; at most kKeep idle ones are kept.  Held by the seas, freed with the
+// last of them.
+class PinPool {
+public:
+    static constexpr size_t kBytes = size_t(512) << 10;
+    static constexpr size_t kKeep = 4;
+    ~PinPool();
+    void* take();                            // nullptr: not available (the caller then copies)
+    void put(void* p);
+private:
+    std::mutex mu_;
+    std::vector<void*> idle_;
+};
+
 // Kernel timing with HIP events on the engine stream (enabled on request).
 struct KernelTimes {
     double total_ms = 0;
@@ -268,6 +284,7 @@ public:
     // stream's, forked and joined with events; created on first use
     hipStream_t side_stream();
     std::shared_ptr<QdSpace> qd_space();
+    std::shared_ptr<PinPool> pin_pool();
     // timing: record an event pair around a launch when enabled
     void prof_enable(bool on) { prof_ = on; }
     bool prof_on() const { return prof_; }
@@ -286,6 +303,7 @@ private:
     hipEvent_t take_event();
     std::mutex qd_mu_;
     std::weak_ptr<QdSpace> qd_space_;
+    std::weak_ptr<PinPool> pin_pool_;
 };
 
 // A launch timed with an event pair when timing is on; errors return -3.
@@ -319,6 +337,7 @@ public:
     int prec = kFP64;
     int64_t nfilt() const { return (int64_t)tab.filt.rec.size(); }
     int upload(bool with_direct);
+    std::shared_ptr<PinPool> pins;           // set by upload
     template <typename R>
     const SeaDev<R>& dev() const;
     // balanced split of a pair table into nseg segments (cached on the device)

@@ -175,9 +175,23 @@ class Grid:
         return out
 
     def query(self, t, x, y, z):
-        t, x, y, z = (_f64(np.ravel(a)) for a in np.broadcast_arrays(t, x, y, z))
-        out = np.zeros((t.size, 4))
-        check(self.L.cfdwm_grid_query(self.h, t.size, _p(t), _p(x), _p(y), _p(z), _p(out)), "cfdwm_grid_query")
+        # one array holds the four inputs: rows filled by assignment, which
+        # broadcasts and converts (np.broadcast_arrays and a pointer object per
+        # array cost more than a small query on the GPU)
+        args = [np.asarray(a) for a in (t, x, y, z)]
+        shape = args[0].shape
+        for a in args[1:]:
+            if a.shape != shape:
+                shape = np.broadcast_shapes(*(b.shape for b in args))
+                break
+        q = np.empty((4,) + shape)
+        for k in range(4):
+            q[k] = args[k]
+        n = q[0].size
+        out = np.empty((n, 4))
+        p = q.ctypes.data
+        check(self.L.cfdwm_grid_query(self.h, n, p, p + 8 * n, p + 16 * n, p + 24 * n, out.ctypes.data),
+              "cfdwm_grid_query")
         return out
 
     def write_vtu(self, path, last=False, time_label="TimeValue"):
