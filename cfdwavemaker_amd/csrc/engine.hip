@@ -208,7 +208,68 @@ UvwRec<R> uvw_rec(const PairRec64& p, double h) {
     r.pkM = (R)(p.kM * s); r.pgM = (R)(-2.0 * h * p.kM * s);
     return r;
 }
+
+// Seas whose unfiltered pair sums at points go through the point forms run in
+// one direction with k ascending: there the pair profiles split.  At every size
+// measured the forms win (pair loop -> forms: 256 components, 4,096 points FP64
+// 1330 -> 184 us; 512 components, 131,072 points FP32 31.9 -> 6.9 ms; 48
+// components, 16 points 131 -> 39 us FP64, 101 -> 36 us FP32).  Directional
+// seas keep the pair loop: |k_i + k_m| has no such split.
+bool long_crested(const SeaTables& T) {
+    for (int i = 1; i < T.comp.n; ++i)
+        if (T.in.theta[i] != T.in.theta[0] || !(T.comp.k[i] >= T.comp.k[i - 1])) return false;
+    return true;
+}
 }  // namespace
+
+// Tables of the point forms.  Returns 0 where the tables' combined wavenumbers
+// (a square root of differences) are not those the split profiles use, k_m +
+// k_i and k_m - k_i, to a tolerance far below the working precision's effect.
+template <typename R>
+int Sea::point_build() {
+    const CompTable& c = tab.comp;
+    const int N = c.n, nrb = (N + 15) / 16;
+    const double tol = sizeof(R) == 4 ? 1e-8 : 1e-10;
+    hipStream_t st = Engine::get().stream();
+    std::vector<int> off(nrb + 1, 0);
+    for (int rb = 0; rb < nrb; ++rb) off[rb + 1] = off[rb] + (N - 16 * rb + 3) / 4;
+    const int steps = off[nrb];
+    std::vector<R> b((size_t)steps * 6 * 64, (R)0);
+    std::atomic<bool> fits(true);
+    parallel_rows(nrb, [&](int rb) {
+        const int i0 = 16 * rb, ie = std::min(N, i0 + 16);
+        R* o = b.data() + (size_t)off[rb] * 6 * 64;
+        for (int m0 = i0; m0 < N; m0 += 4, o += 6 * 64)
+            for (int i = i0; i < ie; ++i)
+                for (int m = std::max(m0, i + 1); m < std::min(N, m0 + 4); ++m) {
+                    const PairRec64& d = tab.direct.rec[tab.direct.rowoff[i] + (m - i - 1)];
+                    const double sp = c.k[m] + c.k[i], sm = c.k[m] - c.k[i];
+                    if (!(std::abs(d.kP - sp) <= tol * sp) || !(std::abs(d.kM - sm) <= tol * sm)) fits = false;
+                    R* e = o + (m - m0) * 16 + (i - i0);
+                    e[0] = (R)d.cwP; e[64] = (R)d.xP; e[128] = (R)d.cwM; e[192] = (R)d.xM;
+                    if (m < tab.filt.mhi[i]) {
+                        const PairRec64& f = tab.filt.rec[tab.filt.rowoff[i] + (m - i - 1)];
+                        e[256] = (R)(f.xP + f.xM); e[320] = (R)(f.xM - f.xP);
+                    }
+                }
+    }, 24);
+    if (!fits) return 0;
+    std::vector<PointRec> r((size_t)(N + 3) / 4 * 4);
+    for (size_t q = 0; q < r.size(); ++q) {
+        const int i = (int)std::min<size_t>(q, N - 1);
+        const double tau = 2. * 3.14159265358979323846;
+        r[q] = PointRec{c.k[i], c.k[i] / tau, c.omega[i] / tau, c.ph0[i] / tau, q < (size_t)N ? c.Zk[i] : 0.,
+                        (float)(c.k[i] * kLog2e), (float)(c.k[i] * kLog2e - (double)(float)(c.k[i] * kLog2e)), c.omega[i],
+                        c.ph0[i]};
+    }
+    if (pt_.coef.upload(b.data(), b.size() * sizeof(R), st)) return -3;
+    if (pt_.rec.upload(r.data(), r.size() * sizeof(PointRec), st)) return -3;
+    CFDWM_HIP(hipStreamSynchronize(st));
+    pt_.cth = c.cth[0];
+    pt_.sth = c.sth[0];
+    pt_.steps = steps;
+    return 0;
+}
 
 template <typename R>
 int Sea::upload_t(bool with_direct) {
@@ -245,7 +306,8 @@ int Sea::upload_t(bool with_direct) {
         return 0;
     };
     if (put_table(tab.filt, true, frow_, &fmhi_, fuvw_, fx_)) return -3;
-    if (with_direct && put_table(tab.direct, false, drow_, nullptr, duvw_, dx_)) return -3;
+    if (with_direct && long_crested(tab) && point_build<R>()) return -3;
+    if (with_direct && !pt_.steps && put_table(tab.direct, false, drow_, nullptr, duvw_, dx_)) return -3;
     SeaDev<R> d{};
     d.n = N;
     d.h = h; d.swl = tab.in.swl; d.x0 = tab.in.x0; d.y0 = tab.in.y0; d.rho = tab.in.rho;
@@ -643,6 +705,48 @@ int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, cons
     return 1;
 }
 
+// Segments of a point-forms launch: about equal shares of the table's steps,
+// the count that needs the fewest steps in sequence over the rounds of
+// resident blocks (three a CU in FP32, two in FP64, by their registers), each
+// row block entered counted as four steps more.
+int point_segments(int64_t n, int steps, bool fp32) {
+    if (const char* e = std::getenv("CFDWM_NSEG")) return std::max(1, std::min(std::atoi(e), steps));
+    const int64_t tiles = (n + 63) / 64, slots = fp32 ? 768 : 512;
+    int best = 1;
+    double cost = 0.;
+    for (int s = 1; s <= std::min(128, std::max(1, steps / 4)); ++s) {
+        const double c = (double)((tiles * s + slots - 1) / slots) * ((double)steps / s + 8.);
+        if (s == 1 || c < cost) { best = s; cost = c; }
+    }
+    return best;
+}
+
+// Long-crested seas: every output of the call from one pass over the pairs.
+// out: eta1, eta2, the four gradients, u, v, w, p (null: not asked for).
+template <typename R>
+int run_point_forms(Sea& s, const Sea::PointTables& T, int64_t n, const double* dx, const double* dy, const double* dz,
+                    const double* dt, uint32_t flags, bool want_eta2, double* const* out) {
+    PointJob J;
+    J.n = n; J.x = dx; J.y = dy; J.z = dz; J.t = dt;
+    J.cth = T.cth; J.sth = T.sth;
+    J.kmax = s.tab.kmax; J.swl = s.tab.in.swl; J.rho = s.tab.in.rho;
+    J.flags = flags;
+    J.want_eta2 = want_eta2 ? 1 : 0;
+    J.steps = T.steps;
+    J.nseg = point_segments(n, T.steps, sizeof(R) == 4);
+    J.coef = T.coef.get();
+    J.mr = (const PointRec*)T.rec.get();
+    J.o_eta1 = out[0]; J.o_eta2 = out[1];
+    for (int k = 0; k < 4; ++k) J.o_g[k] = out[2 + k];
+    J.o_u = out[6]; J.o_v = out[7]; J.o_w = out[8]; J.o_p = out[9];
+    if (J.nseg > 1) {
+        if (s.partial.alloc((size_t)J.nseg * n * 11 * sizeof(double))) return -3;
+        J.partial = (double*)s.partial.get();
+    }
+    PROF("k_point_forms", launch_point_forms<R>(s.dev<R>(), J, Engine::get().stream()));
+    return 0;
+}
+
 template <typename R>
 int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const double* dz, const double* dt,
                uint32_t flags, bool want_cols, bool want_eta2, bool want_lev, double* o) {
@@ -685,6 +789,21 @@ int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const doub
         PROF("k_levels_points", launch_levels<R>(S, J, false, 1, st));
     }
     return 0;
+}
+
+// Whether any two of a call's arrays of n doubles share memory, outputs with
+// inputs or with each other: outputs then go through the scratch arrays.
+bool overlap(int64_t n, std::initializer_list<const double*> in, double* const* out) {
+    auto meet = [n](const double* a, const double* b) {
+        return a && b && (uintptr_t)a < (uintptr_t)(b + n) && (uintptr_t)b < (uintptr_t)(a + n);
+    };
+    for (int q = 0; q < 10; ++q) {
+        for (const double* i : in)
+            if (meet(out[q], i)) return true;
+        for (int k = 0; k < q; ++k)
+            if (meet(out[q], out[k])) return true;
+    }
+    return false;
 }
 
 // Smit et al. u, v, w, p at points (smit.hip); o[0..n) and o[n..2n) hold the
@@ -739,10 +858,25 @@ int Sea::eval_points(int64_t n, const double* x, const double* y, const double* 
         else CFDWM_HIP(hipMemsetAsync(b + 2 * n, 0, n * sizeof(double), st));
         dx = b; dy = b + n; dz = b + 2 * n; dt = b + 3 * n;
     }
+    const PointTables* pf = want_lev && !smit && (flags & EV_SEC) && (flags & EV_DIRECT) ? point_tables() : nullptr;
+    double* const user[10] = {eta1, eta2, grads4, grads4 ? grads4 + n : nullptr,
+                              grads4 ? grads4 + 2 * n : nullptr, grads4 ? grads4 + 3 * n : nullptr, u, v, w, p};
+    if (pf && device_ptrs && !overlap(n, {x, y, z, t}, user)) {
+        if (const int e = prec == kFP32 ? run_point_forms<float>(*this, *pf, n, dx, dy, dz, dt, flags, want_eta2, user)
+                                        : run_point_forms<double>(*this, *pf, n, dx, dy, dz, dt, flags, want_eta2, user))
+            return e;
+        CFDWM_HIP(hipStreamSynchronize(st));
+        return 0;
+    }
     if (pts_out.alloc(10 * n * sizeof(double))) return -3;
     double* o = (double*)pts_out.get();
     int rc;
-    if (smit) {
+    if (pf) {
+        double* out[10];
+        for (int q = 0; q < 10; ++q) out[q] = o + q * n;
+        rc = prec == kFP32 ? run_point_forms<float>(*this, *pf, n, dx, dy, dz, dt, flags, want_eta2, out)
+                           : run_point_forms<double>(*this, *pf, n, dx, dy, dz, dt, flags, want_eta2, out);
+    } else if (smit) {
         // the stretch height eta1 + eta2 of every point, then the Smit kernels
         const bool e2 = tab.in.order >= 1;
         rc = prec == kFP32 ? run_points<float>(*this, n, dx, dy, dz, dt, 0, true, e2, false, o)

@@ -342,6 +342,13 @@ public:
     const SeaDev<R>& dev() const;
     // balanced split of a pair table into nseg segments (cached on the device)
     const Segment* segments(bool direct, int nseg);
+    // tables of the point forms (points.hip); null where the sea has none
+    struct PointTables {
+        DevBuf coef, rec;
+        int steps = 0;
+        double cth = 1, sth = 0;
+    };
+    const PointTables* point_tables() const { return pt_.steps ? &pt_ : nullptr; }
     // nseg segments of the components alone (no pair rows), for passes whose
     // pair sums come from the quadratic forms
     const Segment* comp_segments(int nseg);
@@ -424,6 +431,9 @@ public:
                     double* u, double* v, double* w, double* p, bool device_ptrs, bool smit_always = false);
 private:
     DevBuf ph_, cr_, act_, frow_, fmhi_, fuvw_, fx_, drow_, duvw_, dx_;
+    PointTables pt_;
+    template <typename R>
+    int point_build();
     std::map<std::pair<bool, int>, std::unique_ptr<DevBuf>> seg_cache_;
     std::map<int, std::unique_ptr<DevBuf>> cseg_cache_;
     std::unique_ptr<QfTables> qf_;

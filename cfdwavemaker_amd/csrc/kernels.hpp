@@ -68,6 +68,32 @@ enum : uint32_t {
     EV_ZSHIFT = 64u,    // profiles at z - swl (order 0)
 };
 
+// Points of long-crested seas (points.hip): the component as a column of the
+// pair tables, and the launch.  Tables: 16 rows i x 4 components m a step, row
+// blocks in turn, m from the block's first row; a step holds the sum and
+// difference coefficients of w and p and of eta2 (B1, B2) as six operands of
+// 64 values, value (m % 4) * 16 + i % 16, zero for m <= i.
+struct PointRec {
+    double k, kr, wr, pr;                 // k; k, omega and the phase over 2 pi
+    double X;                             // g k / omega C_k (dp2 kinetic terms)
+    float khi, klo;                       // k log2 e in two parts
+    double omega, ph0;
+};
+struct PointJob {
+    int64_t n = 0;
+    const double *x = nullptr, *y = nullptr, *z = nullptr, *t = nullptr;
+    double cth = 1, sth = 0, kmax = 0, swl = 0, rho = 0;
+    uint32_t flags = 0;
+    int steps = 0, nseg = 1, want_eta2 = 1;
+    const void* coef = nullptr;
+    const PointRec* mr = nullptr;
+    double *o_eta1 = nullptr, *o_eta2 = nullptr, *o_g[4] = {nullptr, nullptr, nullptr, nullptr};
+    double *o_u = nullptr, *o_v = nullptr, *o_w = nullptr, *o_p = nullptr;
+    double* partial = nullptr;            // [nseg][11][n] totals with several segments
+};
+template <typename R>
+hipError_t launch_point_forms(const SeaDev<R>& S, const PointJob& J, hipStream_t st);
+
 // A contiguous range of pair records (split-K over the pair sum).  Rows
 // [rlo, rhi) have pairs in it (row rlo from m = mstart, row rhi-1 up to
 // m = mend); rows [own_lo, own_hi) get their per-row terms (linear,

@@ -3,9 +3,7 @@
 #include "sea_tables.hpp"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
-#include <thread>
 
 namespace cfdwm {
 
@@ -48,23 +46,6 @@ void direct_D(double ki, double km, double thi, double thm, double depth,
     Dm = (2. * R2m * (ki * km * gamma + Rn * Rm)) / (R2m - kn * std::tanh(kn * depth)) +
          ((Rsn - Rsm) * (-Rsn * (km * km - Rm * Rm) + Rsm * (ki * ki - Rn * Rn))) /
              (R2m - kn * std::tanh(kn * depth));
-}
-
-// Runs body(i) for i in [0, n) on the host cores (rows have uneven cost:
-// rows are handed out one at a time).
-template <typename F>
-void parallel_rows(int n, F body) {
-    unsigned nt = std::thread::hardware_concurrency();
-    nt = std::max(1u, std::min(nt, 16u));
-    if (n < 64) nt = 1;
-    std::atomic<int> next(0);
-    auto work = [&]() {
-        for (int i = next++; i < n; i = next++) body(i);
-    };
-    std::vector<std::thread> th;
-    for (unsigned q = 1; q < nt; ++q) th.emplace_back(work);
-    work();
-    for (auto& t : th) t.join();
 }
 
 // 1 / (1 + exp(-2 k h)): folds cosh(k h) out of cosh(k (z+h)) / cosh(k h).

@@ -4,8 +4,11 @@
 //   filtered ("pair cache") set:  src/Irregular.cpp:805-967  (eta2, uvw2)
 //   unfiltered (direct) set:      src/Irregular.cpp:450-803  (u2, v2, w2, dp2)
 #pragma once
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace cfdwm {
@@ -81,6 +84,23 @@ struct SeaTables {
     PairTable direct;                // unfiltered semantics (u2, v2, w2, dp2): direct mode
     int64_t diag_filtered = 0;       // diagonal terms present in uvw2
 };
+
+// Runs body(i) for i in [0, n) on the host cores (rows have uneven cost:
+// rows are handed out one at a time).
+template <typename F>
+void parallel_rows(int n, F body, int serial_below = 64) {
+    unsigned nt = std::thread::hardware_concurrency();
+    nt = std::max(1u, std::min(nt, 16u));
+    if (n < serial_below) nt = 1;
+    std::atomic<int> next(0);
+    auto work = [&]() {
+        for (int i = next++; i < n; i = next++) body(i);
+    };
+    std::vector<std::thread> th;
+    for (unsigned q = 1; q < nt; ++q) th.emplace_back(work);
+    work();
+    for (auto& t : th) t.join();
+}
 
 // Builds all tables.  Returns an empty string on success, else an error text.
 std::string build_tables(const SeaInput& in, SeaTables& out, bool with_direct);

@@ -1,0 +1,146 @@
+"""Direct-mode points of long-crested seas through the split pair profiles on the
+matrix cores: against the oracle, and against the pair loop (the same sea with one
+component's direction an ulp away) at the edges of tiles, row blocks and segments."""
+import numpy as np
+import pytest
+
+from cfdwavemaker_amd.seastate import make_sea
+
+# FP64: rounding of sums over up to 1e4 pairs, exponents up to 100 eps.
+# FP32: terms good to a few FP32 ulps, at most 130 in a row in a chain.
+TOL = {"fp64": 1e-11, "fp32": 1e-5}
+FIELDS = ("eta1", "eta2", "u", "v", "w", "p")
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from cfdwavemaker_amd import engine
+    engine.load()
+    return engine
+
+
+def _sea(n, depth, **kw):
+    s = make_sea(n, 3.0, 9.0, depth, seed=n, ndir=1).as_dict()
+    s["theta"] = np.full(len(s["omega"]), 0.4)
+    s.update(kw)
+    return s
+
+
+def _pair_loop(s):
+    r = dict(s, theta=np.array(s["theta"], float))
+    r["theta"][0] = np.nextafter(r["theta"][0], 1.0)
+    return r
+
+
+def _points(m, depth, seed, lo=-1.0, hi=2.0):
+    rng = np.random.default_rng(seed)
+    return (rng.uniform(0.0, 40.0, m), rng.uniform(-60.0, 90.0, m), rng.uniform(-30.0, 30.0, m),
+            np.concatenate([rng.uniform(lo * depth, hi, m)]))
+
+
+def _fields(eng, sea, q):
+    import torch
+    f = sea.eval_fields_device(*(torch.tensor(a, device="cuda") for a in q))
+    return {k: v.cpu().numpy() for k, v in f.items()}
+
+
+def _check(got, ref, tol):
+    for k in FIELDS:
+        ok = np.isfinite(ref[k])          # coth(k h) itself is not a number past k h = 710
+        assert np.array_equal(ok, np.isfinite(got[k])), k
+        scale = np.max(np.abs(ref[k][ok]), initial=0.0)
+        err = np.max(np.abs(got[k] - ref[k])[ok], initial=0.0)
+        assert err <= tol * scale or (scale == 0 and err == 0), (k, err, scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,m,depth", [(1, 5, 20.0), (2, 64, 20.0), (15, 65, 30.0), (16, 1, 30.0), (17, 63, 8.0),
+                                       (32, 1000, 150.0), (33, 129, 50.0), (130, 300, 60.0)])
+def test_against_the_pair_loop(eng, prec, n, m, depth):
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    extra = dict(bandwidth=0.8, cutoff=1.7, swl=0.5) if n % 2 else {}
+    s = _sea(n, depth, **extra)
+    q = _points(m, depth, n)
+    _check(_fields(eng, eng.Sea(s, precision=p), q), _fields(eng, eng.Sea(_pair_loop(s)), q), TOL[prec])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nseg", ["1", "2", "7", "1000"])
+def test_segments(eng, prec, nseg, monkeypatch):
+    """Runs of the table that end anywhere: inside a row block, between two, in its first steps."""
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    s, q = _sea(50, 30.0), _points(70, 30.0, 3)
+    ref = _fields(eng, eng.Sea(_pair_loop(s)), q)
+    monkeypatch.setenv("CFDWM_NSEG", nseg)
+    _check(_fields(eng, eng.Sea(s, precision=p), q), ref, TOL[prec])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_components_far_apart(eng, prec):
+    """Rows of a block so far apart in k that the split leaves the number range in
+    FP32: those waves go pair by pair."""
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    s = _sea(20, 400.0, omega=np.linspace(0.2, 6.0, 20), k=np.linspace(0.2, 6.0, 20) ** 2 / 9.81)
+    q = _points(200, 400.0, 4)
+    _check(_fields(eng, eng.Sea(s, precision=p), q), _fields(eng, eng.Sea(_pair_loop(s)), q), TOL[prec])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_raw_depths(eng, prec):
+    """The second-order terms alone take z as given: above the surface and below the bed."""
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    s = _sea(40, 25.0)
+    t, x, y, z = _points(300, 25.0, 5, lo=-2.5, hi=6.0)
+    a, b = eng.Sea(s, precision=p), eng.Sea(_pair_loop(s))
+    for kind in ("u2", "v2", "w2", "dp2"):
+        g, r = a.eval(kind, t, x, y, z), b.eval(kind, t, x, y, z)
+        # every point on its own: the profiles span many orders of magnitude
+        # over these depths, so the scale is the largest field of points as high
+        assert np.all(np.isfinite(g) == np.isfinite(r))
+        order = np.argsort(z)
+        scale = np.maximum.accumulate(np.abs(r[order]))
+        deep = z[order] < -25.0
+        scale = np.where(deep, np.max(np.abs(r)), scale)
+        assert np.all(np.abs(g - r)[order] <= 4 * TOL[prec] * np.max(scale)), kind
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_against_the_oracle(eng, oracle, prec):
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    s = _sea(45, 35.0, ramptime=np.full(45, 20.0), starttime=np.zeros(45), duration=np.full(45, 30.0))
+    t, x, y, z = _points(50, 35.0, 6)
+    a, o = eng.Sea(s, precision=p), oracle.sea(s)
+    for kind in ("u", "v", "w", "dp"):
+        g, r = a.eval(kind, t, x, y, z), o.eval(kind, t, x, y, z)
+        assert np.max(np.abs(g - r)) <= TOL[prec] * np.max(np.abs(r)), kind
+
+
+@pytest.mark.gpu
+def test_outputs_that_share_memory_with_inputs(eng):
+    import torch
+    s, q = _sea(30, 30.0), _points(100, 30.0, 7)
+    sea = eng.Sea(s)
+    ref = _fields(eng, sea, q)
+    t, x, y, z = (torch.tensor(a, device="cuda") for a in q)
+    u = torch.empty(100, dtype=torch.float64, device="cuda")
+    eng.check(sea.L.cfdwm_eval_fields(sea.h, 99, t.data_ptr(), x.data_ptr(), y.data_ptr(), z.data_ptr(), None, None,
+                                      u.data_ptr(), x[1:].data_ptr(), z.data_ptr(), None, 1), "cfdwm_eval_fields")
+    assert np.array_equal(u[:99].cpu().numpy(), ref["u"][:99])
+    assert np.array_equal(x[1:].cpu().numpy(), ref["v"][:99])
+    assert np.array_equal(z[:99].cpu().numpy(), ref["w"][:99])
+
+
+@pytest.mark.gpu
+def test_unordered_components_take_the_pair_loop(eng):
+    """k out of order: the split does not hold, the fields do not change."""
+    s, q = _sea(40, 30.0), _points(80, 30.0, 8)
+    o = np.random.default_rng(1).permutation(40)
+    r = dict(s)
+    for k in ("omega", "A", "k", "phase", "theta"):
+        r[k] = np.asarray(s[k])[o]
+    _check(_fields(eng, eng.Sea(r), q), _fields(eng, eng.Sea(_pair_loop(r)), q), TOL["fp64"])
