@@ -749,13 +749,14 @@ int run_point_forms(Sea& s, const Sea::PointTables& T, int64_t n, const double* 
 
 template <typename R>
 int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const double* dz, const double* dt,
-               uint32_t flags, bool want_cols, bool want_eta2, bool want_lev, double* o) {
+               uint32_t flags, bool want_cols, bool want_lin, bool want_eta2, bool want_lev, double* o) {
     hipStream_t st = Engine::get().stream();
     const SeaDev<R>& S = s.dev<R>();
     if (want_cols) {
         ColumnJob<R> J;
         J.nslot = 1; J.ncol = n;
         J.x = dx; J.y = dy; J.t = dt;
+        J.want_lin = want_lin ? 1 : 0;
         J.want_eta2 = want_eta2 ? 1 : 0;
         J.o_eta1 = o; J.o_eta2 = o + n; J.o_gx = o + 2 * n; J.o_gy = o + 3 * n; J.o_gz = o + 4 * n; J.o_gp = o + 5 * n;
         J.nseg = want_eta2 ? pick_nseg(n, s.table_records(false)) : 1;
@@ -879,14 +880,15 @@ int Sea::eval_points(int64_t n, const double* x, const double* y, const double* 
     } else if (smit) {
         // the stretch height eta1 + eta2 of every point, then the Smit kernels
         const bool e2 = tab.in.order >= 1;
-        rc = prec == kFP32 ? run_points<float>(*this, n, dx, dy, dz, dt, 0, true, e2, false, o)
-                           : run_points<double>(*this, n, dx, dy, dz, dt, 0, true, e2, false, o);
+        rc = prec == kFP32 ? run_points<float>(*this, n, dx, dy, dz, dt, 0, true, true, e2, false, o)
+                           : run_points<double>(*this, n, dx, dy, dz, dt, 0, true, true, e2, false, o);
         if (!rc)
             rc = prec == kFP32 ? run_smit<float>(*this, n, dx, dy, dz, dt, o)
                                : run_smit<double>(*this, n, dx, dy, dz, dt, o);
     } else {
-        rc = prec == kFP32 ? run_points<float>(*this, n, dx, dy, dz, dt, flags, want_cols, want_eta2, want_lev, o)
-                           : run_points<double>(*this, n, dx, dy, dz, dt, flags, want_cols, want_eta2, want_lev, o);
+        const bool want_lin = eta1 || grads4;
+        rc = prec == kFP32 ? run_points<float>(*this, n, dx, dy, dz, dt, flags, want_cols, want_lin, want_eta2, want_lev, o)
+                           : run_points<double>(*this, n, dx, dy, dz, dt, flags, want_cols, want_lin, want_eta2, want_lev, o);
     }
     if (rc) return rc;
     const hipMemcpyKind kind = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;

@@ -25,6 +25,7 @@ struct ColumnJob {
     R* eta_grid = nullptr;
     const double *x = nullptr, *y = nullptr, *t = nullptr;
     int want_eta2 = 1;
+    int want_lin = 1;                     // 0: of the points only eta2 is asked for
     int pairs = 1;                        // 0: eta2 pair sum comes from the MFMA partials q2
     const float* q2 = nullptr;            // [nq2][q2stride] per-point partials (GRID)
     int nq2 = 0;
