@@ -435,19 +435,24 @@ int Sea::qform_meta(const QfTables** out) {
     qf_fallback = st_c != 0 || st_s != 0 || !(BC.err <= tol) || !(BS.err <= tol) || R < 1 || R > 32 || Rw < 1 ||
                   Rw > 32;
     if (qf_fallback) return 0;
-    const int nform = 1 + 2 * R + Rw;
+    // long-crested along x: every v coefficient is zero, no v forms (a third of
+    // the velocity forms' work; their sums were exact zeros)
+    int Rv = 0;
+    for (const PairRec64& r : P.rec)
+        if ((float)r.cvP != 0.f || (float)r.cvM != 0.f) { Rv = R; break; }
+    const int nform = 1 + R + Rv + Rw;
     const int nbarr = nlv == 1 ? 2 : 4;
     const int npad = (N + 127) / 128 * 128;
     const size_t nn = (size_t)npad * npad;
     std::vector<int8_t> ftype(nform, 0);
-    for (int q = 0; q < Rw; ++q) ftype[1 + 2 * R + q] = 1;
+    for (int q = 0; q < Rw; ++q) ftype[1 + R + Rv + q] = 1;
     std::vector<int32_t> kend(npad / 64, 0);
     for (int i = 0; i < N; ++i) {
         int& ke = kend[i / 64];
         ke = std::max(ke, std::min(npad, (P.mhi[i] + 15) / 16 * 16));
     }
     auto T = std::make_unique<QfTables>();
-    T->npad = npad; T->nform = nform; T->rank = R; T->rank_w = Rw; T->mu = BC.mu; T->mu_w = BS.mu;
+    T->npad = npad; T->nform = nform; T->rank = R; T->rank_v = Rv; T->rank_w = Rw; T->mu = BC.mu; T->mu_w = BS.mu;
     T->basis_err = std::max(BC.err, BS.err);
     // The level pass's first-order and diagonal terms through profile bases
     // over [0, 2 kmax] (the diagonal's profile is that of 2 k_i): by default in
@@ -521,7 +526,7 @@ int Sea::qform_build(QfTables& T, uint16_t* b, uint16_t* beta) {
     if (split) CFDWM_HIP(hipMemsetAsync(beta, 0, T.eta_bytes, st));
     CFDWM_HIP(hipMemsetAsync(b, 0, T.table_bytes, st));
     QfBuild Bq;
-    Bq.n = tab.comp.n; Bq.npad = T.npad; Bq.R = T.rank; Bq.Rw = T.rank_w; Bq.nform = T.nform; Bq.nbarr = T.nbarr;
+    Bq.n = tab.comp.n; Bq.npad = T.npad; Bq.R = T.rank; Bq.Rv = T.rank_v; Bq.Rw = T.rank_w; Bq.nform = T.nform; Bq.nbarr = T.nbarr;
     Bq.h = tab.in.depth;
     Bq.frow = d32_.frow; Bq.fmhi = d32_.fmhi; Bq.uvw = d32_.fuvw; Bq.x = d32_.fx;
     Bq.zs = (const double*)T.zs.get(); Bq.finv = (const double*)T.finv.get();
@@ -1154,7 +1159,7 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
         Q.b = T->bp;
         Q.nbarr = 4; Q.nlv = 3;
         Q.nform = T->nform;
-        Q.ncos = 1 + 2 * R;
+        Q.ncos = 1 + R + T->rank_v;
     } else {                                      // eta2 at three products; velocity forms at one
         Q.b = T->betap;
         Q.nbarr = 4; Q.nlv = 3;
@@ -1165,7 +1170,7 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
         V.nbarr = T->nbarr; V.nlv = 1;
         V.ftype = Q.ftype + 1;
         V.nform = T->nform - 1;
-        V.ncos = 2 * R;
+        V.ncos = R + T->rank_v;
         V.out = Q.out + ppad_all;
     }
     // executed MFMA flops per padded point and form: a 128-wide i tile runs
@@ -1181,6 +1186,7 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
     qf_nlv = T->nlv;
     qf_nform = T->nform;
     qf_rank = R;
+    qf_rank_v = T->rank_v;
     qf_rank_w = T->rank_w;
     qf_basis_err = T->basis_err;
     qf_flop = 0;
@@ -1271,6 +1277,7 @@ void Grid::qform_attach(ColumnJob<float>& C, LevelJob<float>& L) {
     for (int s = 0; s < 4; ++s) C.q2scale[s] = qf_scale_[s];
     L.qf = (const float*)qout_.get() + qj_.ostride;
     L.qf_rank = R;
+    L.qf_rank_v = qf_rank_v;
     L.qf_rank_w = qf_rank_w;
     L.qf_stride = qj_.ostride;
     constexpr double kL2e = 1.4426950408889634074;

@@ -57,8 +57,8 @@ struct LevelJob {
     // u, v += scale * sum_q (e^{mu_q z} + e^{-mu_q (z + 2h)}) Q_{f,q}(column) (cosh-type
     // basis, rank qf_rank), w += scale * sum_q (e^{nu_q z} - e^{-nu_q (z + 2h)}) Q_{w,q}
     // (sinh-type basis, rank qf_rank_w)
-    const float* qf = nullptr;            // [2 qf_rank + qf_rank_w][qf_stride]: u, v, w forms
-    int qf_rank = 0, qf_rank_w = 0;
+    const float* qf = nullptr;            // [qf_rank + qf_rank_v + qf_rank_w][qf_stride]: u, v, w forms
+    int qf_rank = 0, qf_rank_v = 0, qf_rank_w = 0;   // qf_rank_v: qf_rank, or 0 where v has no pair terms
     int64_t qf_stride = 0;
     float qf_mu2[32] = {};                // mu_q log2 e
     float qf_mg[32] = {};                 // -2 h mu_q log2 e
@@ -361,6 +361,7 @@ public:
     // cosh-type profile basis and the w forms (sin-type) of the sinh-type one
     struct QfTables {
         int npad = 0, nform = 0, rank = 0, rank_w = 0;   // ranks of the cosh- and sinh-type profile bases
+        int rank_v = 0;                      // forms of v: rank, or 0 where every v coefficient is zero
         int nlv = 3, nbarr = 4;              // bf16 products per term, table arrays per form
         double basis_err = 0, basis_tol = 0;
         std::vector<double> mu, mu_w;        // skeleton wavenumbers of the two profile bases
@@ -512,7 +513,7 @@ public:
     // explicit switch runs about 14x slower: say so once per grid on stderr
     void warn_pair_loop(const char* why);
     bool qf_warned_ = false;
-    int qf_nform = 0, qf_rank = 0, qf_rank_w = 0, qf_nlv = 3;
+    int qf_nform = 0, qf_rank = 0, qf_rank_v = 0, qf_rank_w = 0, qf_nlv = 3;
     double qf_flop = 0, qf_basis_err = 0;
     // shader clock of the forms launches of later fills (diagnostic)
     void qform_clock_enable(bool on) { qf_clock_on_ = on; }

@@ -376,7 +376,8 @@ __device__ __forceinline__ void lb_levels_out(const LevelJob<float>& J, const Le
         R fu[4] = {0, 0, 0, 0}, fv[4] = {0, 0, 0, 0}, fw[4] = {0, 0, 0, 0};
         for (int q = 0; q < Rk; ++q) {
             const R m2 = (R)J.qf_mu2[q], mg = (R)J.qf_mg[q];
-            const R qu = (R)J.qf[(int64_t)q * J.qf_stride + cq], qv = (R)J.qf[(int64_t)(Rk + q) * J.qf_stride + cq];
+            const R qu = (R)J.qf[(int64_t)q * J.qf_stride + cq];
+            const R qv = J.qf_rank_v ? (R)J.qf[(int64_t)(Rk + q) * J.qf_stride + cq] : (R)0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 R E, G;
@@ -387,7 +388,7 @@ __device__ __forceinline__ void lb_levels_out(const LevelJob<float>& J, const Le
         }
         for (int q = 0; q < Rw; ++q) {
             const R m2 = (R)J.qf_mu2w[q], mg = (R)J.qf_mgw[q];
-            const R qw = (R)J.qf[(int64_t)(2 * J.qf_rank + q) * J.qf_stride + cq];
+            const R qw = (R)J.qf[(int64_t)(J.qf_rank + J.qf_rank_v + q) * J.qf_stride + cq];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 R E, G;
@@ -826,7 +827,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
             const int Rk = J.qf_rank, Rw = J.qf_rank_w;
             for (int q = 0; q < Rk; ++q) {            // cosh-type basis: u, v
                 const R Qu = (R)J.qf[(int64_t)q * J.qf_stride + cq];
-                const R Qv = (R)J.qf[(int64_t)(Rk + q) * J.qf_stride + cq];
+                const R Qv = J.qf_rank_v ? (R)J.qf[(int64_t)(Rk + q) * J.qf_stride + cq] : (R)0;
                 const R m2 = (R)J.qf_mu2[q], mg = (R)J.qf_mg[q];
 #pragma unroll
                 for (int l = 0; l < LC; ++l) {
@@ -837,7 +838,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
                 }
             }
             for (int q = 0; q < Rw; ++q) {            // sinh-type basis: w
-                const R Qw = (R)J.qf[(int64_t)(2 * Rk + q) * J.qf_stride + cq];
+                const R Qw = (R)J.qf[(int64_t)(Rk + J.qf_rank_v + q) * J.qf_stride + cq];
                 const R m2 = (R)J.qf_mu2w[q], mg = (R)J.qf_mgw[q];
 #pragma unroll
                 for (int l = 0; l < LC; ++l) {

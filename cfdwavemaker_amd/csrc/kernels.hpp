@@ -165,7 +165,7 @@ CFDWM_HD inline void qf_pair(int nform, int ncos, int q, int* form, bool* two) {
 // Device build of the form tables from the FP32 pair records (qform.hip).
 struct QfBuild {
     int n = 0, npad = 0, nform = 0;
-    int R = 0, Rw = 0;                    // depth-basis ranks: cosh-type (u, v) and sinh-type (w) profiles
+    int R = 0, Rv = 0, Rw = 0;            // forms of u, v (R or none) and w: depth-basis ranks, cosh- and sinh-type
     double h = 0;                         // sea depth of the profiles e^{kz} +- e^{-k (z + 2h)}
     const int64_t* frow = nullptr;        // filtered table rows
     const int32_t* fmhi = nullptr;

@@ -920,8 +920,10 @@ __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
             if (nf == 2) {                            // u, v (cos-type)
                 put(f0 + q, 0, r.cuP * cp + r.cuM * cm);
                 put(f0 + q, 1, r.cuM * cm - r.cuP * cp);
-                put(f0 + R + q, 0, r.cvP * cp + r.cvM * cm);
-                put(f0 + R + q, 1, r.cvM * cm - r.cvP * cp);
+                if (B.Rv) {
+                    put(f0 + R + q, 0, r.cvP * cp + r.cvM * cm);
+                    put(f0 + R + q, 1, r.cvM * cm - r.cvP * cp);
+                }
             } else {                                  // w (sin-type)
                 put(f0 + q, 0, r.cwP * cp + r.cwM * cm);
                 put(f0 + q, 1, r.cwP * cp - r.cwM * cm);
@@ -929,13 +931,13 @@ __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
         }
     };
     family(B.R, B.zs, B.finv, 1.0, 1, 2);
-    family(B.Rw, B.zsw, B.finvw, -1.0, 1 + 2 * B.R, 1);
+    family(B.Rw, B.zsw, B.finvw, -1.0, 1 + B.R + B.Rv, 1);
 }
 
 }  // namespace
 
 hipError_t launch_qf_build(const QfBuild& B, hipStream_t st) {
-    if (B.n <= 0 || B.R < 0 || B.R > 32 || B.Rw < 0 || B.Rw > 32 || B.nform != 1 + 2 * B.R + B.Rw ||
+    if (B.n <= 0 || B.R < 0 || B.R > 32 || B.Rw < 0 || B.Rw > 32 || (B.Rv && B.Rv != B.R) || B.nform != 1 + B.R + B.Rv + B.Rw ||
         (B.npad & 127) || B.npad < B.n || (B.nbarr != 2 && B.nbarr != 4))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_qf_build, dim3((unsigned)((B.npad + 255) / 256), (unsigned)B.n), dim3(256), 0, st, B);

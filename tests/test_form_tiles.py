@@ -46,3 +46,24 @@ def test_large_launch_equals_small(eng, mode, nfreq, ndir, depth, kw):
             assert not np.any(a)
             continue
         assert scaled_err(a, b) <= 1e-5, (f, scaled_err(a, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp32", "bf16"])
+@pytest.mark.parametrize("n,depth,nl", [(2, 30.0, 4), (130, 30.0, 16), (200, 120.0, 9)])
+def test_seas_along_x_leave_the_v_forms_out(prec, n, depth, nl):
+    """Along x every v coefficient is zero and the v forms are left out: the other
+    fields are the bits of the same sea with directions of 1e-20, whose v forms run."""
+    from cfdwavemaker_amd import engine as eng
+    from cfdwavemaker_amd.seastate import make_sea
+    p = eng.FP32 if prec == "fp32" else eng.BF16
+    s = make_sea(n, 2.0, 8.0, depth, seed=n, ndir=1).as_dict()
+    g = []
+    for th in (0.0, 1e-20):
+        s["theta"] = np.full(len(s["omega"]), th)
+        g.append(eng.Sea(s, precision=p, with_direct=False).grid((0.0, 60.0, 0.0, 45.0), 21, 16, nl, 0.0, 0.5, 0.7, 1.5,
+                                                                 depth))
+    assert g[0].qform_info()["nform"] < g[1].qform_info()["nform"]
+    for f in ("ETA", "UX", "UZ"):
+        assert np.array_equal(g[0].export(f), g[1].export(f)), f
+    assert not np.any(g[0].export("UY"))
