@@ -1433,7 +1433,6 @@ int Grid::batch_end() {
     batch_pending_ = false;
     if (rc) return rc;
     if ((rc = gradients<float>())) return rc;
-    if ((rc = pack<float>())) return rc;
     filled = true;
     return 0;
 }
@@ -1733,36 +1732,20 @@ int refill_batched(Grid** grids, int n, int64_t budget_bytes, bool release, Batc
 
 template <typename R>
 int Grid::gradients() {
-    hipStream_t st = Engine::get().stream();
-    const int tid0 = (tstep + 1) % 4, tid1 = (tstep + 2) % 4;
-    const int64_t c = (int64_t)g.nx * g.ny, v = c * g.nl;
-    auto P = [&](int f) { return (R*)f_[f].get(); };
-    PROF("k_grad_xyz", launch_grad_xyz<R>(P(0), P(1), P(2), (R*)nullptr, g.nx, g.ny, 1, tid0, tid1, g.dx, g.dy, g.ds, st));
-    PROF("k_grad_dt", launch_grad_dt<R>(P(0), P(3), c, tstep, d.dt, st));
-    for (int f = 0; f < 3; ++f) {
-        PROF("k_grad_xyz", launch_grad_xyz<R>(P(4 + f), P(10 + 3 * f), P(11 + 3 * f), P(12 + 3 * f), g.nx, g.ny, g.nl,
-                                              tid0, tid1, g.dx, g.dy, g.ds, st));
-        PROF("k_grad_dt", launch_grad_dt<R>(P(4 + f), P(7 + f), v, tstep, d.dt, st));
-    }
-    return 0;
-}
-
-template <typename R>
-int Grid::pack() {
     const size_t esz = sizeof(R);
     const int64_t c = (int64_t)g.nx * g.ny, v = c * g.nl;
     if (pk_eta_.alloc(8 * c * esz) || pk_C_.alloc(16 * v * esz) || pk_D_.alloc(16 * v * esz)) return -3;
-    PackJob<R> J;
-    J.nx = g.nx; J.ny = g.ny; J.nl = g.nl;
-    J.tid1 = (tstep + 1) % 4; J.tid2 = (tstep + 2) % 4;
-    auto P = [&](int f) { return (const R*)f_[f].get(); };
+    GradPack<R> J;
+    J.nx = g.nx; J.ny = g.ny; J.nl = g.nl; J.tstep = tstep;
+    J.dx = g.dx; J.dy = g.dy; J.ds = g.ds; J.dt = d.dt;
+    auto P = [&](int f) { return (R*)f_[f].get(); };
     J.E = P(0); J.Ex = P(1); J.Ey = P(2); J.Et = P(3);
     for (int f = 0; f < 3; ++f) {
         J.F[f] = P(4 + f); J.Ft[f] = P(7 + f);
         J.Fx[f] = P(10 + 3 * f); J.Fy[f] = P(11 + 3 * f); J.Fs[f] = P(12 + 3 * f);
     }
     J.pk_eta = (R*)pk_eta_.get(); J.pk_C = (R*)pk_C_.get(); J.pk_D = (R*)pk_D_.get();
-    PROF("k_pack", launch_pack<R>(J, Engine::get().stream()));
+    PROF("k_grad_pack", launch_grad_pack<R>(J, Engine::get().stream()));
     return 0;
 }
 
@@ -1779,8 +1762,6 @@ int Grid::refill() {
                            : fill_slots<double>(4, ign ? tb : ta, dst, ign);
     if (rc) return rc;
     rc = prec == kFP32 ? gradients<float>() : gradients<double>();
-    if (rc) return rc;
-    rc = prec == kFP32 ? pack<float>() : pack<double>();
     if (rc) return rc;
     CFDWM_HIP(hipStreamSynchronize(Engine::get().stream()));
     filled = true;
@@ -1799,8 +1780,6 @@ int Grid::force_update(double t, int* n) {
         int rc = prec == kFP32 ? fill_slots<float>(1, &t2, &slot, true) : fill_slots<double>(1, &t2, &slot, true);
         if (rc) return rc;
         rc = prec == kFP32 ? gradients<float>() : gradients<double>();
-        if (rc) return rc;
-        rc = prec == kFP32 ? pack<float>() : pack<double>();
         if (rc) return rc;
         ++k;
         if (vtk.on) {                             // update (lsgrid_spline.cpp:924-926)

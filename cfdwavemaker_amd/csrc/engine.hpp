@@ -85,11 +85,15 @@ struct LevelJob {
     double* partial = nullptr;            // nseg > 1: [seg][thread][3 LC + 6] partial sums
 };
 
+// Derivatives and packed records after a fill or an update (k_grad_pack):
+// fields of four time slots, their x, y, s derivatives of the two a query
+// reads, d/dt by time slot.
 template <typename R>
-struct PackJob {
-    int nx, ny, nl, tid1, tid2;
-    const R *E, *Et, *Ex, *Ey;
-    const R *F[3], *Ft[3], *Fx[3], *Fy[3], *Fs[3];
+struct GradPack {
+    int nx, ny, nl, tstep;
+    double dx, dy, ds, dt;
+    const R *E, *F[3];
+    R *Et, *Ex, *Ey, *Ft[3], *Fx[3], *Fy[3], *Fs[3];
     R *pk_eta, *pk_C, *pk_D;
 };
 
@@ -163,14 +167,9 @@ hipError_t launch_smit(const SmitJob& J, hipStream_t st);
 int64_t column_threads(int64_t nslot, int64_t ncol);
 int64_t level_threads(int64_t nslot, int64_t ncol, int nl, int lc, bool grid);
 template <typename R>
-hipError_t launch_grad_xyz(const R* D, R* GX, R* GY, R* GS, int nx, int ny, int L, int tid0, int tid1,
-                           double dx, double dy, double ds, hipStream_t st);
-template <typename R>
-hipError_t launch_grad_dt(const R* D, R* GD, int64_t per, int tstep, double dt, hipStream_t st);
+hipError_t launch_grad_pack(const GradPack<R>& J, hipStream_t st);
 template <typename R, typename TQ>
 hipError_t launch_query(const QueryJob<R, TQ>& J, hipStream_t st);
-template <typename R>
-hipError_t launch_pack(const PackJob<R>& J, hipStream_t st);
 // Cell order of a query batch (qsort.hip): recs receives (x, y, z, p) of every
 // query p, grouped by tiles of neighbouring columns; counts holds
 // query_bins_bytes bytes of scratch.
@@ -584,8 +583,6 @@ private:
     DevBuf q_in_, q_out_;
     DevBuf pk_eta_, pk_C_, pk_D_;             // query records of the two active slots
     DevBuf qs_cnt_, qs_rec_;                  // cell-ordered query batches
-    template <typename R>
-    int pack();
     template <typename R>
     int fill_slots(int nslot, const double* slot_t, const int* slot_dst, bool use_ignore);
     template <typename R>

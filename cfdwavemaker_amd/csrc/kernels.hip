@@ -978,107 +978,85 @@ __global__ __launch_bounds__(256) void k_levels_reduce(SeaDev<R> S, LevelJob<R> 
     lev_store<R, LC, GRID, WP>(S, J, fl, PP, a);
 }
 
-// ======================================================== FD gradient kernels
-// update_gradient_eta_dxdy / update_gradient_dxdydz (lsgrid_spline.cpp:163-366):
-// central differences inside, one-sided at the edges, zero for a single point.
-// Output slot o (0, 1) holds ring slot tids[o].
-template <typename R>
-__global__ __launch_bounds__(256) void k_grad_xyz(const R* __restrict__ D, R* __restrict__ GX,
-                                                  R* __restrict__ GY, R* __restrict__ GS,
-                                                  int nx, int ny, int L, int tid0, int tid1,
-                                                  double dx, double dy, double ds) {
-    const int64_t per = (int64_t)nx * ny * L;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= 2 * per) return;
-    const int o = (int)(e / per);
-    const int64_t qq = e % per;
-    const int m = (int)(qq % L);
-    const int j = (int)((qq / L) % ny);
-    const int i = (int)(qq / ((int64_t)L * ny));
-    const R* d = D + (int64_t)(o ? tid1 : tid0) * per;
-    const int64_t sx = (int64_t)ny * L, sy = L;
-    R vx, vy;
-    if (nx == 1) vx = 0;
-    else if (i == 0) vx = (R)((d[qq + sx] - d[qq]) / dx);
-    else if (i == nx - 1) vx = (R)((d[qq] - d[qq - sx]) / dx);
-    else vx = (R)((d[qq + sx] - d[qq - sx]) / (2 * dx));
-    if (ny == 1) vy = 0;
-    else if (j == 0) vy = (R)((d[qq + sy] - d[qq]) / dy);
-    else if (j == ny - 1) vy = (R)((d[qq] - d[qq - sy]) / dy);
-    else vy = (R)((d[qq + sy] - d[qq - sy]) / (2 * dy));
-    GX[o * per + qq] = vx;
-    GY[o * per + qq] = vy;
-    if (GS) {
-        R vs;
-        if (L == 1) vs = 0;
-        else if (m == 0) vs = (R)((d[qq + 1] - d[qq]) / ds);
-        else if (m == L - 1) vs = (R)((d[qq] - d[qq - 1]) / ds);
-        else vs = (R)((d[qq + 1] - d[qq - 1]) / (2 * ds));
-        GS[o * per + qq] = vs;
-    }
-}
-
-// update_gradient_dt / update_gradient_eta_dt (lsgrid_spline.cpp:124-161)
-template <typename R>
-__global__ __launch_bounds__(256) void k_grad_dt(const R* __restrict__ D, R* __restrict__ GD,
-                                                 int64_t per, int tstep, double dt) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per) return;
-    if (tstep > 0) {
-        const int tid = (tstep + 2) % 4, t1 = (tstep + 3) % 4, t0 = (tstep + 1) % 4;
-        GD[tid * per + e] = (R)((D[t1 * per + e] - D[t0 * per + e]) / (2 * dt));
-    } else {
-        GD[1 * per + e] = (R)((D[2 * per + e] - D[1 * per + e]) / dt);
-        GD[2 * per + e] = (R)((D[3 * per + e] - D[1 * per + e]) / (2 * dt));
-    }
-}
-
 // ================================================================ spline query
 // The two time slots a query reads, (tstep+1)%4 and (tstep+2)%4, are packed
-// after every fill/update by k_pack:
+// after every fill/update by k_grad_pack:
 //   column record (8 R): eta(tid1) eta(tid2) eta_t(tid1) eta_t(tid2) eta_x(0) eta_x(1) eta_y(0) eta_y(1)
 //   node records C and D (16 R each): for u, v, w in turn the piece f, f_x, f_y, f_s,
 //     then the piece u_t, v_t, w_t, pad;
 //     C from time slot tid1 and derivative slot 0, D from tid2 and derivative slot 1.
 // Levels are the fastest index, so the corners l and l+1 of a query share a
 // cache line and one query touches 8 node lines instead of 8 x 30 arrays.
+
+// central difference inside, one-sided at the ends, zero for a single point
+// (update_gradient_dxdydz, lsgrid_spline.cpp:163-366)
 template <typename R>
-__global__ __launch_bounds__(256) void k_pack(PackJob<R> J) {
-    const int64_t per = (int64_t)J.nx * J.ny * J.nl;
-    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ R fd(const R* d, int64_t st, int64_t i, int64_t n, double dx) {
+    if (n == 1) return (R)0;
+    if (i == 0) return (R)((d[st] - d[0]) / dx);
+    if (i == n - 1) return (R)((d[0] - d[-st]) / dx);
+    return (R)((d[st] - d[-st]) / (2 * dx));
+}
+
+// After a fill or an update: the derivatives of the two time slots a query
+// reads (update_gradient_eta_dxdy, _dxdydz, _dt, lsgrid_spline.cpp:124-366),
+// to the field arrays, and the packed records from the same registers.  A
+// thread takes a node; the column's record goes with its lowest level.  Bound
+// by its stores (18 to 24 derivatives and 32 record values a node).  One
+// launch where four derivative pairs and the packing took nine, with the
+// fields and derivatives read back each time: 256 x 256 x 16 FP32 nodes 138 ->
+// 91 us.
+template <typename R, typename I>
+__global__ __launch_bounds__(256) void k_grad_pack(GradPack<R> J) {
+    const I per = (I)J.nx * (I)J.ny * (I)J.nl, n = (I)blockIdx.x * 256 + threadIdx.x;
     if (n >= per) return;
-    // records are assembled in registers and stored as 16-byte vectors (the
-    // packed arrays are 256-byte aligned allocations, records 16 R long)
+    const I col = n / (I)J.nl;
+    const I m = n - col * (I)J.nl, i = col / (I)J.ny, j = col - i * (I)J.ny;
+    const int s0 = (J.tstep + 1) % 4, s1 = (J.tstep + 2) % 4, s2 = (J.tstep + 3) % 4;
+    // d/dt of the second slot; the first has its own from the step before,
+    // or, after a fill, its forward difference
+    auto dt = [&](const R* D, R* T, I w, I e, R& t0, R& t1) {
+        if (J.tstep > 0) {
+            t0 = T[s0 * w + e];
+            t1 = (R)((D[s2 * w + e] - D[s0 * w + e]) / (2 * J.dt));
+        } else {
+            t0 = (R)((D[2 * w + e] - D[1 * w + e]) / J.dt);
+            t1 = (R)((D[3 * w + e] - D[1 * w + e]) / (2 * J.dt));
+            T[s0 * w + e] = t0;
+        }
+        T[s1 * w + e] = t1;
+    };
+    const I sx = (I)J.ny * (I)J.nl, sy = (I)J.nl;
     R c[16], d[16];
 #pragma unroll
     for (int f = 0; f < 3; ++f) {
-        c[4 * f + 0] = J.F[f][J.tid1 * per + n];
-        c[4 * f + 1] = J.Fx[f][n];
-        c[4 * f + 2] = J.Fy[f][n];
-        c[4 * f + 3] = J.Fs[f][n];
-        c[12 + f] = J.Ft[f][J.tid1 * per + n];
-        d[4 * f + 0] = J.F[f][J.tid2 * per + n];
-        d[4 * f + 1] = J.Fx[f][per + n];
-        d[4 * f + 2] = J.Fy[f][per + n];
-        d[4 * f + 3] = J.Fs[f][per + n];
-        d[12 + f] = J.Ft[f][J.tid2 * per + n];
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            const R* F = J.F[f] + (o ? s1 : s0) * per + n;
+            R* r = o ? d : c;
+            r[4 * f] = *F;
+            J.Fx[f][o * per + n] = r[4 * f + 1] = fd(F, (int64_t)sx, (int64_t)i, (int64_t)J.nx, J.dx);
+            J.Fy[f][o * per + n] = r[4 * f + 2] = fd(F, (int64_t)sy, (int64_t)j, (int64_t)J.ny, J.dy);
+            J.Fs[f][o * per + n] = r[4 * f + 3] = fd(F, (int64_t)1, (int64_t)m, (int64_t)J.nl, J.ds);
+        }
+        dt(J.F[f], J.Ft[f], per, n, c[12 + f], d[12 + f]);
     }
     c[15] = 0;
     d[15] = 0;
-    store_rec<16>(J.pk_C + 16 * n, c);
-    store_rec<16>(J.pk_D + 16 * n, d);
-    if (n % J.nl == 0) {
-        const int64_t pc = (int64_t)J.nx * J.ny, col = n / J.nl;
+    store_rec<16>(J.pk_C + 16 * (int64_t)n, c);
+    store_rec<16>(J.pk_D + 16 * (int64_t)n, d);
+    if (m == 0) {
+        const I pc = (I)J.nx * (I)J.ny;
         R e[8];
-        e[0] = J.E[J.tid1 * pc + col];
-        e[1] = J.E[J.tid2 * pc + col];
-        e[2] = J.Et[J.tid1 * pc + col];
-        e[3] = J.Et[J.tid2 * pc + col];
-        e[4] = J.Ex[col];
-        e[5] = J.Ex[pc + col];
-        e[6] = J.Ey[col];
-        e[7] = J.Ey[pc + col];
-        store_rec<8>(J.pk_eta + 8 * col, e);
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            const R* E = J.E + (o ? s1 : s0) * pc + col;
+            e[o] = *E;
+            J.Ex[o * pc + col] = e[4 + o] = fd(E, (int64_t)J.ny, (int64_t)i, (int64_t)J.nx, J.dx);
+            J.Ey[o * pc + col] = e[6 + o] = fd(E, (int64_t)1, (int64_t)j, (int64_t)J.ny, J.dy);
+        }
+        dt(J.E, J.Et, pc, col, e[2], e[3]);
+        store_rec<8>(J.pk_eta + 8 * (int64_t)col, e);
     }
 }
 
@@ -1544,28 +1522,16 @@ hipError_t launch_levels(const SeaDev<R>& S, const LevelJob<R>& J, bool grid, in
 }
 
 template <typename R>
-hipError_t launch_grad_xyz(const R* D, R* GX, R* GY, R* GS, int nx, int ny, int L, int tid0, int tid1,
-                           double dx, double dy, double ds, hipStream_t st) {
-    const int64_t n = 2LL * nx * ny * L;
-    hipLaunchKernelGGL((k_grad_xyz<R>), dim3(nblk(n)), dim3(256), 0, st, D, GX, GY, GS, nx, ny, L,
-                       tid0, tid1, dx, dy, ds);
-    return hipGetLastError();
-}
-
-template <typename R>
-hipError_t launch_grad_dt(const R* D, R* GD, int64_t per, int tstep, double dt, hipStream_t st) {
-    hipLaunchKernelGGL((k_grad_dt<R>), dim3(nblk(per)), dim3(256), 0, st, D, GD, per, tstep, dt);
-    return hipGetLastError();
-}
-
-template <typename R>
-hipError_t launch_pack(const PackJob<R>& J, hipStream_t st) {
+hipError_t launch_grad_pack(const GradPack<R>& J, hipStream_t st) {
     const int64_t n = (int64_t)J.nx * J.ny * J.nl;
-    hipLaunchKernelGGL((k_pack<R>), dim3(nblk(n)), dim3(256), 0, st, J);
+    if (4 * n <= (int64_t)UINT32_MAX)
+        hipLaunchKernelGGL((k_grad_pack<R, uint32_t>), dim3(nblk(n)), dim3(256), 0, st, J);
+    else
+        hipLaunchKernelGGL((k_grad_pack<R, uint64_t>), dim3(nblk(n)), dim3(256), 0, st, J);
     return hipGetLastError();
 }
-template hipError_t launch_pack<double>(const PackJob<double>&, hipStream_t);
-template hipError_t launch_pack<float>(const PackJob<float>&, hipStream_t);
+template hipError_t launch_grad_pack<double>(const GradPack<double>&, hipStream_t);
+template hipError_t launch_grad_pack<float>(const GradPack<float>&, hipStream_t);
 
 hipError_t launch_points_finish(const PointsFinish& F, hipStream_t st) {
     if (F.n <= 0) return hipSuccess;
@@ -1618,10 +1584,6 @@ template hipError_t launch_columns<double>(const SeaDev<double>&, const ColumnJo
 template hipError_t launch_columns<float>(const SeaDev<float>&, const ColumnJob<float>&, bool, hipStream_t);
 template hipError_t launch_levels<double>(const SeaDev<double>&, const LevelJob<double>&, bool, int, hipStream_t);
 template hipError_t launch_levels<float>(const SeaDev<float>&, const LevelJob<float>&, bool, int, hipStream_t);
-template hipError_t launch_grad_xyz<double>(const double*, double*, double*, double*, int, int, int, int, int, double, double, double, hipStream_t);
-template hipError_t launch_grad_xyz<float>(const float*, float*, float*, float*, int, int, int, int, int, double, double, double, hipStream_t);
-template hipError_t launch_grad_dt<double>(const double*, double*, int64_t, int, double, hipStream_t);
-template hipError_t launch_grad_dt<float>(const float*, float*, int64_t, int, double, hipStream_t);
 template hipError_t launch_query<double, double>(const QueryJob<double, double>&, hipStream_t);
 template hipError_t launch_query<float, double>(const QueryJob<float, double>&, hipStream_t);
 template hipError_t launch_query<double, float>(const QueryJob<double, float>&, hipStream_t);
