@@ -59,31 +59,59 @@ __device__ __forceinline__ float gelu_d(float x) {
     return 0.5f * (1.f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
 }
 
-// epilogue of a 32 x 32 accumulator tile (rows m0.., column cn of this lane)
-__device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, int m0, int cn, int hl) {
+// Epilogue of a block's 64 x 64 tile through LDS (64 x 68 floats, the block's
+// threads past a barrier): a thread takes four consecutive columns of a row,
+// four times in a rolled loop.  Straight from the accumulators the 16 unrolled
+// copies of erf and exp ran from cold instruction memory and the stores were
+// single floats (4096 x 256 x 256: 15.2 -> 11.4 us with bias and gelu, 18.2 ->
+// 12.9 with gelu', the longer k steps of mm_tile included).
+constexpr int kMmT = 68;
+__device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, float* T, int m0, int n0) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int m = m0 + 8 * (r >> 2) + 4 * hl + (r & 3);
-        if (m >= a.M || cn >= a.N) continue;
-        float v = acc[r];
-        const int64_t o = (int64_t)m * a.scm + cn;
-        if (a.epi == 1) {
-            v += a.bias[cn];
-            a.Z[o] = v;
-            a.C[o] = gelu(v);
-        } else if (a.epi == 2) {
-            a.C[o] = v + a.bias[cn];
-        } else if (a.epi == 3) {
-            a.C[o] = v * gelu_d(a.Z[o]);
+    for (int r = 0; r < 16; ++r)
+        T[((w & 1) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kMmT + (w >> 1) * 32 + (lane & 31)] = acc[r];
+    __syncthreads();
+    const int c0 = (t & 15) * 4;
+    const bool hasb = a.epi == 1 || a.epi == 2;
+    float bias[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bias[k] = hasb ? a.bias[min(n0 + c0 + k, a.N - 1)] : 0.f;
+    const bool v4 = n0 + 64 <= a.N && (a.scm & 3) == 0 && (a.cz & 3) == 0 &&
+                    ((reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.Z)) & 15) == 0;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
+        const int r = j * 16 + (t >> 4), m = m0 + r;
+        if (m >= a.M) break;
+        const int64_t o = (int64_t)m * a.scm + n0 + c0;
+        const float4 q = *reinterpret_cast<const float4*>(T + r * kMmT + c0);
+        float v[4] = {q.x + bias[0], q.y + bias[1], q.z + bias[2], q.w + bias[3]};
+        if (v4) {
+            float4 z = make_float4(v[0], v[1], v[2], v[3]);
+            if (a.epi == 1) *reinterpret_cast<float4*>(a.Z + o) = z;
+            if (a.epi == 3) z = *reinterpret_cast<const float4*>(a.Z + o);
+            const float zz[4] = {z.x, z.y, z.z, z.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (a.epi == 1) v[k] = gelu(v[k]);
+                if (a.epi == 3) v[k] *= gelu_d(zz[k]);
+            }
+            *reinterpret_cast<float4*>(a.C + o) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
-            a.C[o] = v;
+#pragma unroll 1
+            for (int k = 0; k < 4; ++k) {
+                if (n0 + c0 + k >= a.N) break;
+                const float x = k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+                if (a.epi == 1) a.Z[o + k] = x;
+                a.C[o + k] = a.epi == 1 ? gelu(x) : a.epi == 3 ? x * gelu_d(a.Z[o + k]) : x;
+            }
         }
     }
 }
 
 // Block 256 threads = 4 waves, 64 x 64 outputs; wave (w & 1, w >> 1) takes a
 // 32 x 32 tile (one v_mfma_f32_32x32x16_bf16 accumulator).  Operands are
-// staged through LDS 32 values of k at a time, rounded to bf16 on the way:
+// staged through LDS 64 values of k at a time, rounded to bf16 on the way:
 // [row][k], so that a lane's operand (row l % 32, 8 values of k) is one
 // 16-byte LDS read.  AK, BK: the operand is contiguous in k in memory (a
 // thread stages 8 values of k of one row, two 16-byte loads where the rows
@@ -101,14 +129,17 @@ __device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, int
 // Before, the gradient products read strided scalars per lane (22 us each,
 // 207 us for the 33-wide input) and one thread summed a whole column (851 us
 // for 4096 rows, four times): 4.0 ms per loss and gradient of 4096 rows of the
-// 33-256-256-256-65 network, 0.25 ms now (products 11 to 18 us each).
+// 33-256-256-256-65 network, 0.21 ms now (products 11 to 13 us each).
 template <bool AK, bool BK>
-__global__ __launch_bounds__(256) void k_mm(MmArgs a) {
-    constexpr int LS = 40;                        // LDS row stride in bf16 (80 bytes: no bank conflicts at 16 bytes)
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][64 * LS], Bs[2][64 * LS];
+__device__ __forceinline__ void mm_tile(const MmArgs& a, int bx, int by, int bz) {
+    constexpr int KS = 64, LS = KS + 8;                        // LDS row stride in bf16 (80 bytes: no bank conflicts at 16 bytes)
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][64 * LS];
+    uint16_t(*As)[64 * LS] = lds[0], (*Bs)[64 * LS] = lds[1];
+    float* T = reinterpret_cast<float*>(lds);     // 64 x 68 floats in the end
+    static_assert(sizeof(lds) >= 64 * kMmT * sizeof(float), "the output tile takes the operands' place");
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int kb = (int)blockIdx.z * a.kchunk, ke = min(a.K, kb + a.kchunk);
+    const int m0 = by * 64, n0 = bx * 64;
+    const int kb = bz * a.kchunk, ke = min(a.K, kb + a.kchunk);
     // one operand's 8 values of this thread: row (m or n) r0 + r, k0 + 8 q ..
     const int ra = AK ? t >> 2 : lane, qa = AK ? t & 3 : w;
     const int rb = BK ? t >> 2 : lane, qb = BK ? t & 3 : w;
@@ -138,18 +169,24 @@ __global__ __launch_bounds__(256) void k_mm(MmArgs a) {
         *reinterpret_cast<uint4*>(L + r * LS + q * 8) = o;
     };
     float cs = 0.f;
-    const bool sums = a.colsum && blockIdx.x == 0;
-    float fa[8], fb[8];
+    const bool sums = a.colsum && bx == 0;
+    float fa[KS / 32][8], fb[KS / 32][8];
     auto fetch2 = [&](int k0) {
-        fetch(a.A, a.sam, a.sak, m0 + ra, a.M, k0 + 8 * qa, AK, av4, fa);
-        fetch(a.B, a.sbn, a.sbk, n0 + rb, a.N, k0 + 8 * qb, BK, bv4, fb);
+#pragma unroll
+        for (int s = 0; s < KS / 32; ++s) {
+            fetch(a.A, a.sam, a.sak, m0 + ra, a.M, k0 + 32 * s + 8 * qa, AK, av4, fa[s]);
+            fetch(a.B, a.sbn, a.sbk, n0 + rb, a.N, k0 + 32 * s + 8 * qb, BK, bv4, fb[s]);
+        }
     };
     auto stash2 = [&](int b) {
-        stash(As[b], ra, qa, fa);
-        stash(Bs[b], rb, qb, fb);
-        if (!AK && sums) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) cs += fa[j];
+        for (int s = 0; s < KS / 32; ++s) {
+            stash(As[b], ra, 4 * s + qa, fa[s]);
+            stash(Bs[b], rb, 4 * s + qb, fb[s]);
+            if (!AK && sums) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) cs += fa[s][j];
+            }
         }
     };
     f32x16 acc;
@@ -161,29 +198,53 @@ __global__ __launch_bounds__(256) void k_mm(MmArgs a) {
     const int oa = ((w & 1) * 32 + (lane & 31)) * LS + (lane >> 5) * 8;
     const int ob = ((w >> 1) * 32 + (lane & 31)) * LS + (lane >> 5) * 8;
     int b = 0;
-    for (int k0 = kb; k0 < ke; k0 += 32) {        // block-uniform
-        if (k0 + 32 < ke) fetch2(k0 + 32);
+    for (int k0 = kb; k0 < ke; k0 += KS) {        // block-uniform
+        if (k0 + KS < ke) fetch2(k0 + KS);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < KS / 16; ++h) {
             const bf16x8 A8 = *reinterpret_cast<const bf16x8*>(As[b] + oa + 16 * h);
             const bf16x8 B8 = *reinterpret_cast<const bf16x8*>(Bs[b] + ob + 16 * h);
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A8, B8, acc, 0, 0, 0);
         }
-        if (k0 + 32 < ke) stash2(b ^ 1);          // its readers passed the last barrier
+        if (k0 + KS < ke) stash2(b ^ 1);          // its readers passed the last barrier
         __syncthreads();
         b ^= 1;
     }
     MmArgs o = a;
-    o.C = a.C + (int64_t)blockIdx.z * a.cz;
-    mm_store(o, acc, m0 + (w & 1) * 32, n0 + (w >> 1) * 32 + (lane & 31), lane >> 5);
+    o.C = a.C + (int64_t)bz * a.cz;
+    __syncthreads();                              // the operands have been read
+    mm_store(o, acc, T, m0, n0);
     if (!AK && sums) {                            // block-uniform: the four threads of a column, in order
-        float* red = reinterpret_cast<float*>(As[0]);
+        float* red = T;
+        __syncthreads();
         red[t] = cs;
         __syncthreads();
         if (w == 0 && m0 + lane < a.M)
-            a.colsum[(int64_t)blockIdx.z * a.cz + m0 + lane] =
+            a.colsum[(int64_t)bz * a.cz + m0 + lane] =
                 ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
     }
+}
+
+template <bool AK, bool BK>
+__global__ __launch_bounds__(256) void k_mm(MmArgs a) {
+    mm_tile<AK, BK>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// The weight gradients of up to kMmBatch layers in one launch: block x is an
+// output tile of the layer whose range holds it.  One after the other they
+// cost 11 us each; all four of the network above 20.
+constexpr int kMmBatch = 8;
+struct MmBatch {
+    int n;
+    int tile0[kMmBatch + 1];
+    MmArgs g[kMmBatch];
+};
+__global__ __launch_bounds__(256) void k_mm_grads(MmBatch b) {
+    int l = 0;
+    while (l + 1 < b.n && (int)blockIdx.x >= b.tile0[l + 1]) ++l;      // block-uniform
+    const MmArgs& a = b.g[l];
+    const int q = (int)blockIdx.x - b.tile0[l], nx = (a.N + 63) / 64;
+    mm_tile<false, false>(a, q % nx, q / nx, blockIdx.z);
 }
 
 // g[i] = sum over the chunks z, in order, of part[z np + i]
@@ -369,7 +430,9 @@ __global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict
 
 inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-constexpr int kGradChunks = 32;           // row chunks of a weight gradient, at most
+// Row chunks of a weight gradient, at most: 4096 rows in 32 cost 22 us and 11 for
+// the chunks' sum, in 16 20 and 6.
+constexpr int kGradChunks = 16;
 
 }  // namespace
 
@@ -415,9 +478,7 @@ int Mlp::reserve(int64_t rows) {
     for (int l = 0; l < layers(); ++l) tot += cap * (din[l] + dout[l]);
     tot += cap * nout;
     if (act.alloc((size_t)tot * sizeof(float))) return -3;
-    int64_t wmax = 0;
-    for (int l = 0; l < layers(); ++l) wmax = std::max<int64_t>(wmax, std::max(din[l], dout[l]));
-    if (tmp.alloc((size_t)cap * wmax * 2 * sizeof(float))) return -3;
+    if (tmp.alloc((size_t)cap * nout * 2 * sizeof(float))) return -3;     // dY and the targets
     if (part.alloc((size_t)(nb256(cap * nout) + 1) * sizeof(float))) return -3;
     if (idx.alloc((size_t)cap * sizeof(int64_t))) return -3;
     return 0;
@@ -430,7 +491,6 @@ static hipError_t mm(MmArgs a, hipStream_t st) {
     const dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), (unsigned)((a.K + a.kchunk - 1) / a.kchunk));
     if (a.ak && a.bk) hipLaunchKernelGGL((k_mm<true, true>), grid, dim3(256), 0, st, a);
     else if (a.ak) hipLaunchKernelGGL((k_mm<true, false>), grid, dim3(256), 0, st, a);
-    else if (!a.bk) hipLaunchKernelGGL((k_mm<false, false>), grid, dim3(256), 0, st, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -458,17 +518,9 @@ int Mlp::forward(int64_t n, hipStream_t st) {
     return 0;
 }
 
-// dY must sit at the start of tmp (the first of its two halves); dZ and dH
-// alternate between the halves.
+// dY sits in tmp; dZ_l takes the place of Z_l.
 int Mlp::backward(int64_t n, const float* dY, hipStream_t st) {
     float* A = (float*)act.get();
-    int64_t wmax = 0;
-    for (int l = 0; l < layers(); ++l) wmax = std::max<int64_t>(wmax, std::max(din[l], dout[l]));
-    float* bufA = (float*)tmp.get();
-    float* bufB = bufA + cap * wmax;
-    if (dY != bufA) return -1;
-    float* dZ = bufA;
-    float* dH = bufB;
     // weight gradients sum over the rows: split into at most kGradChunks chunks
     // of 128 rows or more, so that a minibatch's few 64 x 64 output tiles
     // fill the chip; the chunks' gradients (parameter layout) meet at the end
@@ -478,27 +530,33 @@ int Mlp::backward(int64_t n, const float* dY, hipStream_t st) {
     const int nz = (int)((n + chunk - 1) / chunk);
     if (gpart.alloc((size_t)nz * np * sizeof(float))) return -3;
     float* GP = (float*)gpart.get();
-    for (int l = layers() - 1; l >= 0; --l) {
-        // dW_l = dZ^T H_l : (dout x n) . (n x din), db_l = column sums of dZ
-        MmArgs g{};
-        g.M = dout[l]; g.N = din[l]; g.K = (int)n;
-        g.A = dZ; g.sam = 1; g.sak = dout[l];
-        g.B = A + hoff(l); g.sbk = din[l]; g.sbn = 1;
-        g.C = GP + woff[l]; g.scm = din[l]; g.epi = 0;
-        g.kchunk = chunk; g.cz = np; g.colsum = GP + boff[l];
-        CFDWM_HIP(mm(g, st));
-        if (l == 0) break;
-        // dZ_{l-1} = (dZ W_l) * gelu'(Z_{l-1}) : (n x dout) . (dout x din)
-        dH = dZ == bufA ? bufB : bufA;
+    auto dZ = [&](int l) { return l + 1 < layers() ? (const float*)(A + zoff(l)) : dY; };
+    // dZ_{l-1} = (dZ_l W_l) * gelu'(Z_{l-1}) : (n x dout) . (dout x din)
+    for (int l = layers() - 1; l > 0; --l) {
         MmArgs h{};
         h.M = (int)n; h.N = din[l]; h.K = dout[l];
-        h.A = dZ; h.sam = dout[l]; h.sak = 1;
+        h.A = dZ(l); h.sam = dout[l]; h.sak = 1;
         h.B = P() + woff[l]; h.sbk = din[l]; h.sbn = 1;
-        h.C = dH; h.scm = din[l]; h.epi = 3;
-        h.Z = A + zoff(l - 1);
+        h.C = h.Z = A + zoff(l - 1); h.scm = din[l]; h.epi = 3;
         h.ak = true;
         CFDWM_HIP(mm(h, st));
-        dZ = dH;
+    }
+    // dW_l = dZ_l^T H_l : (dout x n) . (n x din), db_l = column sums of dZ_l
+    for (int l0 = 0; l0 < layers(); l0 += kMmBatch) {
+        MmBatch b{};
+        b.n = std::min(kMmBatch, layers() - l0);
+        for (int q = 0; q < b.n; ++q) {
+            const int l = l0 + q;
+            MmArgs& g = b.g[q];
+            g.M = dout[l]; g.N = din[l]; g.K = (int)n;
+            g.A = dZ(l); g.sam = 1; g.sak = dout[l];
+            g.B = A + hoff(l); g.sbk = din[l]; g.sbn = 1;
+            g.C = GP + woff[l]; g.scm = din[l]; g.epi = 0;
+            g.kchunk = chunk; g.cz = np; g.colsum = GP + boff[l];
+            b.tile0[q + 1] = b.tile0[q] + (g.M + 63) / 64 * ((g.N + 63) / 64);
+        }
+        hipLaunchKernelGGL(k_mm_grads, dim3((unsigned)b.tile0[b.n], 1, (unsigned)nz), dim3(256), 0, st, b);
+        CFDWM_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(k_sum_chunks, dim3(nb256(np)), dim3(256), 0, st, np, nz, (const float*)GP, G());
     CFDWM_HIP(hipGetLastError());

@@ -149,3 +149,30 @@ def test_gradient_at_tile_and_chunk_edges(nin, width, nh, nout, n):
             a, b = g[q:q + sz], gr[q:q + sz]
             assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), (d, o, sz)
             q += sz
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh", [7, 8, 16])
+def test_gradient_of_many_layers(nh):
+    """More layers than one launch of weight gradients takes (8).  Tolerance: an
+    operand whose rounding to bf16 flips moves a block by 2^-9 / sqrt(16) at most
+    (few do: 1e3 elements a layer, a flip in 2e4 of them)."""
+    import torch
+    from cfdwavemaker_amd.mlp import Mlp
+    dims, p = _net(9, 16, nh, 4, 18)
+    X, Y, norm = _data(70, 9, 4, 19)
+    X, Y = X.astype(np.float32), Y.astype(np.float32)
+    m = Mlp(9, 16, nh, 4)
+    m.set_params(p)
+    m.set_norm(*norm)
+    loss, g = m.loss_grad(torch.tensor(X, device="cuda"), torch.tensor(Y, device="cuda"))
+    m.close()
+    normf = tuple(np.asarray(a, np.float32).astype(np.float64) for a in norm)
+    lr, gr = mlp_ref.loss_grad(p, dims, X, Y, normf, "bf16")
+    assert abs(loss - lr) <= 5e-4 * lr
+    q = 0
+    for d, o in dims:
+        for sz in (d * o, o):
+            a, b = g[q:q + sz], gr[q:q + sz]
+            assert np.linalg.norm(a - b) <= 5e-4 * np.linalg.norm(b), (d, o, sz)
+            q += sz
