@@ -27,11 +27,8 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ uint16_t to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint16_t to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 // C[M x N] = A[M x K] . B[K x N] with A(m, k) = A[m sam + k sak],
 // B(k, n) = B[k sbk + n sbn]; bf16 operands, FP32 accumulation.

@@ -40,11 +40,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr double kInv2PiQ = 0.15915494309189533577;
 
 // float -> bf16 bits, round to nearest even (finite inputs)
-__device__ __forceinline__ uint32_t bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return u >> 16;
-}
+__device__ __forceinline__ uint32_t bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float bf16_val(uint32_t b) { return __uint_as_float(b << 16); }
 // bf16 element e (< 4) of four packed in a uint2, as float
 __device__ __forceinline__ float bf16_half(uint2 v, int e) {
@@ -88,19 +84,17 @@ __global__ __launch_bounds__(256) void k_qf_zgen(QfJob J) {
         }
     }
     const double dx = x - J.x0, dy = y - J.y0;
+    // no branch around a component: its record's loads would wait one by one
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int m = m0 + j;
-        float c = 0.f, s = 0.f;
-        if (live && m < J.n) {
-            const PhaseRec ph = J.ph[m];
-            double a = ph.k * (ph.cth * dx + ph.sth * dy) - ph.omega * t + ph.ph0;
-            a *= kInv2PiQ;
-            a -= rint(a);
-            const float f = (float)a;
-            s = __builtin_amdgcn_sinf(f);
-            c = __builtin_amdgcn_cosf(f);
-        }
+        const bool in = live && m < J.n;
+        const PhaseRec ph = J.ph[m < J.n ? m : J.n - 1];
+        double a = ph.k * (ph.cth * dx + ph.sth * dy) - ph.omega * t + ph.ph0;
+        a *= kInv2PiQ;
+        a -= rint(a);
+        const float f = (float)a;
+        const float s = in ? __builtin_amdgcn_sinf(f) : 0.f, c = in ? __builtin_amdgcn_cosf(f) : 0.f;
         ch[j] = bf16_bits(c); cl[j] = bf16_bits(c - bf16_val(ch[j]));
         sh[j] = bf16_bits(s); sl[j] = bf16_bits(s - bf16_val(sh[j]));
     }
