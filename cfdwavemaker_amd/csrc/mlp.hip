@@ -261,7 +261,11 @@ __global__ __launch_bounds__(256) void k_sum_chunks(int64_t np, int nz, const fl
 // master parameters, and only the unstandardised outputs reach HBM.  Each
 // wave takes 32-column blocks of a layer in turn, both 32-row halves at once
 // (k order, products and epilogue as k_mm), so the outputs equal
-// the layer-wise path's bit for bit.  Limits: at most kFiL layers, widths up to kFiW.
+// the layer-wise path's bit for bit.  Weights come as bf16 operands laid out
+// once a call (k_mlp_pack, 5 us): read as FP32 rows and rounded in every block
+// they took a third of the time (262,144 rows of the 33-256-256-256-65 network
+// 665 us, 490 now; the erf of 768 values a row bounds it at about 300).
+// Limits: at most kFiL layers, widths up to kFiW.
 constexpr int kFiR = 64, kFiW = 256, kFiS = kFiW + 8, kFiL = 8;   // rows, max width, LDS row stride
 
 struct MlpFused {
@@ -269,11 +273,30 @@ struct MlpFused {
     int L = 0, nin = 0, nout = 0;
     int din[kFiL] = {}, dout[kFiL] = {};
     const float* W[kFiL] = {};            // W_l[j][k], dout x din
+    uint16_t* Wp = nullptr;               // their bf16 operands (k_mlp_pack), layer l from woff[l]
+    int woff[kFiL + 1] = {};
     const float* b[kFiL] = {};
     const float *mu_in = nullptr, *sd_in = nullptr, *mu_out = nullptr, *sd_out = nullptr;
     const float* X = nullptr;             // n x nin
     float* Y = nullptr;                   // n x nout
 };
+
+// Weights as the products take them: layer by layer, a lane's 8 bf16 values of
+// each (32-column block, 16 values of k) consecutive, zero past N and K.
+__global__ __launch_bounds__(256) void k_mlp_pack(MlpFused a) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    int l = 0;
+    while (l < a.L && i * 8 >= a.woff[l + 1]) ++l;
+    if (l >= a.L) return;
+    const int K = a.din[l], N = a.dout[l], ks = (K + 15) / 16;
+    const int e = i - a.woff[l] / 8, lane = e & 63, s = (e >> 6) % ks, ct = (e >> 6) / ks;
+    const int col = ct * 32 + (lane & 31), k0 = s * 16 + (lane >> 5) * 8;
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        v[j] = __builtin_bit_cast(__bf16, to_bf16(col < N && k0 + j < K ? a.W[l][(int64_t)col * K + k0 + j] : 0.f));
+    *reinterpret_cast<bf16x8*>(a.Wp + (int64_t)i * 8) = v;
+}
 
 __global__ __launch_bounds__(256) void k_mlp_fused(MlpFused a) {
     __shared__ __attribute__((aligned(16))) uint16_t H[2][kFiR * kFiS];
@@ -294,54 +317,33 @@ __global__ __launch_bounds__(256) void k_mlp_fused(MlpFused a) {
         const int K = a.din[l], N = a.dout[l];
         const int Kp = (K + 15) & ~15;
         const bool last = l == a.L - 1;
-        const float* __restrict__ W = a.W[l];
+        const uint16_t* __restrict__ W = a.Wp + a.woff[l];
         const float* __restrict__ bias = a.b[l];
-        // 16-byte weight loads when every k step lies inside the row (K a multiple of 16)
-        const bool wvec = (K & 15) == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0;
         const int nct = (N + 31) / 32;
         // column block ct of both 32-row halves: two accumulators sharing each B operand
         for (int ct = w; ct < nct; ct += 4) {
             const int col = ct * 32 + (lane & 31);
-            const float* __restrict__ wc = W + (int64_t)(col < N ? col : 0) * K;
             const uint16_t* h0 = &H[cur][(lane & 31) * kFiS + kh];
             const uint16_t* h1 = h0 + 32 * kFiS;
             f32x16 acc0, acc1;
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc0[r] = acc1[r] = 0.f;
-            if (wvec) {
-                // 16-byte weight loads, the next k step's requested before this step's products
-                const float4* q = reinterpret_cast<const float4*>(wc + kh);
-                float4 u = q[0], v = q[1];
-                for (int k0 = 0; k0 < Kp; k0 += 16) {
-                    const int kn = k0 + 16 < Kp ? k0 + 16 : k0;
-                    const float4 un = q[kn / 4], vn = q[kn / 4 + 1];
-                    const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-                    bf16x8 B8;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) B8[j] = __builtin_bit_cast(__bf16, to_bf16(col < N ? f[j] : 0.f));
-                    const bf16x8 A0 = *reinterpret_cast<const bf16x8*>(h0 + k0);
-                    const bf16x8 A1 = *reinterpret_cast<const bf16x8*>(h1 + k0);
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B8, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B8, acc1, 0, 0, 0);
-                    u = un;
-                    v = vn;
-                }
-            } else {
-                for (int k0 = 0; k0 < Kp; k0 += 16) {
-                    bf16x8 B8;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int k = k0 + kh + j;
-                        B8[j] = __builtin_bit_cast(__bf16, to_bf16(k < K && col < N ? wc[k] : 0.f));
-                    }
-                    const bf16x8 A0 = *reinterpret_cast<const bf16x8*>(h0 + k0);
-                    const bf16x8 A1 = *reinterpret_cast<const bf16x8*>(h1 + k0);
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B8, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B8, acc1, 0, 0, 0);
-                }
+            // the next k step's weights requested before this step's products
+            const uint4* q = reinterpret_cast<const uint4*>(W) + (int64_t)ct * (Kp / 16) * 64 + lane;
+            uint4 u = *q;
+            for (int k0 = 0; k0 < Kp; k0 += 16) {
+                q += k0 + 16 < Kp ? 64 : 0;
+                const uint4 un = *q;
+                const bf16x8 B8 = __builtin_bit_cast(bf16x8, u);
+                const bf16x8 A0 = *reinterpret_cast<const bf16x8*>(h0 + k0);
+                const bf16x8 A1 = *reinterpret_cast<const bf16x8*>(h1 + k0);
+                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B8, acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B8, acc1, 0, 0, 0);
+                u = un;
             }
             if (col >= N) continue;
             const float bc = bias[col];
+            const float so = last ? a.sd_out[col] : 0.f, mo = last ? a.mu_out[col] : 0.f;
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
 #pragma unroll
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(256) void k_mlp_fused(MlpFused a) {
                     if (!last) {
                         H[cur ^ 1][row * kFiS + col] = to_bf16(gelu(v));
                     } else if (r0 + row < a.n) {
-                        a.Y[(r0 + row) * a.nout + col] = v * a.sd_out[col] + a.mu_out[col];
+                        a.Y[(r0 + row) * a.nout + col] = v * so + mo;
                     }
                 }
             }
@@ -442,6 +444,14 @@ struct Mlp {
     DevBuf norm;                          // in_mean, in_std, out_mean, out_std
     DevBuf act;                           // H_0..H_L and Z_0..Z_{L-1} for a batch
     DevBuf tmp, part, idx;
+    DevBuf wpk;                          // bf16 weights of the fused kernel
+    bool fused() const {
+        bool f = layers() <= kFiL && nin <= kFiW;
+        for (int l = 0; l < layers(); ++l) f = f && dout[l] <= kFiW;
+        return f;
+    }
+    // bf16 values of layer l in wpk
+    int packed(int l) const { return (dout[l] + 31) / 32 * ((din[l] + 15) / 16) * 512; }
     DevBuf gpart;                         // [chunk][np]: the row chunks' gradients
     int64_t cap = 0;                      // rows the activation buffers hold
     int64_t adam_t = 0;
@@ -589,6 +599,11 @@ int cfdwm_mlp_create(cfdwm_mlp** out, int nin, int width, int nhidden, int nout,
         M.boff.push_back(M.np);
         M.np += M.dout[l];
     }
+    if (M.fused()) {
+        size_t wp = 0;
+        for (int l = 0; l < M.layers(); ++l) wp += M.packed(l);
+        if (M.wpk.alloc(wp * sizeof(uint16_t))) { delete h; return -3; }
+    }
     // He-style uniform initialisation (limit sqrt(6 / fan_in)), zero biases
     std::vector<float> p(M.np, 0.f);
     std::mt19937_64 rng(seed);
@@ -670,17 +685,19 @@ int cfdwm_mlp_forward_device(cfdwm_mlp* h, int64_t n, const float* X, float* Y) 
     hipStream_t st = Engine::get().stream();
     // large batches: the fused kernel (256 blocks of 64 rows fill the GPU);
     // smaller ones run layer by layer, whose 64 x 64 output tiles give more blocks
-    bool fits = M.layers() <= kFiL && M.nin <= kFiW;
-    for (int l = 0; l < M.layers(); ++l) fits = fits && M.dout[l] <= kFiW;
-    if (fits && n >= 256 * kFiR) {
+    if (M.fused() && n >= 256 * kFiR) {
         MlpFused F;
         F.n = n; F.L = M.layers(); F.nin = M.nin; F.nout = M.nout;
         for (int l = 0; l < F.L; ++l) {
             F.din[l] = M.din[l]; F.dout[l] = M.dout[l];
             F.W[l] = M.P() + M.woff[l]; F.b[l] = M.P() + M.boff[l];
+            F.woff[l + 1] = F.woff[l] + M.packed(l);
         }
+        F.Wp = (uint16_t*)M.wpk.get();
         F.mu_in = M.nin_mu(); F.sd_in = M.nin_sd(); F.mu_out = M.nout_mu(); F.sd_out = M.nout_sd();
         F.X = X; F.Y = Y;
+        hipLaunchKernelGGL(k_mlp_pack, dim3(nb256(F.woff[F.L] / 8)), dim3(256), 0, st, F);
+        CFDWM_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_mlp_fused, dim3((unsigned)((n + kFiR - 1) / kFiR)), dim3(256), 0, st, F);
         CFDWM_HIP(hipGetLastError());
         return 0;
