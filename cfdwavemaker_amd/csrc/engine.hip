@@ -454,6 +454,7 @@ int Sea::qform_meta(const QfTables** out) {
     auto T = std::make_unique<QfTables>();
     T->npad = npad; T->nform = nform; T->rank = R; T->rank_v = Rv; T->rank_w = Rw; T->mu = BC.mu; T->mu_w = BS.mu;
     T->basis_err = std::max(BC.err, BS.err);
+    T->kmax = kmx;
     // The level pass's first-order and diagonal terms through profile bases
     // over [0, 2 kmax] (the diagonal's profile is that of 2 k_i): by default in
     // the one-product (bf16) mode, whose velocity error (~1e-3 of the field
@@ -506,10 +507,19 @@ int Sea::qform_meta(const QfTables** out) {
     T->table_bytes = (size_t)(split ? nform - 1 : nform) * nbarr * nn * sizeof(uint16_t);
     T->eta_bytes = split ? 4 * nn * sizeof(uint16_t) : 0;
     hipStream_t st = Engine::get().stream();
-    if (T->zs.upload(BC.zs.data(), R * sizeof(double), st) ||
-        T->finv.upload(BC.finv.data(), (size_t)R * R * sizeof(double), st) ||
-        T->zsw.upload(BS.zs.data(), Rw * sizeof(double), st) ||
-        T->finvw.upload(BS.finv.data(), (size_t)Rw * Rw * sizeof(double), st) ||
+    // rows of 32 doubles, zeros past the rank (what the table build reads)
+    auto rows32 = [](const std::vector<double>& v, int rows, int R) {
+        std::vector<double> o((size_t)rows * 32, 0.0);
+        for (int q = 0; q < rows; ++q)
+            for (int s = 0; s < R; ++s) o[(size_t)q * 32 + s] = v[(size_t)q * R + s];
+        return o;
+    };
+    const std::vector<double> zc = rows32(BC.zs, 1, R), fc = rows32(BC.finv, R, R);
+    const std::vector<double> zw = rows32(BS.zs, 1, Rw), fw = rows32(BS.finv, Rw, Rw);
+    if (T->zs.upload(zc.data(), zc.size() * sizeof(double), st) ||
+        T->finv.upload(fc.data(), fc.size() * sizeof(double), st) ||
+        T->zsw.upload(zw.data(), zw.size() * sizeof(double), st) ||
+        T->finvw.upload(fw.data(), fw.size() * sizeof(double), st) ||
         T->ftype.upload(ftype.data(), ftype.size(), st) ||
         T->kend.upload(kend.data(), kend.size() * sizeof(int32_t), st))
         return -3;
@@ -519,15 +529,14 @@ int Sea::qform_meta(const QfTables** out) {
     return 1;
 }
 
-// Zero the table memory and launch the table build into it (library stream).
+// Launch the table build into the memory (library stream).
 int Sea::qform_build(QfTables& T, uint16_t* b, uint16_t* beta) {
     hipStream_t st = Engine::get().stream();
     const bool split = T.nlv == 1;
-    if (split) CFDWM_HIP(hipMemsetAsync(beta, 0, T.eta_bytes, st));
-    CFDWM_HIP(hipMemsetAsync(b, 0, T.table_bytes, st));
     QfBuild Bq;
     Bq.n = tab.comp.n; Bq.npad = T.npad; Bq.R = T.rank; Bq.Rv = T.rank_v; Bq.Rw = T.rank_w; Bq.nform = T.nform; Bq.nbarr = T.nbarr;
     Bq.h = tab.in.depth;
+    Bq.normal = T.kmax * tab.in.depth <= 300.0;
     Bq.frow = d32_.frow; Bq.fmhi = d32_.fmhi; Bq.uvw = d32_.fuvw; Bq.x = d32_.fx;
     Bq.zs = (const double*)T.zs.get(); Bq.finv = (const double*)T.finv.get();
     Bq.zsw = (const double*)T.zsw.get(); Bq.finvw = (const double*)T.finvw.get();

@@ -360,6 +360,7 @@ public:
     // cosh-type profile basis and the w forms (sin-type) of the sinh-type one
     struct QfTables {
         int npad = 0, nform = 0, rank = 0, rank_w = 0;   // ranks of the cosh- and sinh-type profile bases
+        double kmax = 0;                     // largest combined wavenumber
         int rank_v = 0;                      // forms of v: rank, or 0 where every v coefficient is zero
         int nlv = 3, nbarr = 4;              // bf16 products per term, table arrays per form
         double basis_err = 0, basis_tol = 0;

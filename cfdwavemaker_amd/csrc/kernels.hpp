@@ -171,11 +171,12 @@ struct QfBuild {
     const int32_t* fmhi = nullptr;
     const UvwRec<float>* uvw = nullptr;   // pk = kappa log2 e
     const XRec<float>* x = nullptr;
-    const double* zs = nullptr;           // [R] skeleton depths of the cosh-type basis
-    const double* finv = nullptr;         // [R][R]
-    const double* zsw = nullptr;          // [Rw] skeleton depths of the sinh-type basis
-    const double* finvw = nullptr;        // [Rw][Rw]
-    uint16_t* b = nullptr;                // [nform][nbarr][npad x npad], zeroed by the caller
+    const double* zs = nullptr;           // [32] skeleton depths of the cosh-type basis, zeros past R
+    const double* finv = nullptr;         // [R][32], zeros past R
+    const double* zsw = nullptr;          // [32] skeleton depths of the sinh-type basis
+    const double* finvw = nullptr;        // [Rw][32]
+    uint16_t* b = nullptr;                // [nform][nbarr][npad x npad]; written from each 128-row tile's diagonal block on
+    int normal = 0;                       // e^{-2 kappa h} is a normal number at every kappa
     int nbarr = 4;                        // 4: hi and lo parts, 2: hi parts only
     uint16_t* beta = nullptr;             // when set: form 0 (eta2) goes here as [4][npad x npad]
                                           // and form f > 0 to b at index f - 1

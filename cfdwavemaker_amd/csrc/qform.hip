@@ -863,17 +863,46 @@ void k_qf_forms_persist(const QfJob* __restrict__ jobs, const QfTile* __restrict
     }
 }
 
-// Form tables: one thread per (i, m) of the filtered pair set.  Profile-basis
-// coefficients c_q(kappa) = sum_s finv[q][s] P_kappa(z_s) in FP64 (finv is
-// ill-conditioned: its entries are large while |c| stays O(1)), entries
-// written as bf16 hi + lo into the tiled layout.
+// a wave-uniform element of a table no launch writes: a scalar load
+__device__ __forceinline__ double ro_load(const double* p, int i) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return ((const __attribute__((address_space(4))) double*)p)[i];
+#else
+    return p[i];
+#endif
+}
+// 1 / x to an ulp, x and 1 / x normal
+__device__ __forceinline__ double rcp_nr(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// Form tables: one thread per (i, m).  Profile-basis coefficients c_q(kappa) =
+// sum_s finv[q][s] P_kappa(z_s) in FP64 (finv is ill-conditioned: its entries
+// are large while |c| stays O(1)), entries written as bf16 hi + lo into the
+// tiled layout, zeros where there is no pair, over all the forms kernels read:
+// m from the first row of i's 128-row tile on.  The exponentials bound it, so
+// the second one of a profile is e^{-2 kappa h} over the first while both stay
+// normal numbers; a wave takes 4 rows x 16 m, so that its 2-byte stores fill
+// 64 bytes.  Loads and exponentials go in fours and eights without a branch
+// between them, and ranks to 16 (the one-product mode's) take half the
+// registers.  2048 components, 38 forms: 465 us and 140 for zeroing the tables
+// before, 366 now.
+template <int RM>
 __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
-    const int i = blockIdx.y;
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= B.n || m <= i || m >= B.fmhi[i]) return;
-    const int64_t e = B.frow[i] - (i + 1) + m;
-    const UvwRec<float> r = B.uvw[e];
-    const XRec<float> xr = B.x[e];
+    const int lane = threadIdx.x & 63;
+    if ((int)blockIdx.x * 64 < (((int)blockIdx.y * 4) & ~127)) return;
+    const int i = blockIdx.y * 4 + ((lane >> 3) & 3);
+    const int m = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + (lane & 7) + (lane >> 5) * 8;
+    const bool pair = i < B.n && m > i && m < B.fmhi[i];
+    UvwRec<float> r{};
+    XRec<float> xr{};
+    if (pair) {
+        const int64_t e = B.frow[i] - (i + 1) + m;
+        r = B.uvw[e];
+        xr = B.x[e];
+    }
     constexpr double kL2eInv = 0.69314718055994530942;   // ln 2: kappa = pk / log2 e
     const double kp = (double)r.pkP * kL2eInv, km = (double)r.pkM * kL2eInv;
     const int nkb = B.npad >> 4;
@@ -891,24 +920,51 @@ __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
     };
     put(0, 0, (double)xr.xP + (double)xr.xM);
     put(0, 1, (double)xr.xM - (double)xr.xP);
+    if (!__any(pair)) {
+        for (int f = 1; f < B.nform; ++f) {
+            put(f, 0, 0.0);
+            put(f, 1, 0.0);
+        }
+        return;
+    }
     // profile P_kappa(z) = e^{kappa z} + sg e^{-kappa (z + 2h)} at the
     // skeleton depths, then its basis coefficients c = finv P (one family at a time)
-    double eP[32], eM[32];
+    double eP[RM], eM[RM];
+    const double gP = exp(-2.0 * kp * B.h), gM = exp(-2.0 * km * B.h);
     auto family = [&](int R, const double* zs, const double* finv, double sg, int f0, int nf) {
+        // four depths at a time: their exponentials' chains run side by side
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const double z = q < R ? zs[q] : 0.0;
-            eP[q] = q < R ? exp(kp * z) + sg * exp(-kp * (z + 2.0 * B.h)) : 0.0;
-            eM[q] = q < R ? exp(km * z) + sg * exp(-km * (z + 2.0 * B.h)) : 0.0;
+        for (int c = 0; c < RM; c += 4) {
+            if (c < R) {
+#pragma unroll
+                for (int q = c; q < c + 4; ++q) {
+                    const double z = ro_load(zs, q);
+                    const double E = exp(kp * z), F = exp(km * z);
+                    if (B.normal) {
+                        eP[q] = E + sg * (gP * rcp_nr(E));
+                        eM[q] = F + sg * (gM * rcp_nr(F));
+                    } else {
+                        eP[q] = E + sg * exp(-kp * (z + 2.0 * B.h));
+                        eM[q] = F + sg * exp(-km * (z + 2.0 * B.h));
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int q = c; q < c + 4; ++q) eP[q] = eM[q] = 0.0;
+            }
         }
         for (int q = 0; q < R; ++q) {
             double cp = 0, cm = 0;
+// (rows of 32, zeros past R: eight at a time come with one scalar load)
 #pragma unroll
-            for (int s2 = 0; s2 < 32; ++s2) {
-                if (s2 < R) {
-                    const double w = finv[q * R + s2];
-                    cp += w * eP[s2];
-                    cm += w * eM[s2];
+            for (int c = 0; c < RM; c += 8) {
+                if (c < R) {
+#pragma unroll
+                    for (int s2 = c; s2 < c + 8; ++s2) {
+                        const double w = ro_load(finv, q * 32 + s2);
+                        cp += w * eP[s2];
+                        cm += w * eM[s2];
+                    }
                 }
             }
             if (nf == 2) {                            // u, v (cos-type)
@@ -934,7 +990,10 @@ hipError_t launch_qf_build(const QfBuild& B, hipStream_t st) {
     if (B.n <= 0 || B.R < 0 || B.R > 32 || B.Rw < 0 || B.Rw > 32 || (B.Rv && B.Rv != B.R) || B.nform != 1 + B.R + B.Rv + B.Rw ||
         (B.npad & 127) || B.npad < B.n || (B.nbarr != 2 && B.nbarr != 4))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_qf_build, dim3((unsigned)((B.npad + 255) / 256), (unsigned)B.n), dim3(256), 0, st, B);
+    // ranks to 16 leave twice the waves: 578 us with 32 where 16 takes 366
+    const dim3 grid((unsigned)(B.npad / 64), (unsigned)(B.npad / 4));
+    if (B.R <= 16 && B.Rw <= 16) hipLaunchKernelGGL(k_qf_build<16>, grid, dim3(256), 0, st, B);
+    else hipLaunchKernelGGL(k_qf_build<32>, grid, dim3(256), 0, st, B);
     return hipGetLastError();
 }
 
