@@ -10,8 +10,18 @@ namespace dm {
 
 constexpr double kInv2Pi = 0.15915494309189533577;
 
+// 1 / x to an ulp, x and 1 / x normal
+__device__ __forceinline__ double rcp_nr(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
 // Irregular::freq_ramp (Irregular.cpp:200-204)
 __device__ __forceinline__ double freq_ramp(double t, double rt, double ts, double du) {
+    // past the ramp up and before the ramp down both quotients clamp to one:
+    // no divisions then (they cost as much as a component's sine and cosine)
+    if (t - ts >= rt + 1e-12 && t - ts - du + rt <= 0. && rt + 1e-12 > 0.) return 1.;
     const double a = 1. - ((t - ts - du + rt) / (rt + 1e-12));
     const double b = (t - ts) / (rt + 1e-12);
     const double down = a < 1. ? (a < 0. ? 0. : a) : 1.;

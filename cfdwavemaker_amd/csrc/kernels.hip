@@ -25,6 +25,7 @@ namespace {
 using dm::cs_of;
 using dm::freq_ramp;
 using dm::phase_of;
+using dm::rcp_nr;
 
 // ---------------------------------------------------------------- helpers
 
@@ -65,12 +66,6 @@ __device__ __forceinline__ void prof(float pk, float pg, float z, float& E, floa
 template <typename R>
 __device__ __forceinline__ R fmaR(R a, R b, R c) { return a * b + c; }
 
-// 1 / x to an ulp, x and 1 / x normal
-__device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
 
 // the exponential of prof(): natural base in FP64, base 2 (hardware) in FP32
 __device__ __forceinline__ double pexp(double a) { return exp(a); }

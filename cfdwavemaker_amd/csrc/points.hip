@@ -329,8 +329,8 @@ void k_point_forms(SeaDev<R> S, PointJob J) {
             if (!slow) {
                 R F, f;
                 if constexpr (sizeof(R) == 8) {
-                    F = 1. / (E * Ekr);
-                    f = 1. / (G * Gkr);
+                    F = dm::rcp_nr(E * Ekr);
+                    f = dm::rcp_nr(G * Gkr);
                 } else {
                     const Hl<R> kd = Hl<R>::k(kr - pr.k);
                     F = pe(kd, zh);

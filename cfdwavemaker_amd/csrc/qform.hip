@@ -27,6 +27,7 @@
 // checks this and passes one factor per time slot.
 #include <hip/hip_runtime.h>
 
+#include "device_math.hpp"
 #include "engine.hpp"
 #include "kernels.hpp"
 
@@ -871,12 +872,6 @@ __device__ __forceinline__ double ro_load(const double* p, int i) {
     return p[i];
 #endif
 }
-// 1 / x to an ulp, x and 1 / x normal
-__device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
 
 // Form tables: one thread per (i, m).  Profile-basis coefficients c_q(kappa) =
 // sum_s finv[q][s] P_kappa(z_s) in FP64 (finv is ill-conditioned: its entries
@@ -941,8 +936,8 @@ __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
                     const double z = ro_load(zs, q);
                     const double E = exp(kp * z), F = exp(km * z);
                     if (B.normal) {
-                        eP[q] = E + sg * (gP * rcp_nr(E));
-                        eM[q] = F + sg * (gM * rcp_nr(F));
+                        eP[q] = E + sg * (gP * dm::rcp_nr(E));
+                        eM[q] = F + sg * (gM * dm::rcp_nr(F));
                     } else {
                         eP[q] = E + sg * exp(-kp * (z + 2.0 * B.h));
                         eM[q] = F + sg * exp(-km * (z + 2.0 * B.h));
