@@ -762,7 +762,7 @@ def main():
 
     points = 4 * NX * NY * NL
     value = points * a.steps / el
-    # queries: cell ordering (key pass + radix sort) plus the spline kernel
+    # queries: cell ordering (tile counting passes) plus the spline kernel
     q_ms, q_n = prof.get("k_query", (float("nan"), 1))
     q_ms += prof.get("k_query_sort", (0.0, 1))[0]
     qfi = grid.qform_info()
@@ -790,10 +790,10 @@ def main():
         alg_launch = (24.0 if split else 32.0) * ncomp * ncomp * cs / per_fill
         # the eta2 form runs three products per term, each velocity form one
         flop_launch = fill_exec * nvf / (nvf + 3.0) if split else fill_exec
-        roof = {"bound": "mfma", "kernel": "k_qf_forms_il<1> (velocity forms)" if split else "k_qf_forms_il<3>",
+        roof = {"bound": "mfma", "kernel": "k_qf_pairs (velocity forms)" if split else "k_qf_forms_il<3, 4>",
                 "achieved": alg_launch / avg / 1e12,
                 "peak": PEAK_MFMA_BF16 / 1e12, "unit": "TFLOP/s", "frac": alg_launch / avg / PEAK_MFMA_BF16,
-                "traffic": profiled_traffic("k_qf_forms_il<1>" if split else "k_qf_forms_il<3>", a.precision),
+                "traffic": profiled_traffic("k_qf_pairs" if split else "k_qf_forms_il<3, 4>", a.precision),
                 "traffic_source": "profiles/*_fetch_size.md + *_write_size.md (rocprofv3 --pmc, calibrated)",
                 "avg_launch_ms": avg * 1e3, "flop_per_launch": alg_launch,
                 "flop_rule": ("24 N^2 per column-slot (u, v, w forms x 2 (2N)^2)" if split
@@ -806,7 +806,7 @@ def main():
         if split and e_n:
             e_avg = e_ms / e_n * 1e-3
             step_alg = 32.0 * ncomp * ncomp * cs
-            roof["forms_step"] = {"kernels": "k_qf_forms_il<3> (eta2) + k_qf_forms_il<1> (velocities)",
+            roof["forms_step"] = {"kernels": "k_qf_eta (eta2) + k_qf_pairs (velocities)",
                                   "ms": (avg + e_avg) * 1e3, "eta2_launch_ms": e_avg * 1e3,
                                   "flop": step_alg, "achieved": step_alg / (avg + e_avg) / 1e12,
                                   "frac": step_alg / (avg + e_avg) / PEAK_MFMA_BF16,

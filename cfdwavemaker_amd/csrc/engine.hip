@@ -1184,14 +1184,16 @@ int Grid::qform_prepare(int nslot, const double* slot_t, int64_t ncol, const int
     }
     // executed MFMA flops per padded point and form: a 128-wide i tile runs
     // both 64-row halves from its first row to the larger of their two kend,
-    // 128 x (kend - i0) products, two operand pairs (c and s), 3 or 1 bf16 products
-    double tri = 0;
+    // 128 x (kend - i0) products, two operand pairs (c and s), 3 or 1 bf16
+    // products; but for the eta2 kernel the second half leaves out 64 values of k
+    double tri = 0, skip = 0;
     for (size_t t = 0; t + 1 < T->kend_h.size(); t += 2) {
-        const int ke = std::max(T->kend_h[t], T->kend_h[t + 1]);
-        tri += 128.0 * std::max(0, ke - (int)(64 * t)) * 2 * 2;
+        const int k = std::max(0, std::max(T->kend_h[t], T->kend_h[t + 1]) - (int)(64 * t));
+        tri += 128.0 * k * 2 * 2;
+        skip += 64.0 * std::min(k, 64) * 2 * 2;
     }
-    qf_fpp_ = 3 * tri;
-    qf_fpp1_ = tri;
+    qf_fpp_ = 3 * (qf_split_ ? tri : tri - skip);
+    qf_fpp1_ = tri - skip;
     qf_nlv = T->nlv;
     qf_nform = T->nform;
     qf_rank = R;
