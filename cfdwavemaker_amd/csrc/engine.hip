@@ -766,6 +766,7 @@ int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const doub
                uint32_t flags, bool want_cols, bool want_lin, bool want_eta2, bool want_lev, double* o) {
     hipStream_t st = Engine::get().stream();
     const SeaDev<R>& S = s.dev<R>();
+    bool e2_levels = false;
     if (want_cols) {
         ColumnJob<R> J;
         J.nslot = 1; J.ncol = n;
@@ -774,12 +775,22 @@ int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const doub
         J.want_eta2 = want_eta2 ? 1 : 0;
         J.o_eta1 = o; J.o_eta2 = o + n; J.o_gx = o + 2 * n; J.o_gy = o + 3 * n; J.o_gz = o + 4 * n; J.o_gp = o + 5 * n;
         J.nseg = want_eta2 ? pick_nseg(n, s.table_records(false)) : 1;
+        bool form = false;
         if constexpr (sizeof(R) == 4) {
             const int rc = points_eta2_form(s, n, dx, dy, dt, want_eta2, J);
             if (rc < 0) return rc;
-            if (rc == 1) J.nseg = 1;
+            form = rc == 1;
+            if (form) J.nseg = 1;
         }
-        J.seg = s.segments(false, J.nseg);
+        // with the unfiltered pair loop to follow, eta2's pairs go along with it
+        e2_levels = want_eta2 && !form && want_lev && (flags & EV_SEC) && (flags & EV_DIRECT);
+        if (e2_levels) {
+            J.pairs = 0;
+            J.nseg = std::max(1, std::min(J.nseg, s.tab.comp.n / 16));
+            J.seg = s.comp_segments(J.nseg);
+        } else {
+            J.seg = s.segments(false, J.nseg);
+        }
         if (!J.seg) return -3;
         if (J.nseg > 1) {
             if (s.partial.alloc((size_t)J.nseg * n * 6 * sizeof(double))) return -3;
@@ -793,12 +804,13 @@ int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const doub
         J.x = dx; J.y = dy; J.z = dz; J.t = dt;
         J.flags = flags;
         J.p_u = o + 6 * n; J.p_v = o + 7 * n; J.p_w = o + 8 * n; J.p_p = o + 9 * n;
+        if (e2_levels) J.p_e2 = o + n;
         const bool direct = (flags & EV_DIRECT) != 0;
         J.nseg = (flags & EV_SEC) ? pick_nseg(n, s.table_records(direct)) : 1;
         J.seg = s.segments(direct, J.nseg);
         if (!J.seg) return -3;
         if (J.nseg > 1) {
-            if (s.partial.alloc((size_t)J.nseg * n * 9 * sizeof(double))) return -3;
+            if (s.partial.alloc((size_t)J.nseg * n * 10 * sizeof(double))) return -3;
             J.partial = (double*)s.partial.get();
         }
         PROF("k_levels_points", launch_levels<R>(S, J, false, 1, st));

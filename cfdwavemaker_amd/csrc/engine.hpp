@@ -51,6 +51,7 @@ struct LevelJob {
     R *o_u = nullptr, *o_v = nullptr, *o_w = nullptr;
     const double *x = nullptr, *y = nullptr, *t = nullptr, *z = nullptr;
     double *p_u = nullptr, *p_v = nullptr, *p_w = nullptr, *p_p = nullptr;
+    double* p_e2 = nullptr;               // points: the pair sum is added to the eta2 there
     uint32_t flags = 0;
     const uint32_t* lvl = nullptr;        // GRID: per filtered pair record, pruning level bounds
     // GRID: pair sums from the MFMA quadratic forms instead of the pair loop:

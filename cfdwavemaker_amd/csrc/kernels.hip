@@ -297,7 +297,7 @@ __device__ __forceinline__ LevPos<R, LC, GRID> lev_pos(const SeaDev<R>& S, const
     return P;
 }
 
-// final level outputs.  a = {U[LC], V[LC], W[LC], gx, gy, gz, gp, P, P2}
+// final level outputs.  a = {U[LC], V[LC], W[LC], gx, gy, gz, gp, P, P2}, at points also eta2's pair sum
 template <typename R, int LC, bool GRID, bool WP>
 __device__ __forceinline__ void lev_store(const SeaDev<R>& S, const LevelJob<R>& J, uint32_t fl,
                                           const LevPos<R, LC, GRID>& P, const double* a) {
@@ -319,6 +319,7 @@ __device__ __forceinline__ void lev_store(const SeaDev<R>& S, const LevelJob<R>&
         J.p_u[P.cq] = a[0] + (tay ? gx * z1 : 0.);
         J.p_v[P.cq] = a[LC] + (tay ? gy * z1 : 0.);
         J.p_w[P.cq] = a[2 * LC] + (tay ? gz * z1 : 0.);
+        if (J.p_e2) J.p_e2[P.cq] += a[3 * LC + 6];
         if (WP) J.p_p[P.cq] = a[3 * LC + 4] + S.rho * a[3 * LC + 5] + (tay ? gp * z1 : 0.);
     }
 }
@@ -555,7 +556,7 @@ template <typename R, int LC, int MODE, int F8 = 0>
 __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R>& J) {
     constexpr bool GRID = MODE == 0;
     constexpr bool WP = MODE == 2;
-    constexpr int RS = 3 * LC + 6;
+    constexpr int RS = 3 * LC + 6 + (GRID ? 0 : 1);
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t fl = GRID ? (uint32_t)(EV_LIN | EV_SEC | EV_TAYLOR) : J.flags;
     const LevPos<R, LC, GRID> PP = lev_pos<R, LC, GRID>(S, J, tid, fl);
@@ -572,6 +573,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
 #pragma unroll
     for (int l = 0; l < LC; ++l) U[l] = V[l] = W[l] = 0.;
     double P = 0., P2 = 0.;   // pressure (MODE 2, LC == 1)
+    double E2 = 0.;           // eta2's pair sum (points, J.p_e2)
     double gx = 0, gy = 0, gz = 0, gp = 0;
 
     // dp2 kinetic terms (Irregular.cpp:755-756, 786-787): phase-free and
@@ -728,6 +730,12 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
             const UvwRec<R>* __restrict__ rr = tab + base;
             const XRec<R>* __restrict__ xr = S.dx + base;
             const uint32_t* __restrict__ lvr = J.lvl + base;
+            // points with J.p_e2: the filtered eta2 pairs (i, m < mh) of the same
+            // phases, which took a pass of their own with a sine and cosine a pair
+            // (FP64, 256 components, 4,096 points: 985 + 385 -> 1040 us)
+            const int mh = !GRID && J.p_e2 ? S.fmhi[i] : 0;
+            const XRec<R>* __restrict__ xe = S.fx + S.frow[i] - (i + 1);
+            R er = 0;
             for (int m = m0; m < m1; ++m) {
                 R cm, sm;
                 cs_of(phase_of(S.ph[m], dxp, dyp, t), cm, sm);
@@ -770,6 +778,11 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
                     }
                     continue;
                 }
+                if (!GRID && m < mh) {
+                    const XRec<R> q = xe[m];
+                    er = fmaR(q.xP, cP, er);
+                    er = fmaR(q.xM, cM, er);
+                }
                 R pP = 0, pM = 0;
                 if (WP && direct) {
                     const XRec<R> xq = xr[m];
@@ -793,6 +806,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
                     if (WP && direct) pr = fmaR(pM, ch, pr);
                 }
             }
+            if (!GRID) E2 += (double)er;
         }
         if (!LB && ++nfold == fold_n) {
 #pragma unroll
@@ -917,6 +931,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
     for (int l = 0; l < LC; ++l) { a[l] = U[l]; a[LC + l] = V[l]; a[2 * LC + l] = W[l]; }
     a[3 * LC] = gx; a[3 * LC + 1] = gy; a[3 * LC + 2] = gz; a[3 * LC + 3] = gp;
     a[3 * LC + 4] = P; a[3 * LC + 5] = P2;
+    if constexpr (!GRID) a[3 * LC + 6] = E2;
     if (J.partial) {
         const int64_t nthr = (GRID ? ((int64_t)J.nslot * J.ncol + 63) / 64 * 64 * ((J.g.nl + LC - 1) / LC)
                                    : (int64_t)J.nslot * J.ncol);
@@ -976,7 +991,7 @@ template <typename R, int LC, int MODE>
 __global__ __launch_bounds__(256) void k_levels_reduce(SeaDev<R> S, LevelJob<R> J) {
     constexpr bool GRID = MODE == 0;
     constexpr bool WP = MODE == 2;
-    constexpr int RS = 3 * LC + 6;
+    constexpr int RS = 3 * LC + 6 + (GRID ? 0 : 1);
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nthr = (GRID ? ((int64_t)J.nslot * J.ncol + 63) / 64 * 64 * ((J.g.nl + LC - 1) / LC)
                                : (int64_t)J.nslot * J.ncol);

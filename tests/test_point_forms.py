@@ -144,3 +144,22 @@ def test_unordered_components_take_the_pair_loop(eng):
     for k in ("omega", "A", "k", "phase", "theta"):
         r[k] = np.asarray(s[k])[o]
     _check(_fields(eng, eng.Sea(r), q), _fields(eng, eng.Sea(_pair_loop(r)), q), TOL["fp64"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,ndir,m", [(1, 3, 1), (7, 3, 65), (20, 5, 700)])
+def test_eta2_beside_the_pair_loop(eng, prec, n, ndir, m):
+    """Directional seas: eta2 asked for with the velocities goes along with their pair
+    loop (every pair, filtered ones left out); alone it has its own pass."""
+    import torch
+    p = eng.FP64 if prec == "fp64" else eng.FP32
+    s = make_sea(n, 3.0, 9.0, 30.0, seed=n, ndir=ndir).as_dict()
+    s.update(bandwidth=0.7, cutoff=1.6)
+    sea = eng.Sea(s, precision=p)
+    q = [torch.tensor(a, device="cuda") for a in _points(m, 30.0, n)]
+    a = sea.eval_fields_device(*q)
+    b = sea.eval_fields_device(*q[:3], want=("eta1", "eta2"))
+    for k in ("eta1", "eta2"):
+        x, y = a[k].cpu().numpy(), b[k].cpu().numpy()
+        assert np.max(np.abs(x - y)) <= TOL[prec] * np.max(np.abs(y)), k
