@@ -908,7 +908,9 @@ __global__ __launch_bounds__(256) void k_qf_build(QfBuild B) {
         const bool lo = sep || B.nbarr == 4;
         const int fi = B.beta ? f - 1 : f;
         uint16_t* d = sep ? B.beta + (size_t)(2 * k) * nn : B.b + ((size_t)fi * B.nbarr + (lo ? 2 * k : k)) * nn;
-        const float x = (float)v;
+        // (opaque: else the two roundings become one from FP64)
+        float x = (float)v;
+        __asm__ volatile("" : "+v"(x));
         const uint32_t hi = bf16_bits(x);
         d[o] = (uint16_t)hi;
         if (lo) d[o + nn] = (uint16_t)bf16_bits(x - bf16_val(hi));
