@@ -780,11 +780,12 @@ int run_points(Sea& s, int64_t n, const double* dx, const double* dy, const doub
             const int rc = points_eta2_form(s, n, dx, dy, dt, want_eta2, J);
             if (rc < 0) return rc;
             form = rc == 1;
-            if (form) J.nseg = 1;
         }
-        // with the unfiltered pair loop to follow, eta2's pairs go along with it
+        // with the unfiltered pair loop to follow, eta2's pairs go along with it;
+        // the components alone then are split over segments, as they are beside
+        // the eta2 form (256 components in 16 directions, 4096 points FP32 427 -> 373 us)
         e2_levels = want_eta2 && !form && want_lev && (flags & EV_SEC) && (flags & EV_DIRECT);
-        if (e2_levels) {
+        if (e2_levels || form) {
             J.pairs = 0;
             J.nseg = std::max(1, std::min(J.nseg, s.tab.comp.n / 16));
             J.seg = s.comp_segments(J.nseg);
