@@ -163,8 +163,8 @@ __device__ __forceinline__ u32x4 uni_load4(const uint16_t* base, int off) {
 // __syncthreads() would wait for every request) says that stage j + 1 has
 // landed for all waves and that all waves have read stage j, whose buffer the
 // requests of stage j + 3 then fill; they have two stages' time to land.
-// NP = 4 serves three products; NP = 2 three products in launches too small for
-// two blocks of the wide tile per CU, and one product in launches too small for
+// NP = 4 serves three products; NP = 2 three products in launches of few rounds
+// of the wide tile, and one product in launches too small for
 // a form pair (below) per CU.
 //
 // What bounds three products: the matrix pipe at the clock that random bf16
@@ -611,14 +611,16 @@ __device__ __forceinline__ void qf_pair_tile(const QfJob& J, int ptile, int form
 // Blocks of an XCD (round-robin dispatch) walk the form pairs of two point
 // tiles together: the two tiles' Z operands stay in its L2 (1 MiB of hi parts
 // each at 1024 components), the tables stream through the last-level cache and
-// serve both tiles.  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
+// serve both tiles; the blocks of an odd last tile follow without gaps.  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
 // 32 point tiles, 89 GB one point tile at a time, 73 GB two at a time.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_qf_pairs(QfJob J, int npt) {
-    const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3;
-    const int in = sq % (2 * np);
-    const int ptile = (sq / (2 * np) * 2 + (in & 1)) * 8 + (blockIdx.x & 7);
-    if (ptile >= npt) return;                         // whole block, before any barrier
+    const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+    const int nt = (npt - xcd + 7) >> 3;              // this XCD's point tiles: xcd, xcd + 8, ...
+    const int both = nt / 2 * 2 * np;                 // blocks of those that go two at a time
+    if (sq >= nt * np) return;                        // whole block, before any barrier
+    const int in = sq < both ? sq % (2 * np) : (sq - both) * 2;
+    const int ptile = (sq < both ? sq / (2 * np) * 2 + (in & 1) : nt - 1) * 8 + xcd;
     int form;
     bool two;
     qf_pair(J.nform, J.ncos, in >> 1, &form, &two);
@@ -822,18 +824,21 @@ void k_qf_eta(QfJob J) {
     }
 }
 
-// Single-job launch: block -> (point tile, form) through the swizzle.
+// Single-job launch of nform x npt blocks: block -> (point tile, form) through
+// the swizzle, every block live.  Blocks go round-robin to the XCDs and there to
+// the shader engines, so that groups filled up with blocks that exit at once
+// leave the live ones on some of the engines only: 40 forms, 1008 components,
+// three products, 640 points 732 -> 231 us (NP 2), 3040 points 1330 -> 668 us
+// (NP 4), where 7680 points took 1630 us.
 template <int NLV, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_qf_forms_il(QfJob J, int npt) {
-    const int id = blockIdx.x;
-    const int per = kQfGF * kQfGP;
-    const int grp = id / per, in = id - grp * per;
-    const int nfg = (J.nform + kQfGF - 1) / kQfGF;
-    const int pg = grp / nfg, fg = grp - pg * nfg;
-    const int ptile = pg * kQfGP + in % kQfGP;
-    const int form = fg * kQfGF + in / kQfGP;
-    if (ptile >= npt || form >= J.nform) return;      // whole block, before any barrier
+    const int pg = (int)blockIdx.x / (J.nform * kQfGP);
+    const int rem = (int)blockIdx.x - pg * J.nform * kQfGP;
+    const int gp = min(kQfGP, npt - pg * kQfGP);      // point tiles of this group: 32, fewer in the last
+    const int fg = rem / (kQfGF * gp), in = rem - fg * kQfGF * gp;
+    const int ptile = pg * kQfGP + in % gp;
+    const int form = fg * kQfGF + in / gp;
     if (!J.clk) {
         qf_tile_il<NLV, NP>(J, ptile, form);
         return;
@@ -1033,15 +1038,17 @@ hipError_t launch_qf_forms(const QfJob& J, hipStream_t st) {
     // one product per term: form pairs where they give every CU a block
     if (J.nlv == 1 && J.ppad / 256 * qf_pairs(J.nform, J.ncos) >= 256) {
         const int np = (int)(J.ppad / 256);
-        hipLaunchKernelGGL(k_qf_pairs, dim3((unsigned)((np + 15) / 16 * 16 * qf_pairs(J.nform, J.ncos))), dim3(512), 0, st,
+        hipLaunchKernelGGL(k_qf_pairs, dim3((unsigned)((np + 7) / 8 * 8 * qf_pairs(J.nform, J.ncos))), dim3(512), 0, st,
                            J, np);
         return hipGetLastError();
     }
-    // 256-point tiles where they give every CU its two blocks, else 128
-    const bool wide = J.nlv == 3 && J.ppad / 256 * J.nform >= 512;
+    // 256-point tiles where they come to two and a half rounds of two blocks per
+    // CU, else 128-point ones, whose last round is shorter (40 forms, 1008
+    // components: 600 wide tiles 1001 us against 899, 1000 1680 against 1456,
+    // 1280 1628 against 1658; 320 components, 2560 458 against 478)
+    const bool wide = J.nlv == 3 && J.ppad / 256 * J.nform >= 1280;
     const int npt = (int)(wide ? J.ppad / 256 : (J.P + 127) / 128);
-    const int nfg = (J.nform + kQfGF - 1) / kQfGF, npg = (npt + kQfGP - 1) / kQfGP;
-    const unsigned nblk = (unsigned)((int64_t)nfg * npg * kQfGF * kQfGP);
+    const unsigned nblk = (unsigned)((int64_t)npt * J.nform);
     if (J.nlv == 1)
         hipLaunchKernelGGL((k_qf_forms_il<1, 2>), dim3(nblk), dim3(256), 0, st, J, npt);
     else if (wide)

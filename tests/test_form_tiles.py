@@ -67,3 +67,27 @@ def test_seas_along_x_leave_the_v_forms_out(prec, n, depth, nl):
     for f in ("ETA", "UX", "UZ"):
         assert np.array_equal(g[0].export(f), g[1].export(f)), f
     assert not np.any(g[0].export("UY"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["fp32", "bf16"])
+@pytest.mark.parametrize("nx,ny", [(8, 4), (32, 31), (33, 32), (41, 40), (56, 72), (64, 65), (64, 80), (90, 88)])
+def test_every_tile_of_a_launch(eng, mode, nx, ny):
+    """Every column of launches whose last group of point tiles is whole, short by
+    one, one tile or an odd one, of small and of wide tiles and of form pairs,
+    against the same columns in grids of 8 rows; bound as above."""
+    s = make_sea(40, 2.0, 8.0, 30.0, seed=nx, ndir=4).as_dict()
+    prec = eng.BF16 if mode == "bf16" else eng.FP32
+    sea = eng.Sea(s, precision=prec, with_direct=False)
+
+    def part(j0, j1):
+        return sea.grid((0.0, 6.0 * (nx - 1), 6.0 * j0, 6.0 * (j1 - 1)), nx, j1 - j0, 4, 0.0, 0.5, 0.7, 1.5, 30.0)
+    at = list(range(0, max(ny - 1, 1), 8))
+    rows = [part(j, k) for j, k in zip(at, at[1:] + [ny])]
+    big = part(0, ny)
+    assert big.qform_info()
+    for f, tail in (("ETA", ()), ("UX", (4,)), ("UY", (4,)), ("UZ", (4,))):
+        a = big.export(f).reshape((4, nx, ny) + tail)
+        b = np.concatenate([g.export(f).reshape((4, nx, -1) + tail) for g in rows], axis=2)
+        assert a.shape == b.shape
+        assert scaled_err(a.ravel(), b.ravel()) <= 1e-5, f
