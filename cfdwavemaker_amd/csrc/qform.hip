@@ -824,20 +824,24 @@ void k_qf_eta(QfJob J) {
     }
 }
 
-// Single-job launch of nform x npt blocks: block -> (point tile, form) through
-// the swizzle, every block live.  Blocks go round-robin to the XCDs and there to
+// Single-job launch: block -> (point tile, form) through the swizzle, without
+// idle blocks between live ones.  Blocks go round-robin to the XCDs and there to
 // the shader engines, so that groups filled up with blocks that exit at once
 // leave the live ones on some of the engines only: 40 forms, 1008 components,
 // three products, 640 points 732 -> 231 us (NP 2), 3040 points 1330 -> 668 us
 // (NP 4), where 7680 points took 1630 us.
 template <int NLV, int NP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_qf_forms_il(QfJob J, int npt) {
-    const int pg = (int)blockIdx.x / (J.nform * kQfGP);
-    const int rem = (int)blockIdx.x - pg * J.nform * kQfGP;
-    const int gp = min(kQfGP, npt - pg * kQfGP);      // point tiles of this group: 32, fewer in the last
+void k_qf_forms_il(QfJob J, int npt, int by_xcd) {
+    // the tiles this block's index runs over: all, or its XCD's (xcd, xcd + 8, ...)
+    const int x = by_xcd ? blockIdx.x & 7 : 0, st = by_xcd ? 8 : 1;
+    const int id = (int)blockIdx.x / st, nt = (npt - x + st - 1) / st, full = kQfGP / st;
+    const int pg = id / (J.nform * full);
+    const int rem = id - pg * J.nform * full;
+    const int gp = min(full, nt - pg * full);         // point tiles of this group, fewer in the last
+    if (gp <= 0 || rem >= gp * J.nform) return;       // whole block, before any barrier
     const int fg = rem / (kQfGF * gp), in = rem - fg * kQfGF * gp;
-    const int ptile = pg * kQfGP + in % gp;
+    const int ptile = (pg * full + in % gp) * st + x;
     const int form = fg * kQfGF + in / gp;
     if (!J.clk) {
         qf_tile_il<NLV, NP>(J, ptile, form);
@@ -1048,13 +1052,23 @@ hipError_t launch_qf_forms(const QfJob& J, hipStream_t st) {
     // 1280 1628 against 1658; 320 components, 2560 458 against 478)
     const bool wide = J.nlv == 3 && J.ppad / 256 * J.nform >= 1280;
     const int npt = (int)(wide ? J.ppad / 256 : (J.P + 127) / 128);
-    const unsigned nblk = (unsigned)((int64_t)npt * J.nform);
+    // An XCD that keeps its point tiles reads their Z operands through its own L2,
+    // but where 8 does not divide the tiles some XCDs have one fewer, else the
+    // tiles go block after block.  One product waits for the operands most: kept
+    // from 16 tiles on, if that adds under 30 % (23 forms, 1024 components, 25
+    // tiles 276 us against 329).  Three: kept up to 64 tiles, if it adds under
+    // 5 % (40 forms, 752 components, 61 tiles 1177 us against 1271; 1008
+    // components, 55 tiles 1552 against 1688, but 43 tiles 1320 against 1205, 70
+    // tiles 2061 against 1832).
+    const int npt8 = (npt + 7) / 8 * 8;
+    const int by_xcd = npt >= 16 && (J.nlv == 1 ? npt8 * 10 <= npt * 13 : npt <= 64 && npt8 * 20 <= npt * 21);
+    const unsigned nblk = (unsigned)((int64_t)(by_xcd ? npt8 : npt) * J.nform);
     if (J.nlv == 1)
-        hipLaunchKernelGGL((k_qf_forms_il<1, 2>), dim3(nblk), dim3(256), 0, st, J, npt);
+        hipLaunchKernelGGL((k_qf_forms_il<1, 2>), dim3(nblk), dim3(256), 0, st, J, npt, by_xcd);
     else if (wide)
-        hipLaunchKernelGGL((k_qf_forms_il<3, 4>), dim3(nblk), dim3(256), 0, st, J, npt);
+        hipLaunchKernelGGL((k_qf_forms_il<3, 4>), dim3(nblk), dim3(256), 0, st, J, npt, by_xcd);
     else
-        hipLaunchKernelGGL((k_qf_forms_il<3, 2>), dim3(nblk), dim3(256), 0, st, J, npt);
+        hipLaunchKernelGGL((k_qf_forms_il<3, 2>), dim3(nblk), dim3(256), 0, st, J, npt, by_xcd);
     return hipGetLastError();
 }
 
