@@ -611,16 +611,15 @@ __device__ __forceinline__ void qf_pair_tile(const QfJob& J, int ptile, int form
 // Blocks of an XCD (round-robin dispatch) walk the form pairs of two point
 // tiles together: the two tiles' Z operands stay in its L2 (1 MiB of hi parts
 // each at 1024 components), the tables stream through the last-level cache and
-// serve both tiles; the blocks of an odd last tile follow without gaps.  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
+// serve both tiles.  (An odd last tile's blocks numbered without idle ones
+// between took 4 % longer at 1024 components: 65,536 points, step 4.73 -> 4.93 ms.)  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
 // 32 point tiles, 89 GB one point tile at a time, 73 GB two at a time.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_qf_pairs(QfJob J, int npt) {
-    const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3, xcd = blockIdx.x & 7;
-    const int nt = (npt - xcd + 7) >> 3;              // this XCD's point tiles: xcd, xcd + 8, ...
-    const int both = nt / 2 * 2 * np;                 // blocks of those that go two at a time
-    if (sq >= nt * np) return;                        // whole block, before any barrier
-    const int in = sq < both ? sq % (2 * np) : (sq - both) * 2;
-    const int ptile = (sq < both ? sq / (2 * np) * 2 + (in & 1) : nt - 1) * 8 + xcd;
+    const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3;
+    const int in = sq % (2 * np);
+    const int ptile = (sq / (2 * np) * 2 + (in & 1)) * 8 + (blockIdx.x & 7);
+    if (ptile >= npt) return;                         // whole block, before any barrier
     int form;
     bool two;
     qf_pair(J.nform, J.ncos, in >> 1, &form, &two);
@@ -1042,7 +1041,7 @@ hipError_t launch_qf_forms(const QfJob& J, hipStream_t st) {
     // one product per term: form pairs where they give every CU a block
     if (J.nlv == 1 && J.ppad / 256 * qf_pairs(J.nform, J.ncos) >= 256) {
         const int np = (int)(J.ppad / 256);
-        hipLaunchKernelGGL(k_qf_pairs, dim3((unsigned)((np + 7) / 8 * 8 * qf_pairs(J.nform, J.ncos))), dim3(512), 0, st,
+        hipLaunchKernelGGL(k_qf_pairs, dim3((unsigned)((np + 15) / 16 * 16 * qf_pairs(J.nform, J.ncos))), dim3(512), 0, st,
                            J, np);
         return hipGetLastError();
     }
