@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(256) void k_levels_reduce(SeaDev<R> S, LevelJob<R> 
 // after every fill/update by k_grad_pack:
 //   column record (8 R): eta(tid1) eta(tid2) eta_t(tid1) eta_t(tid2) eta_x(0) eta_x(1) eta_y(0) eta_y(1)
 //   node records C and D (16 R each): for u, v, w in turn the piece f, f_x, f_y, f_s,
-//     then the piece u_t, v_t, w_t, pad;
+//     then the piece 0, u_t, v_t, w_t;
 //     C from time slot tid1 and derivative slot 0, D from tid2 and derivative slot 1.
 // Levels are the fastest index, so the corners l and l+1 of a query share a
 // cache line and one query touches 8 node lines instead of 8 x 30 arrays.
@@ -1076,10 +1076,10 @@ __global__ __launch_bounds__(256) void k_grad_pack(GradPack<R> J) {
             J.Fy[f][o * per + n] = r[4 * f + 2] = fd(F, (int64_t)sy, (int64_t)j, (int64_t)J.ny, J.dy);
             J.Fs[f][o * per + n] = r[4 * f + 3] = fd(F, (int64_t)1, (int64_t)m, (int64_t)J.nl, J.ds);
         }
-        dt(J.F[f], J.Ft[f], per, n, c[12 + f], d[12 + f]);
+        dt(J.F[f], J.Ft[f], per, n, c[13 + f], d[13 + f]);
     }
-    c[15] = 0;
-    d[15] = 0;
+    c[12] = 0;
+    d[12] = 0;
     store_rec<16>(J.pk_C + 16 * (int64_t)n, c);
     store_rec<16>(J.pk_D + 16 * (int64_t)n, d);
     if (m == 0) {
@@ -1185,13 +1185,6 @@ __device__ __forceinline__ Herm4<R> herm_w(R u, R d) {
     const R v = (R)1 - u, w = u * v, e = w * (v - u);
     return {v + e, u - e, d * (w * v), -(d * (w * u))};
 }
-// the same for one lane of the quad: lane 3 interpolates linearly
-template <typename R>
-__device__ __forceinline__ Herm4<R> quad_w(R u, R d, bool lin3) {
-    Herm4<R> w = herm_w(u, d);
-    if (lin3) w = {(R)1 - u, u, (R)0, (R)0};
-    return w;
-}
 template <typename R>
 __device__ __forceinline__ R herm4(const Herm4<R>& w, R f0, R f1, R d0, R d1) {
     return w.a * f0 + w.b * f1 + w.c * d0 + w.d * d1;
@@ -1199,13 +1192,15 @@ __device__ __forceinline__ R herm4(const Herm4<R>& w, R f0, R f1, R d0, R d1) {
 
 // x, y and s stages of spline_interp_velo (lsgrid_spline.cpp:386-502) of one
 // query on one time slot's records, this lane's piece: S[0] is the field's
-// value (lanes 0-2), S[0..2] the three d/dt (lane 3).  Byte offsets of this
+// value (lanes 0-2), S[1..3] the three d/dt (lane 3: places that no other
+// place of a piece enters, so that a field that is not a number, such as w over
+// water too deep for coth(k h), leaves the others alone).  Byte offsets of this
 // lane's piece at level 0 of the cell's columns (i, j), (i, j + 1), (i + 1, j),
 // (i + 1, j + 1) in col, levels l and lp (both edge clamped,
 // lsgrid_spline.cpp:375-384).
 // O: 32-bit byte offsets for packed slots below 4 GiB, else 64-bit ones.
 template <typename O, typename R>
-__device__ __forceinline__ void quad_slot(R (&S)[3], const R* __restrict__ pk, const O (&col)[4], int l, int lp,
+__device__ __forceinline__ void quad_slot(R (&S)[4], const R* __restrict__ pk, const O (&col)[4], int l, int lp,
                                           const Herm4<R>& wx, const Herm4<R>& wy, const Herm4<R>& ws, R xd,
                                           R yd, R sd) {
     R Y[2][4];
@@ -1227,8 +1222,8 @@ __device__ __forceinline__ void quad_slot(R (&S)[3], const R* __restrict__ pk, c
         for (int k = 1; k < 4; ++k) Y[lv][k] = lin(X[0][k], X[1][k], yd);
     }
     S[0] = herm4(ws, Y[0][0], Y[1][0], Y[0][3], Y[1][3]);
-    S[1] = lin(Y[0][1], Y[1][1], sd);
-    S[2] = lin(Y[0][2], Y[1][2], sd);
+#pragma unroll
+    for (int k = 1; k < 4; ++k) S[k] = lin(Y[0][k], Y[1][k], sd);
 }
 
 // A query's cell and the fractions in it, held by its own lane.
@@ -1241,20 +1236,19 @@ struct QueryCell {
 template <int Q, typename O, typename R>
 __device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, const R* __restrict__ pkC,
                                            const R* __restrict__ pkD, int nl, int piece, R dx, R dy, R ds, R dt) {
-    const bool lin3 = piece == 3;
     const O per = (O)nl * (O)(16 * sizeof(R));
     const O c00 = (O)quad_bc<Q>(C.c00) * per + (O)(piece * 4 * sizeof(R));
     const O dj = (O)quad_bc<Q>(C.dj) * per, di = (O)quad_bc<Q>(C.di) * per;
     const O col[4] = {c00, c00 + dj, c00 + di, c00 + di + dj};
     const R xd = quad_bc<Q>(C.xd), yd = quad_bc<Q>(C.yd), s0 = quad_bc<Q>(C.s0), s1 = quad_bc<Q>(C.s1);
     const int l0 = quad_bc<Q>(C.l0), l1 = quad_bc<Q>(C.l1);
-    const Herm4<R> wx = quad_w(xd, dx, lin3), wy = quad_w(yd, dy, lin3);
-    R A[3], B[3];
-    quad_slot<O>(A, pkC, col, l0, min(l0 + 1, nl - 1), wx, wy, quad_w(s0, ds, lin3), xd, yd, s0);
-    quad_slot<O>(B, pkD, col, l1, min(l1 + 1, nl - 1), wx, wy, quad_w(s1, ds, lin3), xd, yd, s1);
+    const Herm4<R> wx = herm_w(xd, dx), wy = herm_w(yd, dy);
+    R A[4], B[4];
+    quad_slot<O>(A, pkC, col, l0, min(l0 + 1, nl - 1), wx, wy, herm_w(s0, ds), xd, yd, s0);
+    quad_slot<O>(B, pkD, col, l1, min(l1 + 1, nl - 1), wx, wy, herm_w(s1, ds), xd, yd, s1);
     // the t stage of lane f's field with lane 3's d/dt of that field
-    R ta = quad_bc<3>(A[0]), tb = quad_bc<3>(B[0]);
-    const R ta1 = quad_bc<3>(A[1]), tb1 = quad_bc<3>(B[1]), ta2 = quad_bc<3>(A[2]), tb2 = quad_bc<3>(B[2]);
+    R ta = quad_bc<3>(A[1]), tb = quad_bc<3>(B[1]);
+    const R ta1 = quad_bc<3>(A[2]), tb1 = quad_bc<3>(B[2]), ta2 = quad_bc<3>(A[3]), tb2 = quad_bc<3>(B[3]);
     if (piece == 1) { ta = ta1; tb = tb1; }
     if (piece == 2) { ta = ta2; tb = tb2; }
     const R r = herm4(herm_w(quad_bc<Q>(C.td), dt), A[0], B[0], ta, tb);
@@ -1274,9 +1268,11 @@ __device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, co
 // only in part; a register cap that gives more waves spills and loses.  Cell-
 // ordered blocks are dealt so that each XCD takes one contiguous range of them:
 // neighbouring cells then share an L2 (past L2 154 instead of 270 MB per 1e6
-// queries).
+// queries).  The wave bounds keep the scheduler from giving up loads in flight
+// for waves (1e6 queries of a resident grid: FP32 104 us, 114 left to itself; FP64 196).
 template <typename R, typename TQ, typename O>
-__global__ __launch_bounds__(256) void k_query(QueryJob<R, TQ> J, QueryConst K) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 3 : 1, sizeof(R) == 4 ? 3 : 2)))
+void k_query(QueryJob<R, TQ> J, QueryConst K) {
     int64_t blk = blockIdx.x;
     if (J.srec) {
         const int64_t per = gridDim.x >> 3;           // a multiple of 8 blocks (launch_query)

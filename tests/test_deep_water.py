@@ -1,0 +1,40 @@
+"""Seas with components of k h > 710: coth(k h) there is not a number in FP64,
+and with it the vertical Taylor gradient and the s-grid's w.  Everything that
+does not contain it stays as good as in shallower water."""
+import numpy as np
+import pytest
+
+from cfdwavemaker_amd.seastate import make_sea, wavenumber
+
+pytestmark = pytest.mark.gpu
+DEPTH = 1000.0
+
+
+def _sea(n=24, theta=None):
+    s = make_sea(n, 3.0, 9.0, DEPTH, seed=n, ndir=1).as_dict()
+    s["omega"] = np.linspace(0.4, 3.0, n)
+    s["k"] = wavenumber(s["omega"], DEPTH)
+    assert np.max(s["k"]) * DEPTH > 710.0
+    s["theta"] = np.full(n, 0.4) if theta is None else theta
+    return s
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_query_of_u_and_v_beside_a_w_that_is_no_number(prec):
+    """At a node of the bed level and the time of the grid's first slot the
+    interpolation is the node value itself (FP32: but for the rounding of the
+    depth map, the library's 2e-5 of the field); elsewhere it is finite."""
+    from cfdwavemaker_amd import engine as eng
+    sea = eng.Sea(_sea(), precision=eng.FP64 if prec == "fp64" else eng.FP32, with_direct=False)
+    nx, ny, nl = 6, 5, 7
+    g = sea.grid((0.0, 50.0, 0.0, 40.0), nx, ny, nl, 0.0, 0.5, 0.7, 1.5, DEPTH)
+    node = {f: g.export(f).reshape(4, nx, ny, nl)[1, :, :, 0].ravel() for f in ("UX", "UY", "UZ")}
+    assert np.all(np.isnan(node["UZ"])) and np.all(np.isfinite(node["UX"])) and np.any(node["UX"])
+    x, y = (a.ravel() for a in np.meshgrid(10.0 * np.arange(nx), 10.0 * np.arange(ny), indexing="ij"))
+    q = g.query(0.0, x, y, -DEPTH)
+    for k, f in ((1, "UX"), (2, "UY")):
+        tol = 0.0 if prec == "fp64" else 2e-5 * np.max(np.abs(g.export(f)))
+        assert np.max(np.abs(q[:, k] - node[f])) <= tol, f
+    rng = np.random.default_rng(1)
+    q = g.query(rng.uniform(0, 0.5, 300), rng.uniform(-5, 55, 300), rng.uniform(-5, 45, 300), rng.uniform(-DEPTH, 1, 300))
+    assert np.all(np.isfinite(q[:, :3])) and np.all(np.isnan(q[:, 3]))
