@@ -181,15 +181,18 @@ __device__ __attribute__((noinline)) PairSum<R> pairs_one_by_one(const PhaseRec*
 // the point's outputs from its totals
 __device__ __forceinline__ void point_store(const PointJob& J, int64_t q, const double* a) {
     const double z = J.z[q];
-    const double z1 = (J.flags & EV_TAYLOR) && z - J.swl > 0. ? z - J.swl : 0.;
+    const double z1 = z - J.swl > 0. ? z - J.swl : 0.;
+    // (without the Taylor terms their gradients, which deep water may leave
+    // without a value, stay out)
+    const bool tay = (J.flags & EV_TAYLOR) != 0;
     if (J.o_eta1) J.o_eta1[q] = a[0];
     if (J.o_eta2) J.o_eta2[q] = J.want_eta2 ? a[1] : 0.;
     for (int k = 0; k < 4; ++k)
         if (J.o_g[k]) J.o_g[k][q] = a[2 + k];
-    if (J.o_u) J.o_u[q] = a[6] + a[2] * z1;
-    if (J.o_v) J.o_v[q] = a[7] + a[3] * z1;
-    if (J.o_w) J.o_w[q] = a[8] + a[4] * z1;
-    if (J.o_p) J.o_p[q] = a[9] + J.rho * a[10] + a[5] * z1;
+    if (J.o_u) J.o_u[q] = a[6] + (tay ? a[2] * z1 : 0.);
+    if (J.o_v) J.o_v[q] = a[7] + (tay ? a[3] * z1 : 0.);
+    if (J.o_w) J.o_w[q] = a[8] + (tay ? a[4] * z1 : 0.);
+    if (J.o_p) J.o_p[q] = a[9] + J.rho * a[10] + (tay ? a[5] * z1 : 0.);
 }
 
 template <typename R>

@@ -38,3 +38,22 @@ def test_query_of_u_and_v_beside_a_w_that_is_no_number(prec):
     rng = np.random.default_rng(1)
     q = g.query(rng.uniform(0, 0.5, 300), rng.uniform(-5, 55, 300), rng.uniform(-5, 45, 300), rng.uniform(-DEPTH, 1, 300))
     assert np.all(np.isfinite(q[:, :3])) and np.all(np.isnan(q[:, 3]))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_points_without_taylor_terms(prec):
+    """The second-order members (no Taylor terms asked for) of a long-crested sea
+    against the pair loop, which the same sea takes with its components in
+    descending order.  Tolerance: FP64 rounding of sums over 276 pairs; FP32
+    terms good to a few ulps, at most 24 in a chain."""
+    from cfdwavemaker_amd import engine as eng
+    s = _sea()
+    r = dict(s, **{k: np.asarray(s[k])[::-1].copy() for k in ("omega", "A", "k", "phase", "theta")})
+    a = eng.Sea(s, precision=eng.FP64 if prec == "fp64" else eng.FP32)
+    b = eng.Sea(r)
+    rng = np.random.default_rng(2)
+    q = rng.uniform(0, 40, 90), rng.uniform(-60, 90, 90), rng.uniform(-30, 30, 90), rng.uniform(-30.0, 0.0, 90)
+    for kind in ("u2", "w2"):
+        g, ref = a.eval(kind, *q), b.eval(kind, *q)
+        assert np.all(np.isfinite(ref)) and np.any(ref)
+        assert np.max(np.abs(g - ref)) <= (1e-11 if prec == "fp64" else 1e-5) * np.max(np.abs(ref)), kind
