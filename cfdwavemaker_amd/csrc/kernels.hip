@@ -630,11 +630,20 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
     if constexpr (LB) {
         lb_component_sums<LRM>(S, J, sg.own_lo, sg.own_hi, dxp, dyp, t, ri_f8, lin, secf, LU, LV, LW, gxr, gyr, gzr);
     }
+    // The depth nodes (J.qd) carry the pair sums down to the bed.  A trough below
+    // the bed puts its column's levels there as well, where the interpolation
+    // would run away from the profiles: such waves walk the pairs of their own rows.
+    bool below = false;
+    if constexpr (GRID && sizeof(R) == 8) {
+#pragma unroll
+        for (int l = 0; l < LC; ++l) below = below || zp[l] < -J.qd_h * (1. + 1e-9);
+        below = J.qd && __any(below);
+    }
     for (int i = ia; !LB && i < ib; ++i) {
         const bool own = i >= sg.own_lo && i < sg.own_hi;
         const bool sec = secf && (direct || (sizeof(R) == 4 ? row_active(S.rowActive, i) : S.rowActive[i] != 0));
         // (form-assisted fills, F8, launch only with the forms: no pair rows)
-        const bool prs = F8 == 0 && sec && !(GRID && (J.qf || J.qd)) && i >= sg.rlo && i < sg.rhi;
+        const bool prs = F8 == 0 && sec && (below ? own : !(GRID && (J.qf || J.qd)) && i >= sg.rlo && i < sg.rhi);
         if (!own && !prs) continue;
         const PhaseRec pi = ld_rec<R>(S.ph, i);
         const CompRec<R> c = ld_rec<R>(S.cr, i);
@@ -725,7 +734,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
         }
         if (prs) {
             // pair terms, m in [m0, m1)
-            const int m0 = i == sg.rlo ? sg.mstart : i + 1;
+            const int m0 = i == sg.rlo && !below ? sg.mstart : i + 1;
             const int m1 = i == sg.rhi - 1 ? sg.mend : (direct ? S.n : S.fmhi[i]);
             const int64_t base = (direct ? S.drow[i] : S.frow[i]) - (i + 1);
             const UvwRec<R>* __restrict__ rr = tab + base;
@@ -889,7 +898,7 @@ __device__ __forceinline__ void levels_body(const SeaDev<R>& S, const LevelJob<R
         }
     }
     if constexpr (GRID && sizeof(R) == 8) {
-        if (J.qd && blockIdx.y == 0) {
+        if (J.qd && !below && blockIdx.y == 0) {
             // pair sums from the depth nodes: sum_s w_s Q_s / (xi - xi_s) over
             // sum_s w_s / (xi - xi_s); a level on a node takes that node's
             // value through a weight of 1e290

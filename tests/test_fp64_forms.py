@@ -76,3 +76,24 @@ def test_components_ramped_apart_take_the_pair_loop(eng, oracle):
     g, o = eng.Sea(s, with_direct=False).grid(*args), oracle.sea(s).grid(*args)
     for f in ("ETA", "UX", "UZ"):
         assert scaled_err(g.export(f), o.export(f)) <= TOL, f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nseg", ["", "1", "5"])
+def test_troughs_below_the_bed(eng, oracle, nseg, monkeypatch):
+    """Waves far too high for the depth: columns whose elevation lies below the
+    bed have levels there, past the depth nodes; their neighbours do not."""
+    if nseg:
+        monkeypatch.setenv("CFDWM_NSEG", nseg)
+    s = make_sea(30, 9.0, 8.0, 6.0, seed=3, ndir=2).as_dict()
+    args = ((0.0, 600.0, 0.0, 60.0), 41, 12, 9, 1.0, 0.5, 0.7, 1.5, s["depth"])
+    o = oracle.sea(s).grid(*args)
+    eta = o.export("ETA")
+    assert 20 < np.sum(eta < -1.05 * s["depth"]) < 0.3 * eta.size
+    g = eng.Sea(s, with_direct=False).grid(*args)
+    for step in range(2):
+        if step:
+            g.force_update(1.6)
+            o.force_update(1.6)
+        for f in ("ETA", "UX", "UY", "UZ"):
+            assert scaled_err(g.export(f), o.export(f)) <= TOL, (step, f)
