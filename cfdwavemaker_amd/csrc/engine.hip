@@ -271,6 +271,25 @@ int Sea::point_build() {
     return 0;
 }
 
+// A pair table on the device in the working precision.
+template <typename R>
+int Sea::put_table(const PairTable& P, DevBuf& row, DevBuf* mhi, DevBuf& uvw, DevBuf& xr) {
+    hipStream_t st = Engine::get().stream();
+    const int64_t ne = (int64_t)P.rec.size();
+    std::vector<UvwRec<R>> u(ne > 0 ? ne : 1);
+    std::vector<XRec<R>> x(ne > 0 ? ne : 1);
+    for (int64_t e = 0; e < ne; ++e) {
+        u[e] = uvw_rec<R>(P.rec[e], tab.in.depth);
+        x[e] = XRec<R>{(R)P.rec[e].xP, (R)P.rec[e].xM};
+    }
+    if (row.upload(P.rowoff.data(), P.rowoff.size() * sizeof(int64_t), st)) return -3;
+    if (mhi && mhi->upload(P.mhi.data(), P.mhi.size() * sizeof(int32_t), st)) return -3;
+    if (uvw.upload(u.data(), u.size() * sizeof(UvwRec<R>), st)) return -3;
+    if (xr.upload(x.data(), x.size() * sizeof(XRec<R>), st)) return -3;
+    CFDWM_HIP(hipStreamSynchronize(st));       // host staging vectors go out of scope
+    return 0;
+}
+
 template <typename R>
 int Sea::upload_t(bool with_direct) {
     Engine& E = Engine::get();
@@ -289,25 +308,8 @@ int Sea::upload_t(bool with_direct) {
     if (ph_.upload(ph.data(), ph.size() * sizeof(PhaseRec), st)) return -3;
     if (cr_.upload(cr.data(), cr.size() * sizeof(CompRec<R>), st)) return -3;
     if (act_.upload(act.data(), act.size(), st)) return -3;
-    auto put_table = [&](const PairTable& P, bool eta, DevBuf& row, DevBuf* mhi, DevBuf& uvw, DevBuf& xr) -> int {
-        const int64_t ne = (int64_t)P.rec.size();
-        std::vector<UvwRec<R>> u(ne > 0 ? ne : 1);
-        std::vector<XRec<R>> x(ne > 0 ? ne : 1);
-        for (int64_t e = 0; e < ne; ++e) {
-            u[e] = uvw_rec<R>(P.rec[e], h);
-            x[e] = XRec<R>{(R)P.rec[e].xP, (R)P.rec[e].xM};
-        }
-        (void)eta;
-        if (row.upload(P.rowoff.data(), P.rowoff.size() * sizeof(int64_t), st)) return -3;
-        if (mhi && mhi->upload(P.mhi.data(), P.mhi.size() * sizeof(int32_t), st)) return -3;
-        if (uvw.upload(u.data(), u.size() * sizeof(UvwRec<R>), st)) return -3;
-        if (xr.upload(x.data(), x.size() * sizeof(XRec<R>), st)) return -3;
-        CFDWM_HIP(hipStreamSynchronize(st));   // host staging vectors go out of scope
-        return 0;
-    };
-    if (put_table(tab.filt, true, frow_, &fmhi_, fuvw_, fx_)) return -3;
+    if (put_table<R>(tab.filt, frow_, &fmhi_, fuvw_, fx_)) return -3;
     if (with_direct && long_crested(tab) && point_build<R>()) return -3;
-    if (with_direct && !pt_.steps && put_table(tab.direct, false, drow_, nullptr, duvw_, dx_)) return -3;
     SeaDev<R> d{};
     d.n = N;
     d.h = h; d.swl = tab.in.swl; d.x0 = tab.in.x0; d.y0 = tab.in.y0; d.rho = tab.in.rho;
@@ -318,13 +320,22 @@ int Sea::upload_t(bool with_direct) {
     d.fmhi = (const int32_t*)fmhi_.get();
     d.fuvw = (const UvwRec<R>*)fuvw_.get();
     d.fx = (const XRec<R>*)fx_.get();
-    d.drow = (const int64_t*)drow_.get();
-    d.duvw = (const UvwRec<R>*)duvw_.get();
-    d.dx = (const XRec<R>*)dx_.get();
     if constexpr (sizeof(R) == 8) d64_ = d; else d32_ = d;
+    if (with_direct && !pt_.steps && direct_upload()) return -3;
     CFDWM_HIP(hipStreamSynchronize(st));
     return 0;
 }
+
+template <typename R>
+int Sea::direct_upload_t(SeaDev<R>& d) {
+    if (d.drow) return 0;
+    if (put_table<R>(tab.direct, drow_, nullptr, duvw_, dx_)) return -3;
+    d.duvw = (const UvwRec<R>*)duvw_.get();
+    d.dx = (const XRec<R>*)dx_.get();
+    d.drow = (const int64_t*)drow_.get();
+    return 0;
+}
+int Sea::direct_upload() { return prec == kFP32 ? direct_upload_t(d32_) : direct_upload_t(d64_); }
 
 int Sea::upload(bool with_direct) {
     if (int e = Engine::get().init()) return e;
@@ -669,14 +680,19 @@ int64_t qf_chunk_cap(int npad) {
     return std::max<int64_t>(kQfTile, ((int64_t)1 << 31) / ((int64_t)npad * 8) / kQfTile * kQfTile);
 }
 
+// CFDWM_QFORM=0: point batches take the pair loops
+bool qform_on() {
+    const char* e = std::getenv("CFDWM_QFORM");
+    return !e || std::atoi(e) != 0;
+}
+
 // FP32 point batches: the filtered eta2 pair sum as the MFMA quadratic form
 // (form 0 of the sea's tables) when the batch is large and every component
 // has the same frequency-ramp triple (the ramp factor is then one number per
 // point, applied by the column kernel).  Returns 1 when used.
 int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, const double* dt, bool want_eta2,
                      ColumnJob<float>& J) {
-    const char* e = std::getenv("CFDWM_QFORM");
-    if (!want_eta2 || n < 2048 || (e && std::atoi(e) == 0) || s.nfilt() == 0) return 0;
+    if (!want_eta2 || n < 2048 || !qform_on() || s.nfilt() == 0) return 0;
     const CompTable& c = s.tab.comp;
     for (int i = 1; i < c.n; ++i)
         if (c.rt[i] != c.rt[0] || c.ts[i] != c.ts[0] || c.du[i] != c.du[0]) return 0;
@@ -886,7 +902,10 @@ int Sea::eval_points(int64_t n, const double* x, const double* y, const double* 
         else CFDWM_HIP(hipMemsetAsync(b + 2 * n, 0, n * sizeof(double), st));
         dx = b; dy = b + n; dz = b + 2 * n; dt = b + 3 * n;
     }
-    const PointTables* pf = want_lev && !smit && (flags & EV_SEC) && (flags & EV_DIRECT) ? point_tables() : nullptr;
+    const PointTables* pf =
+        want_lev && !smit && (flags & EV_SEC) && (flags & EV_DIRECT) && qform_on() ? point_tables() : nullptr;
+    // (a sea with point tables gets the pair loop's on the first call that asks for it)
+    if (!pf && want_lev && !smit && (flags & EV_DIRECT) && direct_upload()) return -3;
     double* const user[10] = {eta1, eta2, grads4, grads4 ? grads4 + n : nullptr,
                               grads4 ? grads4 + 2 * n : nullptr, grads4 ? grads4 + 3 * n : nullptr, u, v, w, p};
     if (pf && device_ptrs && !overlap(n, {x, y, z, t}, user)) {

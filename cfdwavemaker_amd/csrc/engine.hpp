@@ -437,6 +437,12 @@ private:
     PointTables pt_;
     template <typename R>
     int point_build();
+    template <typename R>
+    int put_table(const PairTable& P, DevBuf& row, DevBuf* mhi, DevBuf& uvw, DevBuf& xr);
+    // the unfiltered pair loop's tables, where they are not on the device yet
+    template <typename R>
+    int direct_upload_t(SeaDev<R>& d);
+    int direct_upload();
     std::map<std::pair<bool, int>, std::unique_ptr<DevBuf>> seg_cache_;
     std::map<int, std::unique_ptr<DevBuf>> cseg_cache_;
     std::unique_ptr<QfTables> qf_;

@@ -163,3 +163,32 @@ def test_eta2_beside_the_pair_loop(eng, prec, n, ndir, m):
     for k in ("eta1", "eta2"):
         x, y = a[k].cpu().numpy(), b[k].cpu().numpy()
         assert np.max(np.abs(x - y)) <= TOL[prec] * np.max(np.abs(y)), k
+
+
+def _kernels(eng, call):
+    """The launches of a call, by the library's own timers."""
+    eng.prof_enable(True)
+    eng.prof_read()
+    try:
+        return call(), set(eng.prof_read())
+    finally:
+        eng.prof_enable(False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 2, 40])
+def test_switched_off(eng, prec, n, monkeypatch):
+    """CFDWM_QFORM=0 at the call takes the pair loop of the same sea (whose tables
+    then go up), without it the forms again."""
+    s, q = _sea(n, 30.0), _points(70, 30.0, 9)
+    sea = eng.Sea(s, precision=eng.FP64 if prec == "fp64" else eng.FP32)
+    a, ka = _kernels(eng, lambda: _fields(eng, sea, q))
+    monkeypatch.setenv("CFDWM_QFORM", "0")
+    b, kb = _kernels(eng, lambda: _fields(eng, sea, q))
+    monkeypatch.delenv("CFDWM_QFORM")
+    c, kc = _kernels(eng, lambda: _fields(eng, sea, q))
+    assert "k_point_forms" in ka and "k_point_forms" in kc
+    assert "k_levels_points" in kb and "k_point_forms" not in kb
+    _check(a, b, TOL[prec])
+    assert all(np.array_equal(a[k], c[k]) for k in FIELDS)
