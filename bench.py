@@ -766,7 +766,19 @@ def main():
     q_ms, q_n = prof.get("k_query", (float("nan"), 1))
     q_ms += prof.get("k_query_sort", (0.0, 1))[0]
     qfi = grid.qform_info()
-    if qfi is not None:
+    if qfi is not None and qfi["products"] == 0:
+        # FP64: every form at the depth nodes on the FP64 matrix cores; algorithmic
+        # work as below, 32 N^2 per column-slot
+        alg = 32.0 * len(s["omega"]) ** 2 * 4 * NX * NY
+        t_f = prof.get("k_qd_forms", (float("nan"), 1))[0] / a.steps * 1e-3
+        roof = {"bound": "mfma", "kernel": "k_qd_forms (all launches of a fill)", "achieved": alg / t_f / 1e12,
+                "peak": PEAK["fp64"] / 1e12, "unit": "TFLOP/s", "frac": alg / t_f / PEAK["fp64"], "traffic": None,
+                "avg_launch_ms": t_f * 1e3, "flop_per_launch": alg,
+                "flop_rule": "32 N^2 per column-slot (eta2, u, v, w forms x 2 (2N)^2)",
+                "exec_flop_per_launch": qfi["mfma_flop"], "exec_achieved": qfi["mfma_flop"] / t_f / 1e12,
+                "exec_frac": qfi["mfma_flop"] / t_f / PEAK["fp64"], "exec_over_alg": qfi["mfma_flop"] / alg,
+                "forms": qfi["nform"], "depth_nodes": qfi["rank"], "depth_basis_err": qfi["basis_err"]}
+    elif qfi is not None:
         # dominant kernel: the second-order velocity pair sums as bf16 MFMA
         # quadratic forms (the launch k_qf_forms times; with one bf16 product
         # per term, k_qf_forms_eta times the separate three-product eta2 launch).

@@ -1213,6 +1213,11 @@ int cfdwm_grid_qform_mode(cfdwm_grid* grid, int* products, double* basis_tol, in
     if (!grid) { set_error("bad arguments"); return -1; }
     const Grid& g = *grid->g;
     if (reason) *reason = g.qf_skip;
+    if (g.qf_used && g.sea->prec != kFP32) {       // FP64 products, profiles exact at the depth nodes
+        if (products) *products = 0;
+        if (basis_tol) *basis_tol = 4e-15;
+        return 1;
+    }
     const Sea::QfTables* T = nullptr;
     if (g.qf_used && g.sea->qform_tables(&T) == 1) {
         if (products) *products = T->nlv;

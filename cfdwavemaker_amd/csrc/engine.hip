@@ -1355,7 +1355,14 @@ int Grid::qform_fill(int nslot, const double* slot_t, int64_t ncol, const int32_
 
 int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<double>& C,
                   LevelJob<double>& L) {
-    if (!qform_ || sea->nfilt() == 0 || ncol <= 0) return 0;
+    qf_used = false;
+    qf_clock_valid_ = false;
+    qf_skip = QF_OFF;
+    if (!qform_) return 0;
+    qf_skip = QF_NO_PAIRS;
+    if (sea->nfilt() == 0) return 0;
+    qf_skip = QF_FP64;
+    if (ncol <= 0) return 0;
     // a fill of few points is over in the pair loop (split over pair segments)
     // before the forms' few waves have walked their tables: one update at 1024
     // components takes 4.1 ms in the pair loop against 5.3 at 1024 points, 6.1
@@ -1367,13 +1374,19 @@ int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* 
         // one ramp factor for all components at a slot's time
         scale[s] = freq_ramp_host(slot_t[s], c.rt[0], c.ts[0], c.du[0]);
         for (int i = 1; i < c.n; ++i)
-            if (freq_ramp_host(slot_t[s], c.rt[i], c.ts[i], c.du[i]) != scale[s]) return 0;
+            if (freq_ramp_host(slot_t[s], c.rt[i], c.ts[i], c.du[i]) != scale[s]) {
+                qf_skip = QF_RAMPS;
+                return 0;
+            }
     }
     // the nodes span [-depth of the sea, 0]
+    qf_skip = QF_DEPTH;
     if (g.h > sea->tab.in.depth) return 0;
     int rc = 0;
+    qf_skip = QF_BASIS;
     const Sea::QdMeta* M = sea->qd_meta(&rc);
     if (!M) return rc;
+    qf_skip = QF_FP64;
     const int npad = M->npad, S = M->S, nf = M->nf, nform = 1 + nf * S;
     if (npad > 4096) return 0;                    // a node's tables would exceed 768 MiB
     const int64_t P = (int64_t)nslot * ncol;
@@ -1431,6 +1444,18 @@ int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* 
     L.qd_a = M->a;
     L.qd_h = sea->tab.in.depth;
     for (int s = 0; s < 4; ++s) C.q2scale[s] = L.qf_scale[s] = scale[s];
+    qf_used = true;
+    qf_skip = QF_USED;
+    qf_nlv = 0;
+    qf_nform = nform;
+    qf_rank = qf_rank_w = S;
+    qf_rank_v = nf == 3 ? S : 0;
+    qf_basis_err = M->err;
+    // executed MFMA flops: 64-row tiles of i, each from its first row to its
+    // kend, a cosine and a sine product, for every padded point and form
+    qf_flop = 0;
+    for (size_t q = 0; q < M->kend_h.size(); ++q)
+        qf_flop += 64.0 * std::max(0, M->kend_h[q] - (int)(64 * q)) * 2 * 2 * (double)ppad_all * nform;
     return 1;
 }
 

@@ -204,7 +204,8 @@ class Grid:
         check(self.L.cfdwm_grid_release_workspace(self.h), "cfdwm_grid_release_workspace")
 
     def qform_info(self):
-        """Quadratic forms of the last fill: None when the pair loop ran."""
+        """Quadratic forms of the last fill: None when the pair loop ran
+        (FP64: products 0, rank the number of depth nodes)."""
         nf, rk = C.c_int(), C.c_int()
         fl, er = C.c_double(), C.c_double()
         used = self.L.cfdwm_grid_qform_info(self.h, C.byref(nf), C.byref(rk), C.byref(fl), C.byref(er))

@@ -246,21 +246,23 @@ CFDWM_EXPORT int cfdwm_grid_query_device_f32_noalloc(cfdwm_grid* grid, int64_t n
  * query instead of four scattered 4-byte stores. */
 CFDWM_EXPORT int cfdwm_grid_kinematics_device_f32(cfdwm_grid* grid, int64_t n, double t, const float* x,
                                                   const float* y, const float* z, float* out4);
-/* Second-order quadratic forms of the last FP32 fill (no reference
- * counterpart: measurement hook).  Returns 1 when the fill ran the pair sums
- * as MFMA quadratic forms (then nform, the depth-basis rank, the executed MFMA
- * flops of that fill and the basis' max error are filled in), 0 when it ran
- * the pair loop. */
+/* Second-order quadratic forms of the last fill (no reference counterpart:
+ * measurement hook).  Returns 1 when the fill ran the pair sums as MFMA
+ * quadratic forms (then nform, the depth-basis rank (FP64: depth nodes), the
+ * executed MFMA flops of that fill and the basis' max error are filled in), 0
+ * when it ran the pair loop. */
 CFDWM_EXPORT int cfdwm_grid_qform_info(cfdwm_grid* grid, int* nform, int* rank, double* mfma_flop,
                                        double* basis_err);
 /* Product mode of the last fill's quadratic forms (no reference
- * counterpart): bf16 products per term (3: hi/lo split, 1: hi only), the
- * depth-basis tolerance, and why the forms were or were not used: 0 used,
- * 1 FP64 sea, 2 switched off (CFDWM_QFORM=0), 3 no second-order pairs,
- * 4 frequency ramps differ between components at a slot time, 5 grid depth
- * beyond the depth basis, 6 no depth basis within the tolerance (the last
- * three print a one-time warning: the pair loop is much slower).  Returns 1
- * when that fill used the forms, else 0 (products and tolerance 0). */
+ * counterpart): bf16 products per term (3: hi/lo split, 1: hi only, 0: FP64
+ * products), the depth-basis tolerance, and why the forms were or were not
+ * used: 0 used, 1 an FP64 fill of too few points for its components, more than
+ * 4096 components or no memory for the workspace, 2 switched off
+ * (CFDWM_QFORM=0), 3 no second-order pairs, 4 frequency ramps differ between
+ * components at a slot time, 5 grid depth beyond the depth basis, 6 no depth
+ * basis within the tolerance (in FP32 and bf16 the last three print a one-time
+ * warning: the pair loop is much slower).  Returns 1 when that fill used the
+ * forms, else 0 (products and tolerance 0). */
 CFDWM_EXPORT int cfdwm_grid_qform_mode(cfdwm_grid* grid, int* products, double* basis_tol, int* reason);
 /* Shader clock of the MFMA form launches (no reference counterpart: a
  * measurement aid).  Writes the mean shader clock in MHz over the blocks of

@@ -97,3 +97,30 @@ def test_troughs_below_the_bed(eng, oracle, nseg, monkeypatch):
             o.force_update(1.6)
         for f in ("ETA", "UX", "UY", "UZ"):
             assert scaled_err(g.export(f), o.export(f)) <= TOL, (step, f)
+
+
+@pytest.mark.gpu
+def test_report_of_the_route(eng, monkeypatch):
+    """Forms used, with what they took, or why not."""
+    def grid(s, nx=32, depth=None):
+        return eng.Sea(s, with_direct=False).grid((0.0, 100.0, 0.0, 60.0), nx, 16, 4, 0.5, 0.5, 0.7, 1.5,
+                                                  depth or s["depth"])
+    s = make_sea(12, 3.0, 9.0, 40.0, seed=5, ndir=2).as_dict()
+    g = grid(s)
+    info = g.qform_info()
+    assert g.qform_reason() == "used" and info["products"] == 0
+    assert info["nform"] == 1 + 3 * info["rank"] and info["basis_err"] <= 4e-15
+    # 24 components in one 64-row tile up to 32, 2048 points, a cosine and a sine product
+    assert info["mfma_flop"] == 64 * 32 * 4 * 2048 * info["nform"]
+    few = grid(s, nx=1)                      # 256 points and levels: the pair loop up to 128
+    assert few.qform_reason() == "used"
+    small = eng.Sea(s, with_direct=False).grid((0.0, 9.0, 0.0, 9.0), 2, 2, 4, 0.5, 0.5, 0.7, 1.5, 40.0)
+    assert small.qform_info() is None and small.qform_reason() == "fp64"
+    assert grid(s, depth=41.0).qform_reason() == "grid deeper than the depth basis"
+    r = dict(s, ramptime=np.linspace(1, 4, 24), starttime=np.zeros(24), duration=np.full(24, 1e6))
+    assert grid(r).qform_reason() == "frequency ramps differ"
+    one = make_sea(1, 3.0, 9.0, 40.0, seed=5).as_dict()
+    assert grid(one).qform_reason() == "no second-order pairs"
+    monkeypatch.setenv("CFDWM_QFORM", "0")
+    off = grid(s)
+    assert off.qform_info() is None and off.qform_reason() == "switched off"
