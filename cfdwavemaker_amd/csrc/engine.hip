@@ -1060,6 +1060,7 @@ int Grid::fill_slots(int nslot, const double* slot_t, const int* slot_dst, bool 
     C.nseg = pick_nseg(C.ncol * nslot, nrec);
     LevelJob<R> L;
     bool qf_used = false;
+    std::unique_lock<std::mutex> space;       // FP64 forms: their workspace, until the level pass is queued
     // every return below joins the side stream's velocity forms first
     struct Join {
         Grid* g;
@@ -1070,7 +1071,7 @@ int Grid::fill_slots(int nslot, const double* slot_t, const int* slot_dst, bool 
         if (rc < 0) return rc;
         qf_used = rc == 1;
     } else {
-        const int rc = qd_fill(nslot, slot_t, C.ncol, C.cols, C, L);
+        const int rc = qd_fill(nslot, slot_t, C.ncol, C.cols, C, L, space);
         if (rc < 0) return rc;
         qf_used = rc == 1;
     }
@@ -1354,7 +1355,7 @@ int Grid::qform_fill(int nslot, const double* slot_t, int64_t ncol, const int32_
 }
 
 int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<double>& C,
-                  LevelJob<double>& L) {
+                  LevelJob<double>& L, std::unique_lock<std::mutex>& space) {
     qf_used = false;
     qf_clock_valid_ = false;
     qf_skip = QF_OFF;
@@ -1391,15 +1392,17 @@ int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* 
     if (npad > 4096) return 0;                    // a node's tables would exceed 768 MiB
     const int64_t P = (int64_t)nslot * ncol;
     // workspace: at most 512 MiB of Z operands and 256 MiB of tables (or one
-    // node's); without the memory the pair loop runs
+    // node's), and the forms' values (121 at 40 nodes: 254 MB for 4 x 65,536
+    // points); without the memory the pair loop runs
     const int64_t ppad_all = (P + 63) / 64 * 64;
     const int64_t chunk = std::min(ppad_all, std::max<int64_t>(64, (int64_t(512) << 20) / (16LL * npad) / 64 * 64));
     const size_t zn = (size_t)chunk * npad, nn = (size_t)npad * npad;
     const int grp = (int)std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(256) << 20) / (int64_t)(2 * nf * nn * sizeof(double))));
-    if (!qout_.try_alloc((size_t)nform * ppad_all * sizeof(double))) return 0;
     if (!qd_space_) qd_space_ = Engine::get().qd_space();
-    std::lock_guard<std::mutex> lk(qd_space_->mu);
-    if (!qd_space_->z.try_alloc(2 * zn * sizeof(double)) || !qd_space_->tab.try_alloc((2 + 2 * nf * grp) * nn * sizeof(double)))
+    std::unique_lock<std::mutex> lk(qd_space_->mu);
+    if (!qd_space_->z.try_alloc(2 * zn * sizeof(double)) ||
+        !qd_space_->tab.try_alloc((2 + 2 * nf * grp) * nn * sizeof(double)) ||
+        !qd_space_->out.try_alloc((size_t)nform * ppad_all * sizeof(double)))
         return 0;
     const SeaDev<double>& D = sea->dev<double>();
     hipStream_t st = Engine::get().stream();
@@ -1412,7 +1415,7 @@ int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* 
     J.zs = J.zc + zn;
     J.b = (const double*)qd_space_->tab.get();
     J.kend = (const int32_t*)M->kend.get();
-    J.out = (double*)qout_.get();
+    J.out = (double*)qd_space_->out.get();
     J.ostride = ppad_all;
     J.nf = nf;
     QdBuild B;
@@ -1444,6 +1447,7 @@ int Grid::qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* 
     L.qd_a = M->a;
     L.qd_h = sea->tab.in.depth;
     for (int s = 0; s < 4; ++s) C.q2scale[s] = L.qf_scale[s] = scale[s];
+    space = std::move(lk);
     qf_used = true;
     qf_skip = QF_USED;
     qf_nlv = 0;

@@ -266,14 +266,15 @@ struct KernelTimes {
     int64_t count = 0;
 };
 
-// Workspace of the FP64 forms: Z operands of one chunk of points and the
-// tables of one group of forms, both rebuilt by every fill.  One for all
-// grids: work on the library stream runs in order, and mu is held while a
-// fill's launches are queued, so that fills from several threads do not
-// interleave.  The grids that used it hold it; it is freed with the last.
+// Workspace of the FP64 forms: Z operands of one chunk of points, the tables
+// of one group of forms and the forms' values at all points, rebuilt by every
+// fill.  One for all grids, as large as the largest needs: work on the library
+// stream runs in order, and mu is held while a fill's launches are queued, so
+// that fills from several threads do not interleave.  The grids that used it
+// hold it; it is freed with the last, or when they have released it.
 struct QdSpace {
     std::mutex mu;
-    DevBuf z, tab;
+    DevBuf z, tab, out;
 };
 
 class Engine {
@@ -575,7 +576,7 @@ private:
     // the FP64 forms of a fill: 1 when they ran, 0 when the pair loop has to, < 0 on error
     std::shared_ptr<QdSpace> qd_space_;
     int qd_fill(int nslot, const double* slot_t, int64_t ncol, const int32_t* cols, ColumnJob<double>& C,
-                LevelJob<double>& L);
+                LevelJob<double>& L, std::unique_lock<std::mutex>& space);
     void init_slot_times(double* tt) const;
 public:
     // batched refill over many grids (refill_batched)

@@ -344,7 +344,8 @@ CFDWM_EXPORT int cfdwm_lsgrid_write_vtu(cfdwm_lsgrid* grid, const char* path, in
 CFDWM_EXPORT int cfdwm_lsgrid_set_vtk(cfdwm_lsgrid* grid, int on, const char* dir, const char* prefix,
                                       const char* time_label);
 /* Free the sea's form tables, the grid's operand workspace (rebuilt on the
- * next FP32 fill) and its query-ordering buffers (rebuilt by the next batch of
+ * next fill; that of FP64 fills is shared and goes with the last grid that
+ * holds it) and its query-ordering buffers (rebuilt by the next batch of
  * 65,536 or more queries); the grid's fields are kept. */
 CFDWM_EXPORT int cfdwm_grid_release_workspace(cfdwm_grid* grid);
 CFDWM_EXPORT int cfdwm_grids_refill_batched(cfdwm_grid** grids, int n, double budget_gb, int release,

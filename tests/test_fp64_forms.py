@@ -124,3 +124,36 @@ def test_report_of_the_route(eng, monkeypatch):
     monkeypatch.setenv("CFDWM_QFORM", "0")
     off = grid(s)
     assert off.qform_info() is None and off.qform_reason() == "switched off"
+
+
+@pytest.mark.gpu
+def test_one_workspace_for_all_grids(eng, monkeypatch):
+    """A grid's fields take the same memory with the forms as without, whatever
+    the number of grids; the workspace goes when all have released it."""
+    import torch
+    s = make_sea(12, 3.0, 9.0, 40.0, seed=5, ndir=2).as_dict()
+
+    def grids(n):
+        return [eng.Sea(s, with_direct=False).grid((0.0, 999.0, 0.0, 999.0), 160, 160, 2, 0.0, 0.5, 0.7, 1.5, 40.0)
+                for _ in range(n)]
+
+    def used(n):
+        torch.cuda.synchronize()
+        a = torch.cuda.mem_get_info()[0]
+        g = grids(n)
+        return g, a - torch.cuda.mem_get_info()[0]
+    monkeypatch.setenv("CFDWM_QFORM", "0")
+    loop, plain = used(4)
+    monkeypatch.delenv("CFDWM_QFORM")
+    first = grids(1)
+    values = first[0].qform_info()["nform"] * 4 * 160 * 160 * 8
+    assert values > 40 << 20
+    more, forms = used(4)
+    assert forms < plain + values // 2
+    free = torch.cuda.mem_get_info()[0]
+    for g in first + more:
+        g.release_workspace()
+    assert torch.cuda.mem_get_info()[0] - free >= values
+    more[0].refill()
+    assert all(np.array_equal(more[0].export(f), first[0].export(f)) for f in ("ETA", "UX", "UY", "UZ"))
+    assert scaled_err(more[0].export("UX"), loop[0].export("UX")) <= TOL
