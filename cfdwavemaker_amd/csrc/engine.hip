@@ -738,16 +738,17 @@ int points_eta2_form(Sea& s, int64_t n, const double* dx, const double* dy, cons
 // Segments of a point-forms launch: about equal shares of the table's steps,
 // the count that needs the fewest steps in sequence over the rounds of
 // resident blocks (three a CU in FP32, two in FP64, by their registers), each
-// row block entered counted as four steps more.
+// row block entered counted as four steps more.  Several segments' totals take
+// kPointPartial at most (the sea keeps them), and save 3 % of the steps or more.
+constexpr int64_t kPointRec = 11 * sizeof(double), kPointPartial = int64_t(256) << 20;
 int point_segments(int64_t n, int steps, bool fp32) {
     if (const char* e = std::getenv("CFDWM_NSEG")) return std::max(1, std::min(std::atoi(e), steps));
     const int64_t tiles = (n + 63) / 64, slots = fp32 ? 768 : 512;
+    const int most = (int)std::min<int64_t>({128, steps / 4, kPointPartial / (n * kPointRec)});
+    auto cost = [&](int s) { return (double)((tiles * s + slots - 1) / slots) * ((double)steps / s + 8.); };
     int best = 1;
-    double cost = 0.;
-    for (int s = 1; s <= std::min(128, std::max(1, steps / 4)); ++s) {
-        const double c = (double)((tiles * s + slots - 1) / slots) * ((double)steps / s + 8.);
-        if (s == 1 || c < cost) { best = s; cost = c; }
-    }
+    for (int s = 2; s <= most; ++s)
+        if (cost(s) < cost(best) && cost(s) <= 0.97 * cost(1)) best = s;
     return best;
 }
 
@@ -763,16 +764,14 @@ int run_point_forms(Sea& s, const Sea::PointTables& T, int64_t n, const double* 
     J.flags = flags;
     J.want_eta2 = want_eta2 ? 1 : 0;
     J.steps = T.steps;
-    J.nseg = point_segments(n, T.steps, sizeof(R) == 4);
+    J.nseg = point_segments(J.n, T.steps, sizeof(R) == 4);
     J.coef = T.coef.get();
     J.mr = (const PointRec*)T.rec.get();
+    if (J.nseg > 1 && !s.partial.try_alloc((size_t)J.nseg * J.n * kPointRec)) J.nseg = 1;
+    if (J.nseg > 1) J.partial = (double*)s.partial.get();
     J.o_eta1 = out[0]; J.o_eta2 = out[1];
     for (int k = 0; k < 4; ++k) J.o_g[k] = out[2 + k];
     J.o_u = out[6]; J.o_v = out[7]; J.o_w = out[8]; J.o_p = out[9];
-    if (J.nseg > 1) {
-        if (s.partial.alloc((size_t)J.nseg * n * 11 * sizeof(double))) return -3;
-        J.partial = (double*)s.partial.get();
-    }
     PROF("k_point_forms", launch_point_forms<R>(s.dev<R>(), J, Engine::get().stream()));
     return 0;
 }

@@ -192,3 +192,28 @@ def test_switched_off(eng, prec, n, monkeypatch):
     assert "k_levels_points" in kb and "k_point_forms" not in kb
     _check(a, b, TOL[prec])
     assert all(np.array_equal(a[k], c[k]) for k in FIELDS)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m", [(512, 400_000), (1024, 3_000_000)])
+def test_memory_of_large_batches(eng, n, m):
+    """The segments' totals stay within 256 MiB (2 MiB for the allocator's granules),
+    and the result is that of small batches, which split the pairs otherwise."""
+    import torch
+    s = _sea(n, 30.0)
+    sea = eng.Sea(s, precision=eng.FP32)
+    t, x, y, z = (torch.tensor(a, device="cuda") for a in _points(m, 30.0, 10))
+    u = torch.zeros(m, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+
+    def call(a, b, out):
+        eng.check(sea.L.cfdwm_eval_fields(sea.h, b - a, *(v[a:].data_ptr() for v in (t, x, y, z)), None, None,
+                                          out.data_ptr(), None, None, None, 1), "cfdwm_eval_fields")
+    call(0, m, u)
+    assert free - torch.cuda.mem_get_info()[0] <= (256 + 2) << 20
+    part = torch.zeros(2000, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    for a in (0, m - 2000):
+        call(a, a + 2000, part)
+        assert float((part - u[a:a + 2000]).abs().max()) <= TOL["fp32"] * float(u.abs().max())
