@@ -754,11 +754,13 @@ int point_segments(int64_t n, int steps, bool fp32) {
 
 // Long-crested seas: every output of the call from one pass over the pairs.
 // out: eta1, eta2, the four gradients, u, v, w, p (null: not asked for).
+// At most kPointChunk points a launch (four threads each; a launch holds 2^32).
+constexpr int64_t kPointChunk = int64_t(1) << 28;
 template <typename R>
 int run_point_forms(Sea& s, const Sea::PointTables& T, int64_t n, const double* dx, const double* dy, const double* dz,
                     const double* dt, uint32_t flags, bool want_eta2, double* const* out) {
     PointJob J;
-    J.n = n; J.x = dx; J.y = dy; J.z = dz; J.t = dt;
+    J.n = std::min(n, kPointChunk);
     J.cth = T.cth; J.sth = T.sth;
     J.kmax = s.tab.kmax; J.swl = s.tab.in.swl; J.rho = s.tab.in.rho;
     J.flags = flags;
@@ -769,10 +771,15 @@ int run_point_forms(Sea& s, const Sea::PointTables& T, int64_t n, const double* 
     J.mr = (const PointRec*)T.rec.get();
     if (J.nseg > 1 && !s.partial.try_alloc((size_t)J.nseg * J.n * kPointRec)) J.nseg = 1;
     if (J.nseg > 1) J.partial = (double*)s.partial.get();
-    J.o_eta1 = out[0]; J.o_eta2 = out[1];
-    for (int k = 0; k < 4; ++k) J.o_g[k] = out[2 + k];
-    J.o_u = out[6]; J.o_v = out[7]; J.o_w = out[8]; J.o_p = out[9];
-    PROF("k_point_forms", launch_point_forms<R>(s.dev<R>(), J, Engine::get().stream()));
+    for (int64_t q = 0; q < n; q += kPointChunk) {
+        auto at = [&](double* p) { return p ? p + q : nullptr; };
+        J.n = std::min(n - q, kPointChunk);
+        J.x = dx + q; J.y = dy + q; J.z = dz + q; J.t = dt + q;
+        J.o_eta1 = at(out[0]); J.o_eta2 = at(out[1]);
+        for (int k = 0; k < 4; ++k) J.o_g[k] = at(out[2 + k]);
+        J.o_u = at(out[6]); J.o_v = at(out[7]); J.o_w = at(out[8]); J.o_p = at(out[9]);
+        PROF("k_point_forms", launch_point_forms<R>(s.dev<R>(), J, Engine::get().stream()));
+    }
     return 0;
 }
 

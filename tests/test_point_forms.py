@@ -217,3 +217,22 @@ def test_memory_of_large_batches(eng, n, m):
     for a in (0, m - 2000):
         call(a, a + 2000, part)
         assert float((part - u[a:a + 2000]).abs().max()) <= TOL["fp32"] * float(u.abs().max())
+
+
+@pytest.mark.gpu
+def test_more_points_than_a_launch_holds(eng):
+    """2^30 points and some: four threads a point are more than a launch's 2^32.
+    One array serves as t, x, y and z."""
+    import torch
+    n = (1 << 30) + 100
+    q = torch.linspace(0.0, 30.0, n, dtype=torch.float64, device="cuda")
+    u = torch.full((n,), 1e30, dtype=torch.float64, device="cuda")
+    sea = eng.Sea(_sea(2, 30.0), precision=eng.FP32)
+    p = q.data_ptr()
+    torch.cuda.synchronize()
+    eng.check(sea.L.cfdwm_eval_fields(sea.h, n, p, p, p, p, None, None, u.data_ptr(), None, None, None, 1),
+              "cfdwm_eval_fields")
+    for a in (0, (1 << 28) - 50, (1 << 29) - 50, n - 100):
+        v = sea.eval_fields_device(*[q[a:a + 100].contiguous()] * 4)["u"]
+        assert float(v.abs().max()) > 0 and torch.equal(v, u[a:a + 100]), a
+    assert float(u.max()) < 1e29
