@@ -173,7 +173,9 @@ template <typename R, typename TQ>
 hipError_t launch_query(const QueryJob<R, TQ>& J, hipStream_t st);
 // Cell order of a query batch (qsort.hip): recs receives (x, y, z, p) of every
 // query p, grouped by tiles of neighbouring columns; counts holds
-// query_bins_bytes bytes of scratch.
+// query_bins_bytes bytes of scratch: at most kQueryBins tiles counted by at most
+// kQueryBinBlocks blocks, and the tiles' totals.
+constexpr int kQueryBins = 16384, kQueryBinBlocks = 256;
 size_t query_bins_bytes(int64_t n, int nx, int ny);
 template <typename TQ>
 hipError_t launch_query_bins(int64_t n, const GridGeom& g, const TQ* x, const TQ* y, const TQ* z, uint32_t* counts,

@@ -19,8 +19,11 @@
 namespace cfdwm {
 
 namespace {
-constexpr size_t kScratchBytes = size_t(64) << 20;     // 64 MiB per GPU
-constexpr int64_t kMaxQueries = 1115336;               // the entry's limit; their buffers take 34 MiB at most
+// the entry's limit, and what its ordering buffers take on the grid of most
+// tiles: counts and totals, then records (33.1 MiB)
+constexpr int64_t kMaxQueries = 1115336;
+constexpr size_t kScratchBytes = (size_t)(kQueryBinBlocks + 1) * kQueryBins * sizeof(uint32_t) +
+                                 ((size_t)kMaxQueries * sizeof(QRec<float>) + 255) / 256 * 256;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -57,15 +60,13 @@ int query_device_f32_noalloc(Grid& grid, int64_t n, double t, const float* x, co
                              float* eta, float* u, float* v, float* w) {
     if (n <= 0) return 0;
     if (int e = Engine::get().init()) return e;
-    const size_t need = query_ws_bytes<float>(n, grid.g.nx, grid.g.ny);
-    if (n > kMaxQueries || need > kScratchBytes) {
+    if (n > kMaxQueries) {
         set_error("allocation-free query: " + std::to_string(n) + " queries exceed the maximum of " +
-                  std::to_string(kMaxQueries) + " for this grid (" + std::to_string(kScratchBytes >> 20) +
-                  " MiB of device scratch)");
+                  std::to_string(kMaxQueries));
         return -1;
     }
     void* ws = nullptr;
-    if (need > 0)
+    if (query_ws_bytes<float>(n, grid.g.nx, grid.g.ny) > 0)
         if (int e = scratch_address(&ws)) return e;
     return grid.query_device_f32(n, t, x, y, z, eta, u, v, w, nullptr, ws, kScratchBytes);
 }

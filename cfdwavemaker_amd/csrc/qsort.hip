@@ -27,7 +27,7 @@ namespace cfdwm {
 
 namespace {
 
-constexpr int kBinThreads = 1024, kMaxBins = 16384, kMaxBinBlocks = 256;
+constexpr int kBinThreads = 1024, kMaxBins = kQueryBins, kMaxBinBlocks = kQueryBinBlocks;
 
 // Tiles of 2^shift x 2^shift columns, and the blocks' share of the queries.
 struct BinPlan {

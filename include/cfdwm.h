@@ -231,10 +231,10 @@ CFDWM_EXPORT int cfdwm_grid_query_device_f32(cfdwm_grid* grid, int64_t n, double
  * the reference): for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, kernels and results; the cell-ordering buffers of batches of
- * 65,536 queries or more live in a fixed 64 MiB device array per GPU (held
+ * 65,536 queries or more live in a fixed device array of 34 MiB per GPU (held
  * until the process ends) instead of the grid's own buffers, so the call makes
- * no device allocation.  A batch whose ordering buffers exceed the array
- * (about a million queries) returns -1 with the maximum in the message.  All
+ * no device allocation.  More than 1,115,336 queries are refused: -1 with the
+ * maximum in the message, whatever the grid.  All
  * calls share the GPU's array and are serialised on the library stream; work
  * on other streams that overlaps one of them must not use it. */
 CFDWM_EXPORT int cfdwm_grid_query_device_f32_noalloc(cfdwm_grid* grid, int64_t n, double t, const float* x,

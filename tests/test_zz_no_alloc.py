@@ -73,3 +73,26 @@ def test_noalloc_query_refuses_oversized_batch():
     assert rc == -1
     msg = last_error()
     assert "exceed the maximum" in msg, msg
+
+
+@pytest.mark.parametrize("nx,ny", [(128, 128), (129, 130), (1, 1)])
+def test_noalloc_query_at_its_limit(nx, ny):
+    """1,115,336 queries run, also where they take every tile (16,384) and block of
+    the ordering, as the allocating query's; one more is refused on every grid."""
+    import torch
+    from cfdwavemaker_amd import engine
+    from cfdwavemaker_amd.seastate import make_sea
+    L = _lib()
+    limit = 1_115_336
+    sea = engine.Sea(make_sea(6, 1.0, 8.0, 20.0, seed=1).as_dict(), precision=engine.FP32, with_direct=False)
+    grid = sea.grid((0.0, 2.0 * (nx - 1), 0.0, 2.0 * (ny - 1)), nx, ny, 2, 0.0, 0.5, 0.7, 1.5, 20.0)
+    x, y, z = _queries(torch, limit + 1, 4, 256.0)
+    ref, got = (torch.zeros((4, limit + 1), dtype=torch.float32, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    grid.query_device_f32(limit, 0.3, x.data_ptr(), y.data_ptr(), z.data_ptr(), *[o.data_ptr() for o in ref])
+    args = x.data_ptr(), y.data_ptr(), z.data_ptr(), *[o.data_ptr() for o in got]
+    assert L.cfdwm_grid_query_device_f32_noalloc(grid.h, limit, 0.3, *args) == 0, last_error()
+    engine.sync()
+    assert torch.equal(got, ref) and float(ref[1].abs().max()) > 0
+    assert L.cfdwm_grid_query_device_f32_noalloc(grid.h, limit + 1, 0.3, *args) == -1
+    assert last_error().endswith("exceed the maximum of 1115336")
