@@ -1184,19 +1184,21 @@ __device__ __forceinline__ double quad_bc(double v) {
     return __hiloint2double(quad_bc<Q>(__double2hiint(v)), quad_bc<Q>(__double2loint(v)));
 }
 
-// herm(f0, f1, d f0' - (f1 - f0), -d f1' + (f1 - f0), u) as weights of f0, f1, f0', f1'
+// herm(f0, f1, d f0' - (f1 - f0), -d f1' + (f1 - f0), u) as f0 and weights of
+// f1 - f0, f0', f1' (weights of f0 and f1 themselves would carry their own
+// rounding, of the size of f, into every stage)
 template <typename R>
-struct Herm4 {
-    R a, b, c, d;
+struct Herm3 {
+    R b, c, d;
 };
 template <typename R>
-__device__ __forceinline__ Herm4<R> herm_w(R u, R d) {
-    const R v = (R)1 - u, w = u * v, e = w * (v - u);
-    return {v + e, u - e, d * (w * v), -(d * (w * u))};
+__device__ __forceinline__ Herm3<R> herm_w(R u, R d) {
+    const R v = (R)1 - u, w = u * v;
+    return {u - w * (v - u), d * (w * v), -(d * (w * u))};
 }
 template <typename R>
-__device__ __forceinline__ R herm4(const Herm4<R>& w, R f0, R f1, R d0, R d1) {
-    return w.a * f0 + w.b * f1 + w.c * d0 + w.d * d1;
+__device__ __forceinline__ R herm3(const Herm3<R>& w, R f0, R f1, R d0, R d1) {
+    return f0 + (w.b * (f1 - f0) + (w.c * d0 + w.d * d1));
 }
 
 // x, y and s stages of spline_interp_velo (lsgrid_spline.cpp:386-502) of one
@@ -1210,7 +1212,7 @@ __device__ __forceinline__ R herm4(const Herm4<R>& w, R f0, R f1, R d0, R d1) {
 // O: 32-bit byte offsets for packed slots below 4 GiB, else 64-bit ones.
 template <typename O, typename R>
 __device__ __forceinline__ void quad_slot(R (&S)[4], const R* __restrict__ pk, const O (&col)[4], int l, int lp,
-                                          const Herm4<R>& wx, const Herm4<R>& wy, const Herm4<R>& ws, R xd,
+                                          const Herm3<R>& wx, const Herm3<R>& wy, const Herm3<R>& ws, R xd,
                                           R yd, R sd) {
     R Y[2][4];
 #pragma unroll
@@ -1222,15 +1224,15 @@ __device__ __forceinline__ void quad_slot(R (&S)[4], const R* __restrict__ pk, c
             R a[4], b[4];
             load_rec(a, reinterpret_cast<const R*>(reinterpret_cast<const char*>(pk) + (O)(col[jj] + lo)));
             load_rec(b, reinterpret_cast<const R*>(reinterpret_cast<const char*>(pk) + (O)(col[2 + jj] + lo)));
-            X[jj][0] = herm4(wx, a[0], b[0], a[1], b[1]);
+            X[jj][0] = herm3(wx, a[0], b[0], a[1], b[1]);
 #pragma unroll
             for (int k = 1; k < 4; ++k) X[jj][k] = lin(a[k], b[k], xd);
         }
-        Y[lv][0] = herm4(wy, X[0][0], X[1][0], X[0][2], X[1][2]);
+        Y[lv][0] = herm3(wy, X[0][0], X[1][0], X[0][2], X[1][2]);
 #pragma unroll
         for (int k = 1; k < 4; ++k) Y[lv][k] = lin(X[0][k], X[1][k], yd);
     }
-    S[0] = herm4(ws, Y[0][0], Y[1][0], Y[0][3], Y[1][3]);
+    S[0] = herm3(ws, Y[0][0], Y[1][0], Y[0][3], Y[1][3]);
 #pragma unroll
     for (int k = 1; k < 4; ++k) S[k] = lin(Y[0][k], Y[1][k], sd);
 }
@@ -1251,7 +1253,7 @@ __device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, co
     const O col[4] = {c00, c00 + dj, c00 + di, c00 + di + dj};
     const R xd = quad_bc<Q>(C.xd), yd = quad_bc<Q>(C.yd), s0 = quad_bc<Q>(C.s0), s1 = quad_bc<Q>(C.s1);
     const int l0 = quad_bc<Q>(C.l0), l1 = quad_bc<Q>(C.l1);
-    const Herm4<R> wx = herm_w(xd, dx), wy = herm_w(yd, dy);
+    const Herm3<R> wx = herm_w(xd, dx), wy = herm_w(yd, dy);
     R A[4], B[4];
     quad_slot<O>(A, pkC, col, l0, min(l0 + 1, nl - 1), wx, wy, herm_w(s0, ds), xd, yd, s0);
     quad_slot<O>(B, pkD, col, l1, min(l1 + 1, nl - 1), wx, wy, herm_w(s1, ds), xd, yd, s1);
@@ -1260,7 +1262,8 @@ __device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, co
     const R ta1 = quad_bc<3>(A[2]), tb1 = quad_bc<3>(B[2]), ta2 = quad_bc<3>(A[3]), tb2 = quad_bc<3>(B[3]);
     if (piece == 1) { ta = ta1; tb = tb1; }
     if (piece == 2) { ta = ta2; tb = tb2; }
-    const R r = herm4(herm_w(quad_bc<Q>(C.td), dt), A[0], B[0], ta, tb);
+    const R df = B[0] - A[0];
+    const R r = herm(A[0], B[0], dt * ta - df, df - dt * tb, quad_bc<Q>(C.td));
     const R u = quad_bc<0>(r), v = quad_bc<1>(r), w = quad_bc<2>(r);
     if (piece == Q) { ov[0] = u; ov[1] = v; ov[2] = w; }
 }
