@@ -1127,10 +1127,9 @@ __device__ __forceinline__ double cart2sigmaS(double zpt, double e, double h, do
 }
 
 // The same map in FP32 for FP32 grids (k_query<float, .>): divisions by the
-// grid constants become products with their reciprocals, pow the hardware's
-// 2^(b log2 x) (x in [0, tanab]: its relative error grows only where the result
-// is small), atan the FP32 library function.  The sigma coordinate then carries
-// a few 1e-7 of absolute error, far below the FP32 grid values' own.
+// grid constants become products with their reciprocals, pow and atan the FP32
+// library functions.  The sigma coordinate then carries a few 1e-7 of absolute
+// error, far below the FP32 grid values' own.
 struct QueryConst {
     double inv_dx, inv_dy, inv_dt;     // 1 / dx, 1 / dy, 1 / dt
     float h, swl, tanab;               // the FP64 map's depth, swl and tanab
@@ -1141,7 +1140,7 @@ __device__ __forceinline__ float cart2sigmaS_f(float zpt, float e, const QueryCo
     float sigma = (z - (e - K.swl)) / (K.h + (e - K.swl));
     sigma = sigma < -1.f ? -1.f : sigma;
     sigma = sigma > 0.f ? 0.f : sigma;
-    return 1.f - atanf(__builtin_amdgcn_exp2f(K.itb * __builtin_amdgcn_logf(-sigma * K.tanab))) * K.ita;
+    return 1.f - atanf(powf(-sigma * K.tanab, K.itb)) * K.ita;
 }
 
 // A packed record of N values (N a multiple of 4) at a 16-byte aligned
