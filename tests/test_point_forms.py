@@ -236,3 +236,25 @@ def test_more_points_than_a_launch_holds(eng):
         v = sea.eval_fields_device(*[q[a:a + 100].contiguous()] * 4)["u"]
         assert float(v.abs().max()) > 0 and torch.equal(v, u[a:a + 100]), a
     assert float(u.max()) < 1e29
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_one_component_against_the_oracle(eng, oracle, prec):
+    """No pairs: the linear, diagonal and pressure terms alone (test_against_the_pair_loop's
+    other sea of one component takes the point forms as well)."""
+    s, (t, x, y, z) = _sea(1, 20.0), _points(40, 20.0, 11)
+    sea, o = eng.Sea(s, precision=eng.FP64 if prec == "fp64" else eng.FP32), oracle.sea(s)
+    for kind in ("eta1", "eta2", "u", "v", "w", "dp"):
+        g, r = sea.eval(kind, t, x, y, z), o.eval(kind, t, x, y, z)
+        assert np.max(np.abs(g - r)) <= TOL[prec] * np.max(np.abs(r)), kind
+
+
+@pytest.mark.gpu
+def test_long_chains(eng, monkeypatch):
+    """512 components in FP32: up to 512 terms in a row in an accumulator, four times
+    those of TOL, whose roundings add up as their square root."""
+    s, q = _sea(512, 30.0), _points(300, 30.0, 12)
+    got = _fields(eng, eng.Sea(s, precision=eng.FP32), q)
+    monkeypatch.setenv("CFDWM_QFORM", "0")
+    _check(got, _fields(eng, eng.Sea(s), q), 2 * TOL["fp32"])
