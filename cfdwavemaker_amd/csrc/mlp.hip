@@ -129,7 +129,7 @@ __device__ __forceinline__ void mm_store(const MmArgs& a, const f32x16& acc, flo
 // 33-256-256-256-65 network, 0.21 ms now (products 11 to 13 us each).
 template <bool AK, bool BK>
 __device__ __forceinline__ void mm_tile(const MmArgs& a, int bx, int by, int bz) {
-    constexpr int KS = 64, LS = KS + 8;                        // LDS row stride in bf16 (80 bytes: no bank conflicts at 16 bytes)
+    constexpr int KS = 64, LS = KS + 8;                        // LDS row stride in bf16 (144 bytes: rows start 4 banks apart, no conflicts at 16 bytes)
     __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][64 * LS];
     uint16_t(*As)[64 * LS] = lds[0], (*Bs)[64 * LS] = lds[1];
     float* T = reinterpret_cast<float*>(lds);     // 64 x 68 floats in the end

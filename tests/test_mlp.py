@@ -176,3 +176,32 @@ def test_gradient_of_many_layers(nh):
             a, b = g[q:q + sz], gr[q:q + sz]
             assert np.linalg.norm(a - b) <= 5e-4 * np.linalg.norm(b), (d, o, sz)
             q += sz
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nin,width,nout,n", [(63, 65, 64, 127), (64, 63, 65, 129), (65, 64, 63, 128), (127, 129, 1, 2049),
+                                              (1, 128, 127, 2111), (193, 191, 65, 4161)])
+def test_gradient_at_edges_of_64_wide_k_steps(nin, width, nout, n):
+    """As test_gradient_at_tile_and_chunk_edges for the 64-wide k steps of the
+    products, in the layer widths (63, 64, 65, 127 ...) and in the rows of a
+    weight gradient's chunk (a whole number of steps, one row more, one less,
+    and chunks whose last one is a remainder); the same tolerance."""
+    import torch
+    from cfdwavemaker_amd.mlp import Mlp
+    dims, p = _net(nin, width, 2, nout, 20)
+    X, Y, norm = _data(n, nin, nout, 21)
+    X, Y = X.astype(np.float32), Y.astype(np.float32)
+    m = Mlp(nin, width, 2, nout)
+    m.set_params(p)
+    m.set_norm(*norm)
+    loss, g = m.loss_grad(torch.tensor(X, device="cuda"), torch.tensor(Y, device="cuda"))
+    m.close()
+    normf = tuple(np.asarray(a, np.float32).astype(np.float64) for a in norm)
+    lr, gr = mlp_ref.loss_grad(p, dims, X, Y, normf, "bf16")
+    assert abs(loss - lr) <= 1e-4 * lr
+    q = 0
+    for d, o in dims:
+        for sz in (d * o, o):
+            a, b = g[q:q + sz], gr[q:q + sz]
+            assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), (d, o, sz)
+            q += sz
