@@ -86,12 +86,12 @@ struct SeaTables {
 };
 
 // Runs body(i) for i in [0, n) on the host cores (rows have uneven cost:
-// rows are handed out one at a time).
+// rows are handed out one at a time), on most threads, or (0) by the row count.
 template <typename F>
-void parallel_rows(int n, F body, int serial_below = 64) {
+void parallel_rows(int n, F body, unsigned most = 0) {
     unsigned nt = std::thread::hardware_concurrency();
     nt = std::max(1u, std::min(nt, 16u));
-    if (n < serial_below) nt = 1;
+    if (most ? most < nt : n < 64) nt = std::max(1u, most);
     std::atomic<int> next(0);
     auto work = [&]() {
         for (int i = next++; i < n; i = next++) body(i);
