@@ -347,13 +347,14 @@ def batched_leg(nstates: int, prec_name: str, err_cols: int = 4) -> dict:
         if (st + 1) % 128 == 0:
             print(f"[bench] batched: {st + 1}/{nstates} seas set up", file=sys.stderr, flush=True)
     t_setup = time.perf_counter() - t0
-    # first call: the tuner times its candidate launch shapes on the first
-    # group of each product mode (and the call fills every grid)
+    # first call: the host builds the depth bases of the states (the larger
+    # part), the tuner times its candidate launch shapes on the first group of
+    # each product mode, and the call fills every grid
     t1 = time.perf_counter()
     tune = engine.refill_batched(grids, release=True)
     engine.sync()
     t_first = time.perf_counter() - t1
-    print(f"[bench] batched: first call (tuning) {t_first:.2f} s", file=sys.stderr, flush=True)
+    print(f"[bench] batched: first call (depth bases, tuning) {t_first:.2f} s", file=sys.stderr, flush=True)
     t1 = time.perf_counter()
     stats = engine.refill_batched(grids, release=True)
     engine.sync()

@@ -210,11 +210,14 @@ UvwRec<R> uvw_rec(const PairRec64& p, double h) {
 }
 
 // Seas whose unfiltered pair sums at points go through the point forms run in
-// one direction with k ascending: there the pair profiles split.  At every size
-// measured the forms win (pair loop -> forms: 256 components, 4,096 points FP64
-// 1330 -> 184 us; 512 components, 131,072 points FP32 31.9 -> 6.9 ms; 48
-// components, 16 points 131 -> 39 us FP64, 101 -> 36 us FP32).  Directional
-// seas keep the pair loop: |k_i + k_m| has no such split.
+// one direction with k ascending: there the pair profiles split.  At depths to
+// 150 m the forms win at every size measured (pair loop -> forms: 256
+// components, 4,096 points FP64 1330 -> 184 us; 512 components, 131,072 points
+// FP32 31.9 -> 6.9 ms; 48 components, 16 points 131 -> 39 us FP64, 101 -> 36 us
+// FP32).  In deeper water more and more of their waves go pair by pair
+// (points.hip), which takes between a quarter of the pair loop's time and 1.14
+// of it (48 components FP32, 65,536 points, 500 m and deeper).  Directional seas keep
+// the pair loop: |k_i + k_m| has no such split.
 bool long_crested(const SeaTables& T) {
     for (int i = 1; i < T.comp.n; ++i)
         if (T.in.theta[i] != T.in.theta[0] || !(T.comp.k[i] >= T.comp.k[i - 1])) return false;

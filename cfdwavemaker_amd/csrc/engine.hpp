@@ -406,7 +406,7 @@ public:
     void release_qform();
     // FP64: the depth nodes of this sea's profiles and the tile ends of its
     // pair table (built once); null when no node set of at most 64 reaches
-    // rounding (kmax h beyond about 600), or on a device error (*rc < 0)
+    // rounding (kmax h beyond about 1600), or on a device error (*rc < 0)
     struct QdMeta {
         int npad = 0, S = 0, nf = 3;         // nf 2: every v coefficient is zero (a sea along x)
         double a = 0, err = 0;

@@ -1144,8 +1144,9 @@ __device__ __forceinline__ float cart2sigmaS_f(float zpt, float e, const QueryCo
 }
 
 // A packed record of N values (N a multiple of 4) at a 16-byte aligned
-// address, loaded as 16-byte vectors.  Node records hold 16 values (3 fields x
-// {value, d/dt, d/dx, d/dy, d/ds} + pad), column surface records 8.
+// address, loaded as 16-byte vectors.  Node records hold 16 values (for u, v, w
+// the piece {value, d/dx, d/dy, d/ds}, then {0, u_t, v_t, w_t}), column surface
+// records 8.
 template <int N, typename R>
 __device__ __forceinline__ void load_rec(R (&r)[N], const R* __restrict__ p) {
     if constexpr (sizeof(R) == 4) {
@@ -1273,10 +1274,10 @@ __device__ __forceinline__ void quad_query(R (&ov)[3], const QueryCell<R>& C, co
 // fraction taken in float.  TQ: coordinate/output type of the queries.  With
 // J.srec thread k evaluates the k-th query in cell order; p is always the
 // query's index in the caller's arrays.
-// What bounds it (1e7 queries, 748 us): the loads of the 16 node records, 1 KiB
-// per query through the L1 (260 us), the results' scattered stores (130), and
-// 1314 vector instructions per wavefront (330 at the issue limit), which overlap
-// only in part; a register cap that gives more waves spills and loses.  Cell-
+// What bounds it (1e7 queries, 607 us): the loads of the 16 node records, 1 KiB
+// per query through the L1 (about 260 us), the results' scattered stores (about
+// 130), and 1605 vector instructions per wavefront (408 at the issue limit),
+// which overlap only in part; a register cap that gives more waves spills and loses.  Cell-
 // ordered blocks are dealt so that each XCD takes one contiguous range of them:
 // neighbouring cells then share an L2 (past L2 154 instead of 270 MB per 1e6
 // queries).  The wave bounds keep the scheduler from giving up loads in flight

@@ -128,8 +128,17 @@ __device__ __forceinline__ double over_groups(double v) {
 }
 
 // A row block's steps [a, b) pair by pair, each with its own exponentials:
-// for waves with a point whose split exponents leave the number range (far
-// below the bed or above the surface, or rows far apart in k).  A lane takes
+// for waves with a point whose split exponents leave the number range.  Beside
+// points far below the bed or far above the surface that is deep water, for
+// points near the surface (z + 2h about 2h): in FP64 where kmax (z + 2h) > 600
+// (components to 2.5 rad/s: from 470 m on, all row blocks), in FP32 where half
+// a row block's spread of k times (z + 2h) exceeds 40 (evenly spaced
+// frequencies from 0.3 to 2.5 rad/s: 48 components from 130 m on in the topmost
+// of three row blocks, in all from 430 m; 128 from 320 m; 512 from 1200 m).
+// What it costs there, 65,536 points at 500 m, against the pair loop with a
+// thread a point (matrix path at 150 m): 48 components FP32 283 us, 248 (137),
+// FP64 550, 597 (161); 128 FP32 676, 1030 (361), FP64 3.38 ms, 3.64 (0.57);
+// 4,096 points 48 components FP32 58, 98 (52).  A lane takes
 // its point's rows of group g.  Kept out of line: it would cost the matrix
 // path its registers.
 template <typename R>

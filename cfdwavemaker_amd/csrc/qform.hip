@@ -611,9 +611,12 @@ __device__ __forceinline__ void qf_pair_tile(const QfJob& J, int ptile, int form
 // Blocks of an XCD (round-robin dispatch) walk the form pairs of two point
 // tiles together: the two tiles' Z operands stay in its L2 (1 MiB of hi parts
 // each at 1024 components), the tables stream through the last-level cache and
-// serve both tiles.  (An odd last tile's blocks numbered without idle ones
-// between took 4 % longer at 1024 components: 65,536 points, step 4.73 -> 4.93 ms.)  Past L2 a launch of one-form blocks read 92 GB in groups of 8 forms x
-// 32 point tiles, 89 GB one point tile at a time, 73 GB two at a time.
+// serve both tiles.  Past L2 a launch of one-form blocks read 92 GB in groups of
+// 8 forms x 32 point tiles, 89 GB one point tile at a time, 73 GB two at a time.
+// Tile counts that 16 does not divide leave blocks that exit at once.  A
+// numbering without them was compiled to a kernel 4 % slower at 256 tiles
+// (65,536 points, 1024 components, step 4.73 -> 4.93 ms), where both give every
+// block the same work; why is not known, nor how they compare at other counts.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_qf_pairs(QfJob J, int npt) {
     const int np = qf_pairs(J.nform, J.ncos), sq = blockIdx.x >> 3;
@@ -1053,7 +1056,9 @@ hipError_t launch_qf_forms(const QfJob& J, hipStream_t st) {
     const int npt = (int)(wide ? J.ppad / 256 : (J.P + 127) / 128);
     // An XCD that keeps its point tiles reads their Z operands through its own L2,
     // but where 8 does not divide the tiles some XCDs have one fewer, else the
-    // tiles go block after block.  One product waits for the operands most: kept
+    // tiles go block after block.  The lines are drawn through measurements; that
+    // three products lose at 70 tiles, with 3 % of padding, has no explanation
+    // here.  One product waits for the operands most: kept
     // from 16 tiles on, if that adds under 30 % (23 forms, 1024 components, 25
     // tiles 276 us against 329).  Three: kept up to 64 tiles, if it adds under
     // 5 % (40 forms, 752 components, 61 tiles 1177 us against 1271; 1008

@@ -12,10 +12,11 @@
 // its outputs are scattered (to the caller's order).
 //
 // Measured (256 x 256 x 16 FP32 grid, ordering / query kernel, us): 1e6 queries
-// 33 / 72 with 4096 tiles of 4 x 4 columns (a radix sort by column and a record
-// per lane took 230 / 104), 1e7 queries 315 / 642 with 16384 tiles of 2 x 2
-// columns (4096 tiles: 250 / 748; radix sort: 380 / 806).  At 1e7 the scattered
-// records and results, 16 bytes to a line each, take about 250 of these.
+// 37 / 73 with 4096 tiles of 4 x 4 columns (a radix sort by column and a record
+// per lane took 230 / 104), 1e7 queries 308 / 607 with 16384 tiles of 2 x 2
+// columns (with the query kernel of that time, 642: 4096 tiles 250 / 748, radix
+// sort 380 / 806).  At 1e7 the scattered records and results, 16 bytes to a line
+// each, take about 250 of these.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -57,3 +57,21 @@ def test_points_without_taylor_terms(prec):
         g, ref = a.eval(kind, *q), b.eval(kind, *q)
         assert np.all(np.isfinite(ref)) and np.any(ref)
         assert np.max(np.abs(g - ref)) <= (1e-11 if prec == "fp64" else 1e-5) * np.max(np.abs(ref)), kind
+
+
+@pytest.mark.parametrize("depth", [900.0, 2200.0])
+def test_fp64_forms_in_deep_water(depth, monkeypatch):
+    """kmax h of 570 and 1400, towards the largest the depth nodes serve, against the
+    pair loop; tolerance as in shallower water (rounding of sums over 700 pairs).
+    (One direction: across directions the combined wavenumbers reach beyond kmax.)"""
+    from cfdwavemaker_amd import engine as eng
+    s = make_sea(38, 3.0, 9.0, depth, seed=4, ndir=1).as_dict()
+    s["theta"] = np.full(38, 0.4)
+    args = ((0.0, 310.0, 0.0, 150.0), 32, 16, 9, 0.5, 0.5, 0.7, 1.5, depth)
+    forms = eng.Sea(s, with_direct=False).grid(*args)
+    monkeypatch.setenv("CFDWM_QFORM", "0")
+    loop = eng.Sea(s, with_direct=False).grid(*args)
+    assert forms.qform_reason() == "used" and loop.qform_reason() == "switched off"
+    for f in ("ETA", "UX", "UY") + (("UZ",) if depth < 1000 else ()):
+        a, b = forms.export(f), loop.export(f)
+        assert np.any(b) and np.max(np.abs(a - b)) <= 1e-11 * np.max(np.abs(b)), f
