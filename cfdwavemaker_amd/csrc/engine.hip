@@ -291,10 +291,11 @@ template <typename R>
 int Sea::put_table(const PairTable& P, DevBuf& row, DevBuf* mhi, DevBuf& uvw, DevBuf& xr) {
     hipStream_t st = Engine::get().stream();
     const int64_t ne = (int64_t)P.rec.size();
+    const double h = tab.in.depth;
     std::vector<UvwRec<R>> u(ne > 0 ? ne : 1);
     std::vector<XRec<R>> x(ne > 0 ? ne : 1);
     for (int64_t e = 0; e < ne; ++e) {
-        u[e] = uvw_rec<R>(P.rec[e], tab.in.depth);
+        u[e] = uvw_rec<R>(P.rec[e], h);
         x[e] = XRec<R>{(R)P.rec[e].xP, (R)P.rec[e].xM};
     }
     if (row.upload(P.rowoff.data(), P.rowoff.size() * sizeof(int64_t), st)) return -3;
