@@ -157,3 +157,38 @@ def test_one_workspace_for_all_grids(eng, monkeypatch):
     more[0].refill()
     assert all(np.array_equal(more[0].export(f), first[0].export(f)) for f in ("ETA", "UX", "UY", "UZ"))
     assert scaled_err(more[0].export("UX"), loop[0].export("UX")) <= TOL
+
+
+@pytest.mark.gpu
+def test_fills_from_several_threads(eng):
+    """Grids of different sizes (the shared workspace grows in between) filled and
+    updated side by side give what each gives alone, bit for bit."""
+    import threading
+
+    def run(k, rounds):
+        s = make_sea(10 + 9 * k, 3.0, 9.0, 40.0, seed=k, ndir=1 + k % 3).as_dict()
+        nx = 24 + 20 * k
+        g = eng.Sea(s, with_direct=False).grid((0.0, 300.0, 0.0, 90.0), nx, 20, 3, 0.0, 0.5, 0.7, 1.5, 40.0)
+        assert g.qform_reason() == "used"
+        out = []
+        for r in range(rounds):
+            g.refill() if r % 2 else g.force_update(0.75 + 0.5 * r)
+            out.append([g.export(f) for f in ("ETA", "UX", "UZ")])
+        return out
+    ref = [run(k, 6) for k in range(4)]
+    got, errors = [None] * 4, []
+
+    def worker(k):
+        try:
+            got[k] = run(k, 6)
+        except Exception as e:            # reported below, in the test's own thread
+            errors.append((k, e))
+    th = [threading.Thread(target=worker, args=(k,)) for k in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors
+    for a, b in zip(ref, got):
+        for p, q in zip(a, b):
+            assert all(np.array_equal(x, y) for x, y in zip(p, q))
